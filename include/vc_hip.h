@@ -66,11 +66,11 @@ const char* vc_hip_device_name(void);
 const char* vc_hip_last_error(void);
 /* MetalBackend::gemm_kernel (metal_backend.hpp:22): "mfma" (matrix-core
  * tiles by shape: 256 x 256 for large products, 128 x 128, or 32 x 32 for
- * products of a few tiles, and the FMA tiles for tiny products), "simple"
+ * products of few tiles, and the FMA tiles for tiny products), "simple"
  * (portable FMA tiles for every product, forced by VECTORCORE_HIP_GEMM=simple),
- * "mfma128" (128 x 128 tiles for every product), "mfma256" (256 x 256 tiles
- * for every product with 16-byte aligned rows and no batch reduction, 128 x
- * 128 for the rest), or "unavailable". The last two (also settable through
+ * "mfma128" (128 x 128 tiles for every product; 256 x 128 where rows are not
+ * whole 16-byte groups), "mfma256" (256 x 256 tiles for every product without a
+ * batch reduction, 128 x 128 for the rest), or "unavailable". The last two (also settable through
  * VECTORCORE_HIP_GEMM) exist for tests and tuning: both tile sizes give the
  * same bits for a product that neither splits along K. */
 const char* vc_hip_gemm_kernel(void);
@@ -285,7 +285,7 @@ int vc_hip_matmul_relu_mask_colsum(const float* a, const float* b, float* c, siz
                                    int trans_a, int trans_b, const float* mask, float* column_sum);
 /* vc_hip_matmul_relu_mask_colsum whose column sums may stay pending: when the
  * product's kernel keeps per-tile partial rows (any product not split along
- * K), *pending receives a handle to them and column_sum is not written;
+ * K, or split within one launch and of K <= 2048), *pending receives a handle to them and column_sum is not written;
  * otherwise *pending is NULL and column_sum is written as
  * vc_hip_matmul_relu_mask_colsum writes it. Finishing the handle gives the
  * bits vc_hip_matmul_relu_mask_colsum writes. Serves the same rules. */
@@ -306,7 +306,7 @@ int vc_hip_matmul_bias_relu(const float* a, const float* b, float* c, size_t m, 
  * stands for element (i, j); ceil(m / 32) * n words. */
 /* vc_hip_matmul_bias_relu with relu on, which also writes the ReLU bitmask
  * of [c > 0] when the product runs on the kernel that can (the 256-row
- * tiles, chosen by size): *bits_written is then 1, otherwise 0 and relu_bits
+ * tiles, chosen by size; a forced tile size needs rows of whole 16-byte groups): *bits_written is then 1, otherwise 0 and relu_bits
  * is not written. c is the same bits either way. No counterpart in the
  * reference: the bits stand for the mask that the ReLU's backward rule
  * (src/ops.cpp:395-403) reads from the layer's output, so that the product

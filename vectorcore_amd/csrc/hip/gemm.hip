@@ -13,9 +13,11 @@
 // the device). K advances in slices of 32 through two LDS stages with one
 // barrier per slice (the pipeline is described at gemm_mfma_kernel). Outputs
 // with few tiles and a long K split K into ranges whose partial products are
-// summed in range order by a second pass. Products of a few dozen such tiles
-// at most run on 32 x 32 tiles instead, K split over a workgroup's eight waves
-// (gemm_small_kernel), and tiny ones on the FMA kernel (gemm_simple_kernel).
+// summed in range order by a second pass. Large products run on 256-row tiles
+// (gemm_big_kernel); products that leave the larger tiles' last round mostly
+// idle, or whose rows are not whole 16-byte groups, on 32 x 32 tiles with K
+// split over a workgroup's waves and over workgroups (gemm_small_kernel); and
+// tiny ones on the FMA kernel (gemm_simple_kernel). choose_route picks.
 //
 // Each operand tile sits in LDS as it is laid out in memory, so it is stored
 // as loaded. A k-contiguous operand (A in NN/NT, B in NT/TT) is [128][32 + 4]
@@ -91,7 +93,8 @@ struct GemmArgs {
     double* col_part;              // null, or partial rows of C's column sums (batch 1, no split), in
                                    //   double: MFMA kernel 2 tiles_m rows (one per 64 rows of a tile),
                                    //   FMA kernel tiles_m rows (one per 16-row tile)
-    // ReLU bitmasks (gemm_big_kernel with A k-contiguous, batch 1, no split):
+    float* part;                   // gemm_small_kernel with a split: [tile][split][1024] partial tiles
+    // ReLU bitmasks (batch 1; gemm_big_kernel with A k-contiguous and no split, gemm_small_kernel reads them):
     // bit r % 32 of word (r / 32) N + c stands for element (r, c).
     const uint32_t* relu_bits;     // null, or the fused ReLU backward's mask as such bits: C *= [bit]
     uint32_t* relu_bits_out;       // null, or receives the bits of [C > 0] after the forward epilogue
@@ -148,6 +151,13 @@ constexpr int kWaitVmcnt0 = 0x0F70;
 __device__ inline __amdgpu_buffer_rsrc_t make_rsrc(const void* base) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), short(0), int(kOutOfRange - 1), 0x00020000);
 }
+// As make_rsrc, ending with the `elems` floats from base (none if negative):
+// each dword of a wider load past them reads 0.
+__device__ inline __amdgpu_buffer_rsrc_t make_rsrc(const float* base, int64_t elems) {
+    const int64_t limit = int64_t(kOutOfRange) / 4 - 1;
+    const int bytes = 4 * int(elems < 0 ? 0 : elems < limit ? elems : limit);
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), short(0), bytes, 0x00020000);
+}
 
 // Global -> register loader for one operand tile (128 along m/n, BK along k),
 // in four 16-byte slots per thread. Slot q of a k-contiguous operand is row
@@ -159,8 +169,9 @@ __device__ inline __amdgpu_buffer_rsrc_t make_rsrc(const void* base) {
 // one byte offset (slot 0); slots step by a uniform amount passed as the
 // instruction's scalar offset. The tile origin is uniform (scalar registers).
 // Edges are masked by pointing a slot out of range.
-// KC: operand contiguous along k.
-template <bool KC, bool Vec>
+// KC: operand contiguous along k. Rows are whole 16-byte groups (on any 4-byte
+// boundary: the loads need no more).
+template <bool KC>
 struct TileLoader {
     const float* origin;  // element (mn0, 0) of this operand
     int64_t step;         // elements per BK slice
@@ -196,18 +207,8 @@ struct TileLoader {
         const int k = kt * BK + k0 + (KC ? 0 : 8 * q);
         const int mn = mn0 + (KC ? kKcRowsPerSlot * q : 0);
         const uint32_t soff = uint32_t(q) * qstep;
-        if (Vec) {
-            const bool ok = mn < mn_lim && k < K;
-            return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rs, ok ? voff : kOutOfRange, soff, 0));
-        }
-        f4 v;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const bool ok = KC ? (mn < mn_lim && k + e < K) : (mn + e < mn_lim && k < K);
-            v[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, ok ? voff + 4u * e : kOutOfRange,
-                                                                                    soff, 0));
-        }
-        return v;
+        const bool ok = mn < mn_lim && k < K;
+        return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rs, ok ? voff : kOutOfRange, soff, 0));
     }
 
     // Byte offset in an LDS stage of this thread's first 16-byte store
@@ -220,9 +221,9 @@ struct TileLoader {
 
 // Store q (0..3) of this thread's slice registers into an LDS stage (`off`
 // from TileLoader::lds_off): every slot goes as loaded, in either layout.
-template <bool KC, bool Vec>
+template <bool KC>
 __device__ inline void store_slot(char* __restrict__ lds, uint32_t off, const f4 (&v)[kSlots], int q) {
-    *reinterpret_cast<f4*>(lds + off + q * TileLoader<KC, Vec>::lds_qstep) = v[q];
+    *reinterpret_cast<f4*>(lds + off + q * TileLoader<KC>::lds_qstep) = v[q];
 }
 
 typedef float f2 __attribute__((ext_vector_type(2)));
@@ -260,12 +261,8 @@ __device__ inline void read_part(const float* __restrict__ lds, int off, int g, 
     }
 }
 
-// Vector-load variants fit two workgroups per CU (<= 256 VGPRs). The scalar-load
-// variants (misaligned operands only) keep 32 element loads and their masks
-// in flight, so they get the register file of one workgroup per CU rather
-// than spilling.
-template <bool TA, bool TB, bool Vec>
-__global__ __launch_bounds__(kThreads, Vec ? 2 : 1) void gemm_mfma_kernel(GemmArgs p) {
+template <bool TA, bool TB>
+__global__ __launch_bounds__(kThreads, 2) void gemm_mfma_kernel(GemmArgs p) {
     // Two LDS stages. Step kt multiplies out of stage cur while its second
     // k-group also stores slice kt + 1 (in registers since step kt - 1) into
     // the other stage and issues the global loads of slice kt + 2, each slot
@@ -315,8 +312,8 @@ __global__ __launch_bounds__(kThreads, Vec ? 2 : 1) void gemm_mfma_kernel(GemmAr
                 for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
 
         for (int64_t r = r_begin; r < r_end && kt_begin < kt_end; ++r) {
-            TileLoader<AKC, Vec> la;
-            TileLoader<BKC, Vec> lb;
+            TileLoader<AKC> la;
+            TileLoader<BKC> lb;
             la.init(p.a + aoff + r * p.a_rstride, p.lda, m0, p.M, p.K);
             lb.init(p.b + boff + r * p.b_rstride, p.ldb, n0, p.N, p.K);
             f4 ra[kSlots], rb[kSlots];
@@ -332,8 +329,8 @@ __global__ __launch_bounds__(kThreads, Vec ? 2 : 1) void gemm_mfma_kernel(GemmAr
                 }
 #pragma unroll
                 for (int q = 0; q < kSlots; ++q) {
-                    store_slot<AKC, Vec>(lds_a, a_st, ra, q);
-                    store_slot<BKC, Vec>(lds_b, b_st, rb, q);
+                    store_slot<AKC>(lds_a, a_st, ra, q);
+                    store_slot<BKC>(lds_b, b_st, rb, q);
                 }
                 const __amdgpu_buffer_rsrc_t na = la.slice(kt_begin + 1), nb = lb.slice(kt_begin + 1);
 #pragma unroll
@@ -372,8 +369,8 @@ __global__ __launch_bounds__(kThreads, Vec ? 2 : 1) void gemm_mfma_kernel(GemmAr
                         // own slot only, in either layout).
                         if (g >= 1 && g <= kSlots / 4) {
                             const int q = 4 * (g - 1) + s;
-                            store_slot<AKC, Vec>(st_a, a_st, ra, q);
-                            store_slot<BKC, Vec>(st_b, b_st, rb, q);
+                            store_slot<AKC>(st_a, a_st, ra, q);
+                            store_slot<BKC>(st_b, b_st, rb, q);
                             ra[q] = la.load(sa, kt + 2, q);
                             rb[q] = lb.load(sb, kt + 2, q);
                         }
@@ -533,8 +530,11 @@ __global__ __launch_bounds__(kThreads, Vec ? 2 : 1) void gemm_mfma_kernel(GemmAr
 // loads with the LDS destination: no staging registers, no LDS store
 // instructions; those stores alone cost 3% of the K loop), and the loop holds
 // no vector ALU work. Two stages of two unpadded 32 KiB tiles: 128 KiB of
-// LDS. Vector (16-byte) loads only; misaligned operands stay on the 128 x 128
-// tiles.
+// LDS. Rows need not be whole 16-byte groups (Whole false) nor start on 16-byte
+// boundaries: the loads need 4-byte alignment only. Where a row ends within a
+// group, the group's other values are the next row's, or lie past the matrix:
+// the descriptor then ends with the matrix (they read 0), values past K are
+// zeroed once they are in LDS, and those past M or N reach outputs outside C only.
 constexpr int BT = 256;                   // tile rows (M); tile columns BN_ = 256 or 128
 constexpr int kBigLdsTile = BT * BK;       // floats per operand stage at most (32 KiB)
 
@@ -554,11 +554,12 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 //   k-rows from (1024 / EXT) q + (256 / EXT) w, lane t column 4 t mod EXT.
 // Edges: rows (columns) past the matrix, and k past K, point out of range;
 // such lanes write zeros into LDS.
-template <bool KC, int EXT>
+template <bool KC, int EXT, bool Whole>
 struct BigLoader {
     static constexpr int kSlots = EXT / 32;        // loads per thread per slice
     static constexpr int kRowsPerLoad = 1024 / EXT;  // k-rows of an m/n-contiguous operand per load round
     const float* origin;
+    const float* end;  // the end of the operand's matrix
     int64_t step;
     int K, mn_lim, wave;
     uint32_t qstep, voff;  // soffset step per load; this lane's byte offset of load 0 in a slice
@@ -569,6 +570,7 @@ struct BigLoader {
         mn_lim = MN - mn_origin;
         wave = wave_;
         origin = KC ? base + int64_t(mn_origin) * ld : base + mn_origin;
+        end = base + int64_t(KC ? MN : K_) * ld;
         step = KC ? int64_t(BK) : int64_t(BK) * ld;
         const uint32_t ld4 = uint32_t(ld) * 4u;
         if (KC) {
@@ -583,17 +585,37 @@ struct BigLoader {
         voff = KC ? uint32_t(mn0) * ld4 + uint32_t(k0) * 4u : uint32_t(k0) * ld4 + uint32_t(mn0) * 4u;
     }
 
-    __device__ __amdgpu_buffer_rsrc_t slice(int kt) const { return make_rsrc(origin + int64_t(kt) * step); }
+    __device__ __amdgpu_buffer_rsrc_t slice(int kt) const {
+        const float* const base = origin + int64_t(kt) * step;
+        return Whole ? make_rsrc(base) : make_rsrc(base, end - base);
+    }
+
+    // Zero what slice kt (in LDS at `stage`, this wave's loads landed) holds past K in this wave's groups that K cuts.
+    __device__ void clear_tail(float* stage, int kt, int lane) const {
+        if constexpr (KC && !Whole) {
+            const int left = K - kt * BK;
+            if (left < BK && left % 4 != 0 && lane < EXT / 4) {
+                const int row = 32 * (lane / 8) + 8 * wave + lane % 8;
+                float* const cut = stage + row * BK + 4 * ((left / 4) ^ ((row >> 1) & 7));
+                for (int e = left % 4; e < 4; ++e) cut[e] = 0.0f;
+            }
+        }
+    }
 
     // Load q's offset in slice kt, every edge masked.
     __device__ uint32_t masked_off(int kt, int q) const {
         const int k = kt * BK + k0 + (KC ? 0 : kRowsPerLoad * q);
         const int mn = mn0 + (KC ? 32 * q : 0);
-        return mn < mn_lim && k < K ? voff : kOutOfRange;
+        return mn < mn_lim && k < K ? lane_off(q) : kOutOfRange;
     }
     // Load q's offset in a slice whose k all lie inside K: only rows
     // (columns) past the matrix point out of range.
-    __device__ uint32_t full_slice_off(int q) const { return mn0 + (KC ? 32 * q : 0) < mn_lim ? voff : kOutOfRange; }
+    __device__ uint32_t full_slice_off(int q) const {
+        return mn0 + (KC ? 32 * q : 0) < mn_lim ? lane_off(q) : kOutOfRange;
+    }
+    // This lane's part of load q's offset: the load's step goes with it when
+    // the descriptor ends with the matrix, so that all of it is range-checked.
+    __device__ uint32_t lane_off(int q) const { return Whole ? voff : voff + uint32_t(q) * qstep; }
 
     // Issue load q of the slice at rs into the LDS stage at `stage`. Written
     // as inline assembly so that the compiler does not see an LDS write: it
@@ -610,7 +632,7 @@ struct BigLoader {
         const uint32_t base = uint32_t(reinterpret_cast<uintptr_t>((lds_ptr_t)stage)) + 1024u * uint32_t(wave);
         asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                      :
-                     : "s"(base), "v"(off), "s"(rs), "s"(uint32_t(Q) * qstep), "i"(dst_q)
+                     : "s"(base), "v"(off), "s"(rs), "s"(Whole ? uint32_t(Q) * qstep : 0u), "i"(dst_q)
                      : "memory", "m0", "scc");
     }
 };
@@ -836,7 +858,7 @@ __device__ inline void big_epilogue(const GemmArgs& p, f16v (&acc)[2][2], const 
         }
 }
 
-template <bool TA, bool TB, int BN_>
+template <bool TA, bool TB, int BN_, bool Whole>
 __global__ __launch_bounds__(kThreads, 1) void gemm_big_kernel(GemmArgs p) {
     // Step kt multiplies out of stage cur while k-groups 0 and 1 issue the
     // loads of slice kt + 1 into the other stage (free since the previous
@@ -851,8 +873,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_big_kernel(GemmArgs p) {
     constexpr bool AKC = !TA;
     constexpr bool BKC = TB;
     constexpr int QN = BN_ / 128;  // 64-column halves per wave
-    using LoaderA = BigLoader<AKC, BT>;
-    using LoaderB = BigLoader<BKC, BN_>;
+    using LoaderA = BigLoader<AKC, BT, Whole>;
+    using LoaderB = BigLoader<BKC, BN_, Whole>;
     int tm, tn;
     tile_coords(int(blockIdx.x), p.tiles_m, p.tiles_n, tm, tn);
     const int m0 = tm * BT, n0 = tn * BN_;
@@ -904,6 +926,11 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_big_kernel(GemmArgs p) {
                 });
             }
             __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+            if constexpr (!Whole) {
+                asm volatile("" ::: "memory");
+                la.clear_tail(A0, kt_begin, lane);
+                lb.clear_tail(B0, kt_begin, lane);
+            }
             __syncthreads();
             BigFrag<AKC> fa[2];  // [k-group parity]
             BigFrag<BKC> fb[2];
@@ -940,6 +967,13 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_big_kernel(GemmArgs p) {
                     const int cb = g & 1;
                     if (g == BK / 8 - 1) {
                         __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+                        if constexpr (!Whole && !kFast) {
+                            asm volatile("" ::: "memory");
+                            if (more) {
+                                la.clear_tail(as_next, kt + 1, lane);
+                                lb.clear_tail(bs_next, kt + 1, lane);
+                            }
+                        }
                         __syncthreads();
                     }
                     static_for<4>([&](auto sc) {
@@ -1210,149 +1244,314 @@ __global__ __launch_bounds__(256) void gemm_simple_kernel(GemmArgs p) {
     }
 }
 
-// Small products (a few 128 x 128 tiles, K too long for the FMA kernel): a
-// workgroup of W = kSmallWaves waves computes one 32 x 32 tile of C as one
-// V_MFMA_F32_32X32X2_F32 block per wave, wave w taking the 32-deep K chunks
-// w, w + W, ..., and the W partial tiles are added in wave order through
-// LDS, so one launch finishes the product in a fixed order. Operands go from
-// memory straight into the MFMA operand layout, no LDS staging: in chunk c,
-// half-wave h of MFMA step j takes k = 32 c + 16 h + j (a fixed permutation of
-// the summation index, identical for A and B), lane l row (A) or column (B)
-// l % 32. A k-contiguous operand is read as four 16-byte loads per lane and
-// chunk (vec), an m/n-contiguous one as 16 loads of 32 consecutive floats per
-// half-wave. The next chunk's loads are issued before this chunk's MFMAs.
-// col_part: one partial row per 32-row tile.
-constexpr int kSmallTile = 32;
-// Element `elem` of a buffer (4 floats from it: small_ld4), or 0 when !ok.
-__device__ inline float small_ld1(__amdgpu_buffer_rsrc_t rs, uint32_t elem, bool ok) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, ok ? elem * 4u : kOutOfRange, 0, 0));
-}
-__device__ inline f4 small_ld4(__amdgpu_buffer_rsrc_t rs, uint32_t elem, bool ok) {
-    return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rs, ok ? elem * 4u : kOutOfRange, 0, 0));
-}
+// Small products, products of few rows or columns, and operands whose rows are
+// not on 16-byte boundaries: a workgroup of four waves computes one 32 x 32
+// tile of C as one V_MFMA_F32_32X32X2_F32 block per wave, over a range of the
+// product's 32-deep K chunks (the chunks of product r of a batch reduction
+// follow those of product r - 1). Wave w takes the range's chunks w, w + 4, ...;
+// the four partial tiles are added in wave order through LDS. When the output
+// has too few tiles to fill the chip the chunks are split into ranges
+// (blockIdx.y): each writes its partial tile, and the workgroup of a tile that
+// finishes last adds them in range order, so one launch finishes the product in
+// a fixed order.
+//
+// Every wave stages its own chunks, 32 x 32 floats of each operand, with
+// 16-byte loads straight into LDS (1 KiB of LDS per load, eight 128-byte row
+// segments of memory); no barrier is needed and no register holds a load in
+// flight. The loads need 4-byte alignment only, so operands of any row length
+// take this path. With two stages the next chunk's 8 loads are in flight while
+// this chunk is multiplied.
+// - k-contiguous operand, LDS [32 rows][32 k], 16-byte group c of row r at
+//   c ^ (r / 2 % 8), as BigLoader lays it out: a lane reads 4 consecutive k.
+// - m/n-contiguous operand, LDS [32 k][32], k at row k ^ (k / 4 % 2): a lane
+//   reads one float per step, the two half-waves (k 4 apart) in different banks.
+// Half-wave h of step 4 g + s takes k = 8 g + 4 h + s, in either layout. Even
+// and odd g go to two accumulators, added at the end: eight chains per tile
+// (with the four waves) as short as those of eight waves with one each.
+// Edges: the descriptor ends with the operand's matrix, so rows past the matrix
+// (and k past K of an m/n-contiguous operand) read 0. In the last chunk of a
+// k-contiguous operand whole groups past K are masked, and the rest of a group
+// that K cuts (it holds the next row's first values) is zeroed in LDS. Columns
+// past the matrix of an m/n-contiguous operand read the next row: they reach
+// outputs outside C only.
+//
+// Bound by the matrix units from about 1024^3 on (24 us, 88 TFLOP/s), below that
+// by the latency of a chunk and of the finish. Loads 4 bytes a lane, or operands
+// read straight into registers, as this kernel had them, issue four times the
+// loads: 1024^3 took 40 us, 999 x 515 x 515 NN 26 (now 13) and NT 35 (13), 1 x
+// 4096 x 4096 26.5 (17.5; 67 MB of weights), 256 x 4096 x 256 27.5 (13).
+constexpr int kSmallTile = 32, kSmallDepth = 32;
+constexpr int kSmallWaves = 4;
+constexpr int kSmallThreads = 64 * kSmallWaves;
+constexpr int kSmallStage = 2 * kSmallTile * kSmallDepth;  // floats of one wave's stage, A then B
+constexpr int kSmallLoads = 4;                             // loads per operand and chunk
+constexpr int kMaxSplitTiles = 1 << 14;
+__device__ unsigned int g_small_done[kMaxSplitTiles];
 
-template <bool TA, bool TB, bool Vec>
-struct SmallChunk {
-    float a[16], b[16];
-    // The 16 k from k0 of A (row `row` of op(A)) and B (column `col` of
-    // op(B)); elements outside op(A) / op(B) read as 0.
-    __device__ void load(__amdgpu_buffer_rsrc_t ra, __amdgpu_buffer_rsrc_t rb, const GemmArgs& p, int row, int col,
-                         int k0) {
-        const bool row_ok = row < p.M, col_ok = col < p.N;
+// One operand's chunk loader: the operand's matrices are stored with row stride
+// ld; mn0 is the tile's first row (column).
+template <bool KC>
+struct SmallLoader {
+    uint32_t voff[kSmallLoads];  // this lane's byte offset of load i within a chunk
+    int ld, mn0, K, lane;
+
+    __device__ void init(int ld_, int mn0_, int K_, int lane_) {
+        ld = ld_, mn0 = mn0_, K = K_, lane = lane_;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int k = k0 + 4 * q;
-            if constexpr (!TA && Vec) {  // A [M][K]: 16 consecutive k of one row
-                const f4 v = small_ld4(ra, uint32_t(row * p.lda + k), row_ok && k < p.K);
-                a[4 * q] = v.x, a[4 * q + 1] = v.y, a[4 * q + 2] = v.z, a[4 * q + 3] = v.w;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    a[4 * q + e] = small_ld1(ra, TA ? uint32_t((k + e) * p.lda + row) : uint32_t(row * p.lda + k + e),
-                                             row_ok && k + e < p.K);
-            }
-            if constexpr (TB && Vec) {  // B [N][K]: 16 consecutive k of one column
-                const f4 v = small_ld4(rb, uint32_t(col * p.ldb + k), col_ok && k < p.K);
-                b[4 * q] = v.x, b[4 * q + 1] = v.y, b[4 * q + 2] = v.z, b[4 * q + 3] = v.w;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    b[4 * q + e] = small_ld1(rb, TB ? uint32_t(col * p.ldb + k + e) : uint32_t((k + e) * p.ldb + col),
-                                             col_ok && k + e < p.K);
-            }
+        for (int i = 0; i < kSmallLoads; ++i) {
+            const int row = 8 * i + lane / 8;  // LDS row
+            if constexpr (KC) voff[i] = uint32_t(row * ld + 4 * group(i)) * 4u;
+            else voff[i] = uint32_t((row ^ ((row >> 2) & 1)) * ld + 4 * (lane % 8)) * 4u;
         }
+    }
+
+    // The 16-byte group along k that load i fetches on this lane (k-contiguous operand).
+    __device__ int group(int i) const { return (lane % 8) ^ (((8 * i + lane / 8) >> 1) & 7); }
+
+    // Issue the loads of chunk c of the matrix at base (elems elements) into LDS from byte address `lds`.
+    __device__ void load(const float* base, int64_t elems, int c, uint32_t lds) const {
+        const int64_t first = KC ? int64_t(mn0) * ld + kSmallDepth * c : int64_t(kSmallDepth * c) * ld + mn0;
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(base + first, elems - first);
+        const int left = K - kSmallDepth * c;  // k of a k-contiguous chunk inside K
+        static_for<kSmallLoads>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            load_one<1024 * i>(rs, !KC || 4 * group(i) < left ? voff[i] : kOutOfRange, lds);
+        });
+    }
+
+    // Zero what the last chunk (in LDS at `stage`, landed) holds past K in groups that K cuts.
+    __device__ void clear_tail(float* stage, int c) const {
+        const int left = K - kSmallDepth * c;
+        if (KC && left < kSmallDepth && left % 4 != 0 && lane < kSmallTile) {
+            float* const cut = stage + lane * kSmallDepth + 4 * ((left / 4) ^ ((lane >> 1) & 7));
+            for (int e = left % 4; e < 4; ++e) cut[e] = 0.0f;
+        }
+    }
+
+    // The value of lane's row (column) at the two halves' k of steps 4 g .. 4 g + 3.
+    static __device__ f4 read(const float* stage, int g, int lane) {
+        const int half = lane >> 5, l32 = lane & 31;
+        if constexpr (KC) {
+            return *reinterpret_cast<const f4*>(stage + l32 * kSmallDepth + 4 * ((2 * g + half) ^ ((l32 >> 1) & 7)));
+        } else {
+            f4 v;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) v[s] = stage[(8 * g + 4 * half + (s ^ half)) * kSmallTile + l32];
+            return v;
+        }
+    }
+
+    // Inline assembly for the reason given at BigLoader::load; the loads are
+    // waited for explicitly before their stage is read.
+    template <int At>
+    static __device__ void load_one(__amdgpu_buffer_rsrc_t rs, uint32_t off, uint32_t lds) {
+        asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     :
+                     : "s"(lds), "v"(off), "s"(rs), "i"(At)
+                     : "memory", "m0", "scc");
     }
 };
 
-// Eight waves measured 5-18% faster than four on the products this kernel
-// takes (1024^3: 38.1 against 42.5 us; 512 x 8192 x 512: 62.5 against 75.8);
-// sixteen spill registers.
-constexpr int kSmallWaves = 8;  // waves (K shares) per 32 x 32 tile
-constexpr int kSmallThreads = 64 * kSmallWaves;
-
-template <bool TA, bool TB, bool Vec>
-__global__ __launch_bounds__(kSmallThreads) void gemm_small_kernel(GemmArgs p) {
-    __shared__ float part[kSmallWaves][16][64];         // [wave][accumulator v][lane]
-    __shared__ float tile[kSmallTile][kSmallTile + 1];  // final values, for the column sums
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int tm = int(blockIdx.x) / p.tiles_n, tn = int(blockIdx.x) % p.tiles_n;
+template <bool TA, bool TB, int Stages>
+__global__ __launch_bounds__(kSmallThreads, Stages == 1 ? 5 : 2) void gemm_small_kernel(GemmArgs p) {
+    constexpr bool AKC = !TA, BKC = TB;
+    constexpr int kStaging = kSmallWaves * Stages * kSmallStage;
+    static_assert(kStaging > kSmallWaves * 1024 + kSmallTile * (kSmallTile + 1), "partial tiles exceed the staging LDS");
+    // The waves' stages; after the K loop the waves' partial tiles
+    // ([wave][accumulator v][lane]), the final tile for the column sums and a
+    // flag: five workgroups of one stage fit a CU with nothing beside them.
+    __shared__ __align__(16) float lds[kStaging];
+    float(*const part)[16][64] = reinterpret_cast<float(*)[16][64]>(lds);
+    float(*const tile)[kSmallTile + 1] = reinterpret_cast<float(*)[kSmallTile + 1]>(lds + kSmallWaves * 1024);
+    int* const last_range = reinterpret_cast<int*>(lds + kStaging - 1);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+    int tm, tn;
+    tile_coords(int(blockIdx.x), p.tiles_m, p.tiles_n, tm, tn);
     const int m0 = tm * kSmallTile, n0 = tn * kSmallTile;
-    const int half = lane >> 5;
-    const int chunks = (p.K + 31) / 32;
-    for (int64_t z = blockIdx.y; z < p.batch; z += gridDim.y) {
-        const int64_t aoff = uniform64(p.table ? p.table[2 * z] : z * p.a_bstride);
-        const int64_t boff = uniform64(p.table ? p.table[2 * z + 1] : z * p.b_bstride);
-        f16v acc;
+    const int half = lane >> 5, l32 = lane & 31;
+    const int chunks = (p.K + kSmallDepth - 1) / kSmallDepth;  // of one product
+    const int total = chunks * int(p.reduce);
+    const int64_t a_elems = int64_t(p.M) * p.K, b_elems = int64_t(p.K) * p.N;
+    SmallLoader<AKC> la;
+    SmallLoader<BKC> lb;
+    la.init(p.lda, m0, p.K, lane);
+    lb.init(p.ldb, n0, p.K, lane);
+    float* const own = lds + wave * (Stages * kSmallStage);
+    const uint32_t own_addr = uint32_t(reinterpret_cast<uintptr_t>((lds_ptr_t)own));
+    const int64_t jobs = p.batch * p.splits;
+    for (int64_t job = blockIdx.y; job < jobs; job += gridDim.y) {
+        const int64_t z = uniform64(job / p.splits);
+        const int split = __builtin_amdgcn_readfirstlane(int(job - z * p.splits));
+        const float* const A = p.a + uniform64(p.table ? p.table[2 * z] : z * p.a_bstride);
+        const float* const B = p.b + uniform64(p.table ? p.table[2 * z + 1] : z * p.b_bstride);
+        const int begin = split * p.kt_per_split, end = min(total, begin + p.kt_per_split);
+        const auto issue = [&](int g, int stage) {
+            int r = 0, c = g;
+            if (p.reduce > 1) {
+                r = __builtin_amdgcn_readfirstlane(g / chunks);
+                c = g - r * chunks;
+            }
+            const uint32_t at = own_addr + uint32_t(stage) * (kSmallStage * 4u);
+            la.load(A + r * p.a_rstride, a_elems, c, at);
+            lb.load(B + r * p.b_rstride, b_elems, c, at + kSmallStage * 2u);
+        };
+        f16v acc[2];
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
-        for (int64_t r = 0; r < p.reduce; ++r) {
-            const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.a + aoff + r * p.a_rstride);
-            const __amdgpu_buffer_rsrc_t rb = make_rsrc(p.b + boff + r * p.b_rstride);
-            const int row = m0 + (lane & 31), col = n0 + (lane & 31);
-            SmallChunk<TA, TB, Vec> cur, next;
-            if (wave < chunks) cur.load(ra, rb, p, row, col, 32 * wave + 16 * half);
-            for (int c = wave; c < chunks; c += kSmallWaves) {
-                const bool more = c + kSmallWaves < chunks;
-                if (more) next.load(ra, rb, p, row, col, 32 * (c + kSmallWaves) + 16 * half);
+        for (int v = 0; v < 16; ++v) acc[0][v] = acc[1][v] = 0.0f;
+        int g = begin + wave, stage = 0;
+        if (g < end) issue(g, 0);
+        for (; g < end; g += kSmallWaves) {
+            if (Stages > 1 && g + kSmallWaves < end) {
+                issue(g + kSmallWaves, stage ^ 1);
+                asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // this chunk's loads; the next chunk's 8 stay in flight
+            } else {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            }
+            float* const as = own + stage * kSmallStage;
+            float* const bs = as + kSmallTile * kSmallDepth;
+            if ((AKC || BKC) && p.K % 4 != 0) {
+                const int c = p.reduce > 1 ? g % chunks : g;
+                la.clear_tail(as, c);
+                lb.clear_tail(bs, c);
+            }
+            f4 a[4], b[4];
 #pragma unroll
-                for (int j = 0; j < 16; ++j)
-                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(cur.a[j], cur.b[j], acc, 0, 0, 0);
-                if (more) cur = next;
+            for (int q = 0; q < 4; ++q) {
+                a[q] = SmallLoader<AKC>::read(as, q, lane);
+                b[q] = SmallLoader<BKC>::read(bs, q, lane);
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    acc[q & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q][s], b[q][s], acc[q & 1], 0, 0, 0);
+            // The reads above must be back before their stage is loaded again.
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (Stages > 1) {
+                stage ^= 1;
+            } else if (g + kSmallWaves < end) {
+                issue(g + kSmallWaves, 0);
             }
         }
+        __syncthreads();  // the partial tiles take the stages' place
 #pragma unroll
-        for (int v = 0; v < 16; ++v) part[wave][v][lane] = acc[v];
+        for (int v = 0; v < 16; ++v) part[wave][v][lane] = acc[0][v] + acc[1][v];
         __syncthreads();
-        // Thread t finishes accumulator slots (v, l) = t / 64 + W i, t % 64
-        // (W waves): the waves' partials in wave order, then the epilogue.
-        float* C = p.c + z * int64_t(p.M) * p.N;
+        // Thread t holds accumulator slots (v, l) = (t / 64 + 4 i, t % 64): the
+        // waves' partials in wave order.
+        const int el = epilogue_lane(), et = 64 * wave + el;  // not kept across the K loop
+        float value[4];
+        int row[4], col[4];
+        bool inside[4];
 #pragma unroll
-        for (int i = 0; i < 16 / kSmallWaves; ++i) {
-            const int v = int(threadIdx.x) / 64 + kSmallWaves * i, l = int(threadIdx.x) % 64;
-            float value = part[0][v][l];
-#pragma unroll
-            for (int w = 1; w < kSmallWaves; ++w) value += part[w][v][l];
-            const int tr = 8 * (v / 4) + 4 * (l / 32) + v % 4, tc = l % 32;  // the MFMA's D layout
-            const int row = m0 + tr, col = n0 + tc;
-            const bool inside = row < p.M && col < p.N;
-            const int64_t t = int64_t(row) * p.N + col;
-            if (inside) {
-                if (p.relu_mask) value = value * (p.relu_mask[z * int64_t(p.M) * p.N + t] > 0.0f ? 1.0f : 0.0f);
-                if (p.bias || p.relu) value = bias_relu(value, p.bias ? p.bias[col] : 0.0f, p.relu != 0);
-                C[t] = value;
-            }
-            tile[tr][tc] = inside ? value : 0.0f;
+        for (int i = 0; i < 4; ++i) {
+            const int v = wave + 4 * i, l = el;
+            value[i] = ((part[0][v][l] + part[1][v][l]) + part[2][v][l]) + part[3][v][l];
+            row[i] = m0 + 8 * (v / 4) + 4 * (l / 32) + v % 4;  // the MFMA's D layout
+            col[i] = n0 + l % 32;
+            inside[i] = row[i] < p.M && col[i] < p.N;
         }
-        if (p.col_part) {  // batch 1: the tile's 32 rows of each column, in row order, in double
+        bool finish = true;
+        if (p.splits > 1) {
+            // This range's partial tile, device-scope stores; the range that
+            // counts in last adds all of them (see red::wait_stores_visible).
+            const int64_t tile_id = z * (int64_t(p.tiles_m) * p.tiles_n) + int64_t(tm) * p.tiles_n + tn;
+            float* const mine = p.part + (tile_id * p.splits) * 1024;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (inside[i])
+                    __hip_atomic_store(&mine[split * 1024 + 256 * i + et], value[i], __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+            red::wait_stores_visible();
             __syncthreads();
-            if (threadIdx.x < kSmallTile && n0 + int(threadIdx.x) < p.N) {
-                double sum = 0.0;
-                for (int rr = 0; rr < kSmallTile; ++rr) sum += double(tile[rr][threadIdx.x]);
-                p.col_part[int64_t(tm) * p.N + n0 + threadIdx.x] = sum;
+            if (et == 0) {
+                unsigned* counter = &g_small_done[tile_id];
+                const bool last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 ==
+                                  unsigned(p.splits);
+                if (last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                *last_range = last;
+            }
+            __syncthreads();
+            finish = *last_range != 0;
+            if (finish) {
+                const __amdgpu_buffer_rsrc_t rp =
+                    __builtin_amdgcn_make_buffer_rsrc(mine, short(0), p.splits * 4096, 0x00020000);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) value[i] = 0.0f;
+                for (int s0 = 0; s0 < p.splits; s0 += 8) {
+                    float x[8][4];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            x[u][i] = __builtin_bit_cast(
+                                float, __builtin_amdgcn_raw_buffer_load_b32(
+                                           rp,
+                                           inside[i] ? uint32_t((s0 + u) * 1024 + 256 * i + et) * 4u
+                                                     : kOutOfRange,
+                                           0, 16));  // past the last range: outside the descriptor, reads 0
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        if (s0 + u < p.splits)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) value[i] = s0 + u == 0 ? x[u][i] : value[i] + x[u][i];
+                }
+            }
+        }
+        if (finish) {
+            float* const C = p.c + z * int64_t(p.M) * p.N;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (inside[i]) {
+                    const int64_t t = int64_t(row[i]) * p.N + col[i];
+                    if (p.relu_mask)
+                        value[i] = value[i] * (p.relu_mask[z * int64_t(p.M) * p.N + t] > 0.0f ? 1.0f : 0.0f);
+                    if (p.relu_bits)  // batch 1; a tile's 32 rows are one word row
+                        value[i] = value[i] * float((p.relu_bits[int64_t(tm) * p.N + col[i]] >> (row[i] - m0)) & 1u);
+                    if (p.bias || p.relu) value[i] = bias_relu(value[i], p.bias ? p.bias[col[i]] : 0.0f, p.relu != 0);
+                    C[t] = value[i];
+                }
+                tile[row[i] - m0][col[i] - n0] = inside[i] ? value[i] : 0.0f;
+            }
+            if (p.col_part) {  // batch 1: the tile's 32 rows of each column, in row order, in double
+                __syncthreads();
+                if (et < kSmallTile && n0 + et < p.N) {
+                    double sum = 0.0;
+                    for (int rr = 0; rr < kSmallTile; ++rr) sum += double(tile[rr][et]);
+                    p.col_part[int64_t(tm) * p.N + n0 + et] = sum;
+                }
             }
         }
         __syncthreads();
     }
 }
 
+template <bool TA, bool TB, bool Whole>
+void launch_tiles(const GemmArgs& args, int big_n, dim3 grid, hipStream_t stream) {
+    if (big_n == 256) launch((gemm_big_kernel<TA, TB, 256, Whole>), grid, dim3(kThreads), 0, stream, args);
+    else if (big_n == 128) launch((gemm_big_kernel<TA, TB, 128, Whole>), grid, dim3(kThreads), 0, stream, args);
+    else if constexpr (Whole) launch((gemm_mfma_kernel<TA, TB>), grid, dim3(kThreads), 0, stream, args);
+}
+
 template <bool TA, bool TB>
-void launch_variant(const GemmArgs& args, bool vec, bool simple, bool small, int big_n, dim3 grid,
+void launch_variant(const GemmArgs& args, bool whole, bool simple, bool small, int big_n, dim3 grid,
                     hipStream_t stream) {
-    if (big_n == 256) {
-        launch((gemm_big_kernel<TA, TB, 256>), grid, dim3(kThreads), 0, stream, args);
-    } else if (big_n == 128) {
-        launch((gemm_big_kernel<TA, TB, 128>), grid, dim3(kThreads), 0, stream, args);
-    } else if (small) {
-        if (vec) launch((gemm_small_kernel<TA, TB, true>), grid, dim3(kSmallThreads), 0, stream, args);
-        else launch((gemm_small_kernel<TA, TB, false>), grid, dim3(kSmallThreads), 0, stream, args);
+    if (small) {
+        // One stage holds half the LDS, so twice the workgroups fit a CU: for grids of more than two
+        // workgroups per CU, and where a wave has one chunk only.
+        if (int64_t(grid.x) * grid.y > 2 * int64_t(device().cu_count) || args.kt_per_split <= kSmallWaves)
+            launch((gemm_small_kernel<TA, TB, 1>), grid, dim3(kSmallThreads), 0, stream, args);
+        else
+            launch((gemm_small_kernel<TA, TB, 2>), grid, dim3(kSmallThreads), 0, stream, args);
     } else if (simple) {
         if (args.K <= 16) launch((gemm_simple_kernel<TA, TB, 16>), grid, dim3(256), 0, stream, args);
         else if (args.K <= 64) launch((gemm_simple_kernel<TA, TB, 64>), grid, dim3(256), 0, stream, args);
         else launch((gemm_simple_kernel<TA, TB, 256>), grid, dim3(256), 0, stream, args);
-    } else if (vec) {
-        launch((gemm_mfma_kernel<TA, TB, true>), grid, dim3(kThreads), 0, stream, args);
+    } else if (whole) {
+        launch_tiles<TA, TB, true>(args, big_n, grid, stream);
     } else {
-        launch((gemm_mfma_kernel<TA, TB, false>), grid, dim3(kThreads), 0, stream, args);
+        launch_tiles<TA, TB, false>(args, big_n, grid, stream);
     }
 }
 
@@ -1360,22 +1559,27 @@ const char* variant_label(bool ta, bool tb) {
     return ta ? (tb ? "gemm_tt" : "gemm_tn") : (tb ? "gemm_nt" : "gemm_nn");
 }
 
-// Whether a product takes gemm_small_kernel rather than the 128 x 128 tiles
-// (tiles128 of them, times `products` matrices) or the FMA kernel (tiny).
-// Measured on MI355X with four waves per 32 x 32 tile (eight are faster
-// still): the 32 x 32 tiles run at up to ~60 TFLOP/s, while 9 to 64 tiles of
-// 128 x 128 leave most CUs idle (1024^3: 37.8 against 68.2 us;
-// 512 x 8192 x 512: 86 against 145 us). Up to 8 tiles and K above 2048, the
-// larger tiles split K 32 ways and win (256 x 4096 x 256: 27 against 42 us);
-// from 128 tiles they are as fast or faster (2048 x 1024^2: 69 against 72 us;
-// 2048^2 x 1024: 80 against 133 us). Among tiny products, weight gradients
-// (A transposed, K the batch, at least 128) gain from the waves' K split
-// (256 x 300 x 64: 6.1 against 12.1 us); the others stay on the FMA kernel.
-bool small_tiles(int64_t K, int64_t products, int64_t tiles128, bool tiny, bool ta, bool tb) {
-    if (tiny) return ta && !tb && K >= 128;
-    const int64_t work = tiles128 * products;
-    if (work <= 64 && K <= 2048) return true;
-    return work > 8 && work <= 32;
+// What a product costs on each kernel, in us, from measurements on MI355X:
+// whole rounds of the tiles that the chip holds at once, times what a round
+// costs per 1024 of K and at its ends (k = K / 1024).
+// - 256 x 256 tiles: 226 k + 27 (8192 x 4096 x 4096, two rounds: 1811 us; 4095 x
+//   65 x 4095, one: 43);
+// - 256 x 128: 124 k + 12 (8 x 1024^3: 124-128; 8192 x 33 x 4095, four: 62);
+// - 128 x 128: 120 k + 10 for two per CU (6000 x 1000 x 1000: 125-130; 3000^3,
+//   two rounds: 670), 70 k + 7 for one per CU (2048 x 1024 x 2048: 69-75),
+//   10 to add the partial products of a split K;
+// - the 32 x 32 tiles are small enough to count by area: 0.34 k + 0.05 for each
+//   128 x 128 outputs (3000^3: 516; 2500 x 1500 x 1700: 140, against 185 on the
+//   128 x 128 tiles; 8191 x 257 x 1023: 70, against 47 on the 256 x 128).
+double small_cost(int64_t tiles32, double k) { return double(tiles32) / 16.0 * (0.34 * k + 0.05); }
+double tiles128_cost(int64_t tiles, int64_t splits, double k, int cu_count) {
+    const int64_t n = tiles * splits, rounds = (n + 2 * cu_count - 1) / (2 * cu_count);
+    const double each = k / double(splits);
+    return (n <= cu_count ? 70.0 * each + 7.0 : double(rounds) * (120.0 * each + 10.0)) + (splits > 1 ? 10.0 : 0.0);
+}
+double big_cost(int64_t tiles, int64_t splits, double k, int cu_count, int width) {
+    const double rounds = double((tiles * splits + cu_count - 1) / cu_count);
+    return rounds * (width == 256 ? 226.0 * k / double(splits) + 27.0 : 124.0 * k / double(splits) + 12.0);
 }
 
 // The tile width of gemm_big_kernel (256 or 128 columns of 256 rows) for a
@@ -1411,6 +1615,72 @@ int big_tiles(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t reduce, in
     return 0;
 }
 
+// The kernel of a product: gemm_big_kernel with big_n columns, gemm_small_kernel,
+// gemm_simple_kernel, or else gemm_mfma_kernel. A fused mask, bias or ReLU only
+// decides between kernels that give the same bits.
+struct Route {
+    bool whole;  // both operands' rows are whole 16-byte groups
+    int big_n;
+    bool small, simple;
+};
+
+Route choose_route(int mode, int64_t M, int64_t N, int64_t K, int64_t batch, int64_t reduce, bool ta, bool tb,
+                   int cu_count, bool masked) {
+    Route r{};
+    r.whole = (ta ? M : K) % 4 == 0 && (tb ? K : N) % 4 == 0;
+    if (mode == kGemmSimple) {
+        r.simple = true;
+        return r;
+    }
+    // Byte offsets relative to a tile origin are 32-bit (256 rows of an
+    // operand or of C span less than 2 GiB), and a batch reduction takes the
+    // 256-row tiles only when it splits one product per split: output tiles
+    // times products within one workgroup per CU.
+    const auto big_fits = [&](int width) {
+        return std::max({ta ? M : K, tb ? K : N, N}) * BT < (int64_t(1) << 29) && batch <= 65535 / 32 &&
+               (reduce == 1 || ((M + BT - 1) / BT) * ((N + width - 1) / width) * batch * reduce <= cu_count);
+    };
+    const bool small_fits = reduce * ((K + kSmallDepth - 1) / kSmallDepth) <= std::numeric_limits<int>::max();
+    const double k = double(K) / 1024.0;
+    const double small = small_cost((M + kSmallTile - 1) / kSmallTile * ((N + kSmallTile - 1) / kSmallTile) * batch, k);
+    // The larger tiles' estimates count the splits of a long K that gemm() gives them.
+    const auto big = [&](int width) {
+        const int64_t n = (M + BT - 1) / BT * ((N + width - 1) / width) * batch;
+        return big_cost(n, n >= cu_count || K < 64 * BK ? 1 : std::min<int64_t>(4, (cu_count + n - 1) / n), k, cu_count, width);
+    };
+    const auto tiles128 = [&] {
+        const int64_t n = (M + BM - 1) / BM * ((N + BN - 1) / BN) * batch, slots = 2 * int64_t(cu_count);
+        const int64_t splits = n >= slots || K < 64 * BK ? 1 : std::min<int64_t>({4, (slots + n - 1) / n, K / (32 * BK)});
+        return tiles128_cost(n, splits, k, cu_count);
+    };
+    // Small products (<= 2^20 multiply-adds, K <= 1024): one memory round trip on the FMA kernel up to K of
+    // 128; longer ones take the 32 x 32 tiles, four waves along K (256 x 256 x 10: 7.0 -> 4.9 us, 1 x 1000 x
+    // 1000: 17.0 -> 6.8).
+    const bool tiny = double(M) * double(N) * double(K) * double(batch) * double(reduce) <= kTinyMacs &&
+                      K <= kSimpleMaxK;
+    if (mode == kGemmTiles256) {
+        r.big_n = big_fits(256) ? 256 : 0;
+    } else if (mode == kGemmTiles256x128 || (mode == kGemmTiles128 && !r.whole)) {
+        r.big_n = big_fits(128) ? 128 : 0;
+    } else if (mode == kGemmAuto && tiny) {
+        r.simple = K <= 128 || !small_fits;
+        r.small = !r.simple;
+        return r;
+    } else if (mode == kGemmAuto && r.whole) {
+        const int plain = big_fits(128) ? big_tiles(M, N, K, batch, reduce, cu_count, false) : 0;
+        r.small = small_fits && (!plain || reduce == 1) && small < (plain ? big(plain) : tiles128());
+        if (!r.small && plain) r.big_n = big_tiles(M, N, K, batch, reduce, cu_count, masked);
+    } else if (mode == kGemmAuto && reduce == 1 && big_fits(128)) {
+        r.small = small < std::min(big(128), big(256));
+        if (!r.small) r.big_n = big(256) < big(128) ? 256 : 128;
+    }
+    // Rows that are not whole groups: gemm_big_kernel and gemm_small_kernel only (a batch reduction of
+    // more than 2^31 chunks on neither).
+    if (!r.whole && !r.big_n) r.small = small_fits;
+    r.simple = !r.whole && !r.big_n && !r.small;
+    return r;
+}
+
 // offsets: nullptr for the affine mode (a_bstride / b_bstride).
 void gemm(const float* a, const float* b, float* c, int64_t M, int64_t N, int64_t K, int64_t batch, int64_t a_bstride,
           int64_t b_bstride, const std::vector<int64_t>* offsets, int64_t reduce, int64_t a_rstride, int64_t b_rstride,
@@ -1428,7 +1698,6 @@ void gemm(const float* a, const float* b, float* c, int64_t M, int64_t N, int64_
     if (M == 0 || N == 0 || batch == 0) return;
     if (!a || !b || !c) fail(VC_HIP_ERR_INVALID_ARGUMENT, "matmul: null buffer");
     const int mode = d.gemm_mode.load();  // the kernel setting in force for this call
-    const bool force_simple = mode == kGemmSimple;
     // A single large NN product runs as NT on a transposed copy of B: the
     // 128 x 128 tiles are ~3.5% faster when both operands are contiguous along
     // k, which outweighs the copy (2 K N floats of traffic) once M >= 4096. The
@@ -1437,10 +1706,11 @@ void gemm(const float* a, const float* b, float* c, int64_t M, int64_t N, int64_
     // is as fast as NT, and from K = 2048 on the copy no longer pays
     // (8192 x 4096 x 4096: 1886 us with the copy, 1872 without; at K = 1024
     // the copy still wins, 490 against 495).
+    const Route route = choose_route(mode, M, N, K, batch, reduce, ta, tb, d.cu_count, relu_mask != nullptr);
     const bool big_nn = (mode == kGemmTiles256 || mode == kGemmTiles256x128 ||
                          (mode == kGemmAuto && K >= 2048 && big_tiles(M, N, K, batch, reduce, d.cu_count, false))) &&
                         std::max(K, N) * BT < (int64_t(1) << 29);
-    if (!ta && !tb && batch == 1 && reduce == 1 && !force_simple && M >= kNnViaNtMinRows && N % 4 == 0 &&
+    if (!ta && !tb && batch == 1 && reduce == 1 && !route.simple && !route.small && M >= kNnViaNtMinRows && N % 4 == 0 &&
         K % 4 == 0 && K <= int64_t(65535) * 64 && aligned16(a) && aligned16(b) && !relu_mask && !relu_bits &&
         !big_nn) {
         Profiled prof("gemm_nn", 2.0 * double(M) * double(N) * double(K),
@@ -1457,49 +1727,17 @@ void gemm(const float* a, const float* b, float* c, int64_t M, int64_t N, int64_
     }
     const int64_t tiles_m_simple = (M + 15) / 16, tiles_n_simple = (N + 15) / 16;
     const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-    // Small products (<= 2^20 multiply-adds, K <= 1024) run on the FMA kernel:
-    // a 128 x 128 MFMA tile there is mostly padding, and its fixed latency
-    // (~8 us, plus a second pass when K is split) is several times the FMA
-    // kernel's whole run (one memory round trip per 256 k).
-    const bool tiny = double(M) * double(N) * double(K) * double(batch) * double(reduce) <= kTinyMacs &&
-                      K <= kSimpleMaxK;
-    const int64_t tiles_m32 = (M + kSmallTile - 1) / kSmallTile, tiles_n32 = (N + kSmallTile - 1) / kSmallTile;
-    // A product of a few 128 x 128 tiles takes 32 x 32 tiles with K split over
-    // the workgroup's eight waves (gemm_small_kernel): one launch, no split pass.
-    // Its operand offsets are 32-bit from the operand's origin.
-    const bool small_fits = M * K < (int64_t(1) << 29) && K * N < (int64_t(1) << 29) && M * N < (int64_t(1) << 29);
-    const bool automatic = mode == kGemmAuto;
-    bool small = automatic && small_fits && small_tiles(K, batch * reduce, tiles_m * tiles_n, tiny, ta, tb);
-    bool simple = force_simple || (automatic && !small && tiny);
     // Byte offsets relative to a tile origin are 32-bit: 128 rows of any
     // operand or of C must span less than 2 GiB (256 rows for the 256 x 256 tiles).
     const int64_t kMax = int64_t(1) << 29;
     const int64_t widest = std::max({ta ? M : K, tb ? K : N, N});
     if (M >= kMax || N >= kMax || K >= kMax || widest * 128 >= kMax)
         fail(VC_HIP_ERR_OVERFLOW, "matmul operands exceed the 2 GiB per-matrix addressing of the HIP kernels");
-    // 16-byte vector loads need every row start and batch offset on a 4-float boundary.
-    bool vec = aligned16(a) && aligned16(b) && (ta ? M : K) % 4 == 0 && (tb ? K : N) % 4 == 0 && a_rstride % 4 == 0 &&
-               b_rstride % 4 == 0;
-    if (offsets) {
-        for (int64_t v : *offsets) vec = vec && v % 4 == 0;
-    } else {
-        vec = vec && a_bstride % 4 == 0 && b_bstride % 4 == 0;
-    }
-    // A batch reduction takes the 256-row tiles only when it splits one
-    // product per split (r_per_split 1 below): output tiles times products
-    // within one workgroup per CU.
-    const auto reduce_fits = [&](int64_t width) {
-        return reduce == 1 || ((M + BT - 1) / BT) * ((N + width - 1) / width) * batch * reduce <= d.cu_count;
-    };
-    const bool big_fits = vec && widest * BT < kMax && batch <= 65535 / 32;
-    const int big_n = !big_fits                                        ? 0
-                      : mode == kGemmTiles256                          ? (reduce_fits(256) ? 256 : 0)
-                      : mode == kGemmTiles256x128                      ? (reduce_fits(128) ? 128 : 0)
-                      : automatic && !small && !simple && reduce_fits(128)
-                          ? big_tiles(M, N, K, batch, reduce, d.cu_count, relu_mask != nullptr)
-                          : 0;
+    const bool whole = route.whole, small = route.small, simple = route.simple;
+    const int big_n = route.big_n;
     const bool big = big_n != 0;
-    if (big) small = simple = false;
+    const int64_t tiles_m32 = (M + kSmallTile - 1) / kSmallTile, tiles_n32 = (N + kSmallTile - 1) / kSmallTile;
+    const int64_t small_chunks = reduce * ((K + kSmallDepth - 1) / kSmallDepth);
     const int64_t tiles_m256 = (M + BT - 1) / BT, tiles_n256 = big ? (N + big_n - 1) / big_n : 0;
     const int64_t tiles = big     ? tiles_m256 * tiles_n256
                           : small ? tiles_m32 * tiles_n32
@@ -1562,24 +1800,40 @@ void gemm(const float* a, const float* b, float* c, int64_t M, int64_t N, int64_
             splits = std::min(splits, kt_total / 16);
         }
     }
-    if (reduce == 1 && splits > 1)  // drop the ranges that ceil(kt_total / splits) slices each would leave empty
+    if (small) {
+        // Split while the chip has room for more workgroups and each range keeps two chunks per wave,
+        // unless it saves a wave no more chunks than finishing the partial tiles costs (about 2 us).
+        const auto per_wave = [&](int64_t ranges) {
+            return (small_chunks + ranges * kSmallWaves - 1) / (ranges * kSmallWaves);
+        };
+        int64_t ranges = std::min<int64_t>({2 * int64_t(d.cu_count) / (tiles * batch), small_chunks / 8, 64});
+        if (ranges < 2 || tiles * batch > kMaxSplitTiles || per_wave(1) - per_wave(ranges) <= 3) ranges = 1;
+        const int64_t per = (small_chunks + ranges - 1) / ranges;
+        splits = int((small_chunks + per - 1) / per);
+    }
+    if (!small && reduce == 1 && splits > 1)  // drop the ranges that ceil(kt_total / splits) slices each would leave empty
         splits = (kt_total + (kt_total + splits - 1) / splits - 1) / ((kt_total + splits - 1) / splits);
     if (batch * splits > std::numeric_limits<int>::max()) fail(VC_HIP_ERR_OVERFLOW, "matmul batch too large");
     args.splits = splits;
-    args.kt_per_split = (kt_total + splits - 1) / splits;
+    args.kt_per_split = int(((small ? small_chunks : kt_total) + splits - 1) / splits);
     args.r_per_split = r_per_split;
-    Scratch partials(splits > 1 ? size_t(batch * splits) * size_t(M * N) * sizeof(float) : 4);
-    if (splits > 1) args.c = partials.as<float>();
+    Scratch partials(splits == 1 ? 4
+                                 : (small ? size_t(batch * tiles) * 1024 : size_t(batch) * size_t(M * N)) *
+                                       size_t(splits) * sizeof(float));
+    if (small) args.part = partials.as<float>();
+    else if (splits > 1) args.c = partials.as<float>();
     const dim3 grid(unsigned(tiles), unsigned(std::min<int64_t>(batch * splits, 65535)));
     const char* label = variant_label(ta, tb);
     const double flops = 2.0 * double(M) * double(N) * double(K) * double(batch) * double(reduce);
     // ReLU bitmasks go with gemm_big_kernel's epilogue for one product with A
-    // k-contiguous and no split. Elsewhere a consumer's bits are expanded into
-    // a float mask first (below), and a producer writes none.
-    const bool bits_here = big && !ta && batch == 1 && reduce == 1 && splits == 1;
-    Scratch expanded(relu_bits && !bits_here ? size_t(M * N) * sizeof(float) : 4);
+    // k-contiguous and no split; gemm_small_kernel reads them too. Elsewhere a
+    // consumer's bits are expanded into a float mask first (below), and a
+    // producer writes none.
+    const bool bits_here = big && !ta && batch == 1 && reduce == 1 && splits == 1 && (whole || mode == kGemmAuto);
+    const bool expand = relu_bits && !bits_here && !small;
+    Scratch expanded(expand ? size_t(M * N) * sizeof(float) : 4);
     const uint32_t* expand_from = nullptr;
-    if (relu_bits && !bits_here) {
+    if (expand) {
         expand_from = relu_bits;
         relu_bits = nullptr;
         relu_mask = expanded.as<float>();
@@ -1596,7 +1850,7 @@ void gemm(const float* a, const float* b, float* c, int64_t M, int64_t N, int64_
     // adds them next, or they are handed to the caller as pending sums. A
     // split product's C is summed again afterwards instead.
     ColsumPtr sums;
-    if (column_sum && splits == 1) sums = new_colsum(small ? tiles_m32 : simple ? tiles_m_simple : 2 * tiles_m, N);
+    if (column_sum && (splits == 1 || (small && K <= 2048))) sums = new_colsum(small ? tiles_m32 : simple ? tiles_m_simple : 2 * tiles_m, N);
     if (sums) args.col_part = sums->part;
     const double bytes =
         4.0 * (double(M * K + K * N) * double(reduce) + double(M * N) * (relu_mask ? 2.0 : 1.0)) * double(batch) +
@@ -1608,11 +1862,11 @@ void gemm(const float* a, const float* b, float* c, int64_t M, int64_t N, int64_
                dim3(256), 0, d.stream, expand_from, expanded.as<float>(), M, N);
         after_launch("relu_bits_expand");
     }
-    if (ta && tb) launch_variant<true, true>(args, vec, simple, small, big_n, grid, d.stream);
-    else if (ta) launch_variant<true, false>(args, vec, simple, small, big_n, grid, d.stream);
-    else if (tb) launch_variant<false, true>(args, vec, simple, small, big_n, grid, d.stream);
-    else launch_variant<false, false>(args, vec, simple, small, big_n, grid, d.stream);
-    if (splits > 1) {
+    if (ta && tb) launch_variant<true, true>(args, whole, simple, small, big_n, grid, d.stream);
+    else if (ta) launch_variant<true, false>(args, whole, simple, small, big_n, grid, d.stream);
+    else if (tb) launch_variant<false, true>(args, whole, simple, small, big_n, grid, d.stream);
+    else launch_variant<false, false>(args, whole, simple, small, big_n, grid, d.stream);
+    if (splits > 1 && !small) {
         after_launch(label);
         const int64_t total = batch * M * N;
         launch(split_sum_kernel, dim3(unsigned(std::min<int64_t>((total + 255) / 256, int64_t(d.cu_count) * 16))),
