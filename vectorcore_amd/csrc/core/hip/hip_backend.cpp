@@ -751,8 +751,9 @@ std::shared_ptr<Storage> HipBackend::binary(const Storage& a, std::size_t a_offs
     if (out_shape.size() > 8 || a_shape.size() > 8 || b_shape.size() > 8)
         throw std::invalid_argument("HIP broadcasting supports at most 8 dimensions");
     const std::size_t count = numel(out_shape);
-    // Both operands host-known scalars: the same fp32 operation on the host.
-    if (count == 1 && numel(a_shape) == 1 && numel(b_shape) == 1) {
+    // Both operands host-known scalars: the same fp32 operation on the host
+    // (broadcast to a larger shape, its result fills the output).
+    if (count > 0 && numel(a_shape) == 1 && numel(b_shape) == 1) {
         const auto sa = hip_host_scalar(a), sb = hip_host_scalar(b);
         if (sa && sb) {
             float r = 0.0F;
@@ -762,7 +763,7 @@ std::shared_ptr<Storage> HipBackend::binary(const Storage& a, std::size_t a_offs
                 case cpu::BinaryOp::Multiply: r = *sa * *sb; break;
                 case cpu::BinaryOp::Divide: r = *sa / *sb; break;
             }
-            return std::make_shared<HipStorage>(&r, 1);
+            return count == 1 ? std::make_shared<HipStorage>(&r, 1) : fill(count, r);
         }
     }
     // A host-known scalar against an output-shaped operand: the value goes in
@@ -1183,6 +1184,14 @@ std::pair<std::shared_ptr<Storage>, std::shared_ptr<Storage>> HipBackend::divide
     const Shape& out_shape, bool need_a, bool need_b) {
     require(*this);
     const std::size_t count = numel(out_shape);
+    // The gradient of a mean seeded with a host value, and alike: on the host.
+    if (count == 1 && need_a && !need_b) {
+        const auto g = hip_host_scalar(grad), d = hip_host_scalar(b);
+        if (g && d) {
+            const float r = *g / *d;
+            return {std::make_shared<HipStorage>(&r, 1), nullptr};
+        }
+    }
     if (deferring() && count > 0 && a_shape == out_shape && b_shape == out_shape && contiguous(a_shape, a_strides) &&
         contiguous(b_shape, b_strides)) {
         // grad / b and -(grad * a) / (b * b), as div_backward_kernel computes them.
