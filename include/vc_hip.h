@@ -363,6 +363,21 @@ int vc_hip_reduce_axis_noalloc(const float* in, float* out, size_t outer, size_t
 int vc_hip_scatter_axis(const float* values, const float* indices, float* out, size_t outer, size_t length,
                         size_t inner);
 
+/* ---- softmax --------------------------------------------------------------------- */
+/* Softmax (log_output == 0) or log-softmax along the middle axis of
+ * [outer, length, inner], as src/ops.cpp:416-424 composes it (maximum, then
+ * (x - m) - log(sum(exp(x - m))), the sum in double). stats receives the
+ * maximum and the sum of each of the outer * inner rows, interleaved, for the
+ * backward; NULL to leave them out. No counterpart in the reference's device
+ * interface, which runs the composition op by op. */
+int vc_hip_softmax_forward(const float* in, float* out, float* stats, size_t outer, size_t length, size_t inner,
+                           int log_output);
+/* The gradient of vc_hip_softmax_forward's input from the upstream gradient
+ * of its result, the input and the stats, as the composition's backward rules
+ * (src/ops.cpp:98-154, 346-374) give it. out must not overlap the inputs. */
+int vc_hip_softmax_backward(const float* grad, const float* in, const float* stats, float* out, size_t outer,
+                            size_t length, size_t inner, int log_output);
+
 /* ---- softmax cross-entropy (fused loss node for src/nn.cpp:31-53) ------------- */
 /* loss[0] = -(sum_i log_softmax(logits)_i[targets_i]) / rows, with the
  * reference's composition order; row_stats[2*i] = row max, row_stats[2*i+1] =

@@ -30,7 +30,7 @@ OBJ = PKG / "_build"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-HIP_SOURCES = ["runtime.hip", "elementwise.hip", "reduce.hip", "xent.hip", "gemm.hip", "fused_map.hip"]
+HIP_SOURCES = ["runtime.hip", "elementwise.hip", "reduce.hip", "xent.hip", "softmax.hip", "gemm.hip", "fused_map.hip"]
 # Sources compiled once per define set: the fused-map interpreters, one object
 # per input count, so that they compile in parallel.
 HIP_VARIANT_SOURCES = {"fused_map_inputs.hip": [[f"-DVC_MAP_NIN={k}"] for k in range(1, 9)]}

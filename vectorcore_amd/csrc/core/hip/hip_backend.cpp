@@ -271,6 +271,13 @@ public:
         return *deferred_;
     }
 
+    // The contents a snapshot stands for (HipBackend::snapshot), read where they are.
+    const float* snapshot_ptr() const {
+        std::lock_guard<std::recursive_mutex> lock(state_mutex());
+        if (map_ && map_->kind == MapNode::Kind::Input) return map_->input->ptr() + map_->offset;
+        return ptr();
+    }
+
     // The pending elementwise expression of this storage, if any.
     MapExpr map_expr() const {
         std::lock_guard<std::recursive_mutex> lock(state_mutex());
@@ -1175,6 +1182,42 @@ std::shared_ptr<Storage> HipBackend::activation_backward(Activation kind, const 
         case Activation::Log: status = vc_hip_log_backward(g, s, out->ptr(), count); break;
     }
     check(status, "HIP activation backward failed");
+    return out;
+}
+
+std::pair<std::shared_ptr<Storage>, std::shared_ptr<Storage>> HipBackend::softmax_forward(
+    const Storage& input, std::size_t offset, std::size_t outer, std::size_t length, std::size_t inner, bool log_output) {
+    require(*this);
+    auto out = fresh(outer * length * inner);
+    auto stats = fresh(2 * outer * inner);
+    check(vc_hip_softmax_forward(dptr(input, offset), out->ptr(), stats->ptr(), outer, length, inner, log_output ? 1 : 0),
+          "HIP softmax failed");
+    return {out, stats};
+}
+
+std::shared_ptr<Storage> HipBackend::softmax_backward(const Storage& grad, std::size_t grad_offset, const Storage& input,
+                                                      const Storage& stats, std::size_t outer, std::size_t length,
+                                                      std::size_t inner, bool log_output) {
+    require(*this);
+    auto out = fresh(outer * length * inner);
+    check(vc_hip_softmax_backward(dptr(grad, grad_offset), as_hip(input).snapshot_ptr(), dptr(stats, 0), out->ptr(), outer,
+                                  length, inner, log_output ? 1 : 0),
+          "HIP softmax backward failed");
+    return out;
+}
+
+std::shared_ptr<Storage> HipBackend::snapshot(const std::shared_ptr<Storage>& source, std::size_t offset,
+                                              std::size_t count) {
+    auto h = std::dynamic_pointer_cast<HipStorage>(source);
+    if (!h) throw std::invalid_argument("expected HIP storage");
+    if (offset + count > h->size()) throw std::out_of_range("HIP snapshot exceeds storage");
+    (void)h->ptr();
+    auto n = std::make_shared<MapNode>();
+    n->kind = MapNode::Kind::Input;
+    n->input = h;
+    n->offset = offset;
+    auto out = std::make_shared<HipStorage>(count, MapExpr(std::move(n)));
+    h->add_reader(out);  // an in-place write of the source hands this storage the buffer with the old contents
     return out;
 }
 

@@ -143,6 +143,21 @@ public:
     [[nodiscard]] bool fuse_elementwise() const;
 
     // --- fused kernels used by the hip arm of the backward rules ---
+    // Softmax or log-softmax along the middle axis, with the rows' maxima and
+    // sums for softmax_backward.
+    [[nodiscard]] std::pair<std::shared_ptr<Storage>, std::shared_ptr<Storage>> softmax_forward(
+        const Storage& input, std::size_t offset, std::size_t outer, std::size_t length, std::size_t inner,
+        bool log_output);
+    // `input`: a snapshot of the forward's input.
+    [[nodiscard]] std::shared_ptr<Storage> softmax_backward(const Storage& grad, std::size_t grad_offset,
+                                                            const Storage& input, const Storage& stats,
+                                                            std::size_t outer, std::size_t length, std::size_t inner,
+                                                            bool log_output);
+    // The current contents of elements [offset, offset + count) of a storage,
+    // for a backward rule that reads them later: a later in-place write of the
+    // storage leaves them (nothing is copied until then).
+    [[nodiscard]] std::shared_ptr<Storage> snapshot(const std::shared_ptr<Storage>& source, std::size_t offset,
+                                                    std::size_t count);
     [[nodiscard]] std::shared_ptr<Storage> fill(std::size_t count, float value);
     // out = a op s (scalar_first false) or s op a; s is a host value.
     [[nodiscard]] std::shared_ptr<Storage> binary_scalar(const Storage& a, std::size_t a_offset, std::size_t count,

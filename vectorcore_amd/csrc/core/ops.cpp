@@ -549,13 +549,45 @@ Tensor sigmoid(const Tensor& v) {
     return out;
 }
 
+namespace {
+
+// hip: softmax or log-softmax as one node, its two directions one kernel each.
+// The rule reads a snapshot of v, which the composition does not save either;
+// softmax's checks its result's version, as the composition's exp does. Not
+// for few long columns, where a workgroup per 16 columns leaves the chip idle:
+// the composition's reductions split the axis.
+std::optional<Tensor> softmax_hip(const Tensor& v, std::int64_t axis, bool log_output) {
+    if (v.device() != Device::hip()) return std::nullopt;
+    const AxisSplit s = split_axis(v.shape(), axis);
+    const std::size_t count = v.numel();
+    if (count == 0 || (s.inner > 1 && s.length > 512 && s.outer * ((s.inner + 15) / 16) < 128)) return std::nullopt;
+    auto [result, stats] = hip().softmax_forward(st(v), off(v), s.outer, s.length, s.inner, log_output);
+    Tensor out = detail::make_tensor(std::move(result), v.shape(), false);
+    if (!grad_enabled() || !v.requires_grad()) return out;
+    const std::shared_ptr<Storage> input = hip().snapshot(v.impl()->storage, off(v), count), rows = std::move(stats);
+    std::optional<detail::SavedTensor> saved;
+    if (!log_output) saved.emplace(out);
+    detail::attach_grad_fn(out, {v}, [input, rows, saved, s, log_output](const Tensor& g) {
+        if (saved) (void)saved->unpack();
+        return std::vector<Tensor>{detail::make_tensor(
+            hip().softmax_backward(st(g), off(g), *input, *rows, s.outer, s.length, s.inner, log_output), g.shape(), false)};
+    });
+    return out;
+}
+
+}  // namespace
+
 // log_softmax(x) = (x - m) - log(sum(exp(x - m))), m = max(x.detach()): the
 // shift keeps exp() finite and, being constant, leaves the gradient exact.
 Tensor log_softmax(const Tensor& v, std::int64_t axis) {
+    if (std::optional<Tensor> fused = softmax_hip(v, axis, true)) return *fused;
     const Tensor shifted = v - max(v.detach(), axis, true);
     return shifted - log(sum(exp(shifted), axis, true));
 }
 
-Tensor softmax(const Tensor& v, std::int64_t axis) { return exp(log_softmax(v, axis)); }
+Tensor softmax(const Tensor& v, std::int64_t axis) {
+    if (std::optional<Tensor> fused = softmax_hip(v, axis, false)) return *fused;
+    return exp(log_softmax(v, axis));
+}
 
 }  // namespace vectorcore
