@@ -252,6 +252,32 @@ typedef struct vc_hip_map_program {
     size_t rows, cols;
 } vc_hip_map_program;
 int vc_hip_map(const vc_hip_map_program* program);
+/* vc_hip_map over a rows x cols matrix with inputs that broadcast to it, and
+ * row sums: what a backward pass through means, broadcast products and
+ * quotients, and maxima along an axis computes between its reductions
+ * (src/ops.cpp:98-154, 268-352; src/autograd.cpp:50-91). Input j has, by
+ * input_kinds[j], one value per element, per column (cols values), per row
+ * (rows values) or, the rows being groups of axis_length, per group and column
+ * (rows / axis_length * cols values; axis_length divides rows). Two more
+ * operations: AT_ROW gives slot b where int(slot a) is the row's number within
+ * its group and 0 elsewhere, AT_COLUMN the same for the column (the gradient
+ * of a maximum along an axis). row_sums[s] ([rows]) receives the sums of slot
+ * row_sum_slots[s] over the columns, added in double in a fixed order; a
+ * program has row sums or column sums. Fewer than 2^31 elements, at least one. */
+#define VC_MAP_AT_ROW 6
+#define VC_MAP_AT_COLUMN 7
+#define VC_MAP_FULL 0
+#define VC_MAP_PER_COLUMN 1
+#define VC_MAP_PER_ROW 2
+#define VC_MAP_PER_GROUP 3
+typedef struct vc_hip_map_matrix {
+    unsigned char input_kinds[VC_HIP_MAP_INPUTS];
+    size_t axis_length;
+    float* row_sums[VC_HIP_MAP_SUMS];
+    unsigned char row_sum_slots[VC_HIP_MAP_SUMS];
+    size_t n_row_sums;
+} vc_hip_map_matrix;
+int vc_hip_map_broadcast(const vc_hip_map_program* program, const vc_hip_map_matrix* matrix);
 
 /* ---- matrix multiply ------------------------------------------------------- */
 /* MetalBackend::matmul (metal_backend.hpp:34-40): for z < batch,

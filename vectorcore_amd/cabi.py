@@ -40,6 +40,15 @@ class MapProgram(ctypes.Structure):
                 ("rows", _sz), ("cols", _sz)]
 
 
+MAP_AT_ROW, MAP_AT_COLUMN = 6, 7
+MAP_FULL, MAP_PER_COLUMN, MAP_PER_ROW, MAP_PER_GROUP = range(4)
+
+
+class MapMatrix(ctypes.Structure):
+    _fields_ = [("input_kinds", ctypes.c_ubyte * MAP_INPUTS), ("axis_length", _sz), ("row_sums", _vp * MAP_SUMS),
+                ("row_sum_slots", ctypes.c_ubyte * MAP_SUMS), ("n_row_sums", _sz)]
+
+
 def map_word(op: int, a: int, b: int, dst: int) -> int:
     """One instruction of a vc_hip_map program: slot[dst] = slot[a] op slot[b]."""
     return op | a << 8 | b << 16 | dst << 24
@@ -103,6 +112,7 @@ _SIGNATURES = {
     "vc_hip_exp_backward": ([_vp, _vp, _vp, _sz], _i),
     "vc_hip_log_backward": ([_vp, _vp, _vp, _sz], _i),
     "vc_hip_div_backward": ([_vp, _vp, _szp, _szp, _sz, _vp, _szp, _szp, _sz, _szp, _sz, _vp, _vp], _i),
+    "vc_hip_map_broadcast": ([ctypes.POINTER(MapProgram), ctypes.POINTER(MapMatrix)], _i),
     "vc_hip_map": ([ctypes.POINTER(MapProgram)], _i),
     "vc_hip_matmul": ([_vp, _vp, _vp, _sz, _sz, _sz, _szp, _szp, _sz, _i, _i], _i),
     "vc_hip_matmul_relu_mask": ([_vp, _vp, _vp, _sz, _sz, _sz, _szp, _szp, _sz, _i, _i, _vp], _i),

@@ -18,6 +18,7 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <tuple>
 #include <unordered_map>
 
 namespace vectorcore {
@@ -82,6 +83,11 @@ struct MapNode {
     std::shared_ptr<HipStorage> input;
     std::size_t offset = 0;
     float value = 0.0F;
+    // How an input broadcasts to the expression's elements viewed as a matrix
+    // (VC_MAP_FULL ...), and what that (or an AT operation) asks of the view:
+    // its columns and its groups of rows (0: nothing).
+    unsigned char input_kind = VC_MAP_FULL;
+    std::size_t cols = 0, axis_length = 0;
 };
 using MapExpr = std::shared_ptr<MapNode>;
 
@@ -106,9 +112,10 @@ public:
     // The values of a deferred elementwise expression (computed on first use
     // or by HipBackend::flush_elementwise).
     HipStorage(std::size_t elements, MapExpr expr) : elements_(elements), map_(std::move(expr)), shadow_valid_(false) {}
-    // The column sums of a deferred expression viewed as [rows, elements].
-    HipStorage(std::size_t elements, MapExpr expr, std::size_t rows)
-        : elements_(elements), sum_of_(std::move(expr)), sum_rows_(rows), shadow_valid_(false) {}
+    // The column sums of a deferred expression viewed as [summed, elements],
+    // or its row sums viewed as [elements, summed].
+    HipStorage(std::size_t elements, MapExpr expr, std::size_t summed, bool row_sums)
+        : elements_(elements), sum_of_(std::move(expr)), summed_(summed), row_sums_(row_sums), shadow_valid_(false) {}
 
     ~HipStorage() override {
         if (mirror_) (void)vc_hip_mirror_release(mirror_);
@@ -284,7 +291,10 @@ public:
         return map_;
     }
     MapExpr sum_expr() const { return sum_of_; }
-    std::size_t sum_rows() const { return sum_rows_; }
+    // The matrix that a pending sum adds up.
+    std::size_t sum_rows() const { return row_sums_ ? elements_ : summed_; }
+    std::size_t sum_cols() const { return row_sums_ ? summed_ : elements_; }
+    bool row_sums() const { return row_sums_; }
     bool map_pending() const { return map_ != nullptr || sum_of_ != nullptr; }
     // Takes the buffer a program wrote this storage's values into, and drops
     // the expression (and with it the references to its inputs).
@@ -363,8 +373,9 @@ private:
     std::vector<float> shadow_;
     mutable std::unique_ptr<DeferredProduct> deferred_;
     mutable MapExpr map_;     // deferred elementwise values
-    mutable MapExpr sum_of_;  // deferred column sums of this expression
-    std::size_t sum_rows_ = 0;
+    mutable MapExpr sum_of_;  // deferred column or row sums of this expression
+    std::size_t summed_ = 0;
+    bool row_sums_ = false;
     std::vector<std::weak_ptr<HipStorage>> readers_;
     vc_hip_mirror* mirror_ = nullptr;  // published value of a one-element result
     mutable vc_hip_colsum* pending_sums_ = nullptr;  // see set_pending_sums
@@ -448,6 +459,7 @@ struct MapPlan {
     std::vector<float> constants;
     std::vector<std::uint32_t> code;
     std::unordered_map<const MapNode*, int> root_slot;
+    std::size_t cols = 0, axis_length = 0;  // the matrix view asked for (0: any)
 };
 
 bool plan_program(const std::vector<const MapNode*>& roots, MapPlan& plan) {
@@ -455,12 +467,20 @@ bool plan_program(const std::vector<const MapNode*>& roots, MapPlan& plan) {
     std::vector<const MapNode*> order;
     for (const MapNode* r : roots) collect(r, seen, order);
     std::vector<const MapNode*> ops;
-    std::vector<std::pair<const HipStorage*, std::size_t>> input_keys;
+    std::vector<std::tuple<const HipStorage*, std::size_t, unsigned char>> input_keys;
     std::vector<std::uint32_t> const_bits;
+    // One view for the whole program.
+    for (const MapNode* n : order) {
+        if ((n->cols && plan.cols && n->cols != plan.cols) ||
+            (n->axis_length && plan.axis_length && n->axis_length != plan.axis_length))
+            return false;
+        if (n->cols) plan.cols = n->cols;
+        if (n->axis_length) plan.axis_length = n->axis_length;
+    }
     std::unordered_map<const MapNode*, int> vid;  // value id: input index, then constants, then op index
     for (const MapNode* n : order) {
         if (n->kind == MapNode::Kind::Input) {
-            const std::pair<const HipStorage*, std::size_t> key{n->input.get(), n->offset};
+            const std::tuple<const HipStorage*, std::size_t, unsigned char> key{n->input.get(), n->offset, n->input_kind};
             auto it = std::find(input_keys.begin(), input_keys.end(), key);
             if (it == input_keys.end()) {
                 input_keys.push_back(key);
@@ -524,8 +544,10 @@ bool plan_program(const std::vector<const MapNode*>& roots, MapPlan& plan) {
     return true;
 }
 
-bool fits(const std::vector<const MapNode*>& roots) {
+// cols: the columns that a sum among the roots asks for (0: any).
+bool fits(const std::vector<const MapNode*>& roots, std::size_t cols = 0) {
     MapPlan plan;
+    plan.cols = cols;
     return plan_program(roots, plan);
 }
 
@@ -539,6 +561,7 @@ void run_maps(const std::vector<HipStorage*>& requested) {
     std::vector<const MapNode*> roots;
     std::size_t count = 0, rows = 0, cols = 0;
     std::size_t n_out = 0, n_sum = 0;
+    bool row_sums = false;
     for (HipStorage* o : outputs) {
         if (MapExpr m = o->map_expr()) {
             roots.push_back(m.get());
@@ -547,18 +570,26 @@ void run_maps(const std::vector<HipStorage*>& requested) {
         } else if (MapExpr e = o->sum_expr()) {
             roots.push_back(e.get());
             rows = o->sum_rows();
-            cols = o->size();
+            cols = o->sum_cols();
+            row_sums = o->row_sums();
             count = rows * cols;
             ++n_sum;
         }
     }
     if (roots.empty()) return;
     MapPlan plan;
+    plan.cols = cols;
     if (n_out > VC_HIP_MAP_OUTPUTS || n_sum > VC_HIP_MAP_SUMS || !plan_program(roots, plan))
         throw std::logic_error("deferred elementwise expression exceeds one program");
     vc_hip_map_program prog{};
-    for (std::size_t j = 0; j < plan.inputs.size(); ++j)
+    vc_hip_map_matrix matrix{};
+    bool broadcasts = row_sums;
+    for (const std::uint32_t word : plan.code) broadcasts = broadcasts || (word & 255U) > VC_MAP_STEP;
+    for (std::size_t j = 0; j < plan.inputs.size(); ++j) {
         prog.inputs[j] = plan.inputs[j]->input->ptr() + plan.inputs[j]->offset;
+        matrix.input_kinds[j] = plan.inputs[j]->input_kind;
+        broadcasts = broadcasts || matrix.input_kinds[j] != VC_MAP_FULL;
+    }
     prog.n_inputs = plan.inputs.size();
     for (std::size_t c = 0; c < plan.constants.size(); ++c) prog.constants[c] = plan.constants[c];
     prog.n_constants = plan.constants.size();
@@ -580,19 +611,18 @@ void run_maps(const std::vector<HipStorage*>& requested) {
         if (outputs[i]->map_expr()) {
             prog.outputs[prog.n_outputs] = static_cast<float*>(b);
             prog.output_slots[prog.n_outputs++] = slot;
+        } else if (row_sums) {
+            matrix.row_sums[matrix.n_row_sums] = static_cast<float*>(b);
+            matrix.row_sum_slots[matrix.n_row_sums++] = slot;
         } else {
             prog.sums[prog.n_sums] = static_cast<float*>(b);
             prog.sum_slots[prog.n_sums++] = slot;
         }
     }
-    if (n_sum > 0) {
-        prog.rows = rows;
-        prog.cols = cols;
-    } else {
-        prog.rows = 1;
-        prog.cols = count;
-    }
-    const int status = count || n_sum ? vc_hip_map(&prog) : VC_HIP_OK;
+    prog.cols = plan.cols ? plan.cols : count;
+    prog.rows = n_sum > 0 ? rows : plan.cols ? count / plan.cols : 1;
+    matrix.axis_length = plan.axis_length ? plan.axis_length : 1;
+    const int status = !count && !n_sum ? VC_HIP_OK : broadcasts ? vc_hip_map_broadcast(&prog, &matrix) : vc_hip_map(&prog);
     if (status != VC_HIP_OK) {
         release_all();
         throw_status(status, "HIP fused elementwise pass failed");
@@ -656,14 +686,60 @@ void expr_inputs(const MapNode& root, std::vector<std::shared_ptr<HipStorage>>& 
             out.push_back(n->input);
 }
 
-std::shared_ptr<HipStorage> pending_storage(std::size_t elements, MapExpr expr, std::size_t sum_rows = 0) {
-    auto out = sum_rows ? std::make_shared<HipStorage>(elements, expr, sum_rows)
-                        : std::make_shared<HipStorage>(elements, expr);
+std::shared_ptr<HipStorage> pending_storage(std::size_t elements, MapExpr expr, std::size_t summed = 0,
+                                            bool row_sums = false) {
+    auto out = summed ? std::make_shared<HipStorage>(elements, expr, summed, row_sums)
+                      : std::make_shared<HipStorage>(elements, expr);
     std::vector<std::shared_ptr<HipStorage>> inputs;
     expr_inputs(*expr, inputs);
     for (const auto& in : inputs) in->add_reader(out);
     t_pending.push_back(out);
     return out;
+}
+
+// How an operand of `shape` (contiguous) broadcasts to out_shape viewed as a
+// matrix: the input kind, with the columns and the axis length it asks for;
+// nothing when no view fits (or the matrix has 2^31 elements).
+struct Broadcast {
+    unsigned char kind = VC_MAP_FULL;
+    std::size_t cols = 0, axis_length = 0;
+};
+std::optional<Broadcast> broadcast_of(const Shape& shape, const Strides& strides, const Shape& out_shape) {
+    if (strides != contiguous_strides(shape)) return std::nullopt;
+    if (shape == out_shape) return Broadcast{};
+    const std::size_t count = numel(out_shape);
+    if (count == 0 || count >= (std::size_t(1) << 31) || shape.size() > out_shape.size()) return std::nullopt;
+    // Runs of axes that the operand has (kept) or repeats over, outermost first; axes of 1 belong to any.
+    std::vector<std::pair<bool, std::size_t>> runs;
+    for (std::size_t ax = 0; ax < out_shape.size(); ++ax) {
+        if (out_shape[ax] == 1) continue;
+        const std::size_t lead = out_shape.size() - shape.size();
+        const std::size_t extent = ax < lead ? 1 : shape[ax - lead];
+        if (extent != 1 && extent != out_shape[ax]) return std::nullopt;
+        if (!runs.empty() && runs.back().first == (extent != 1)) runs.back().second *= out_shape[ax];
+        else runs.emplace_back(extent != 1, out_shape[ax]);
+    }
+    const std::size_t n = runs.size();
+    if (n == 0 || (n == 1 && runs[0].first)) return Broadcast{};
+    if (n == 1) return Broadcast{VC_MAP_PER_ROW, count, 0};  // one value: one row
+    if (n == 2) return runs[0].first ? Broadcast{VC_MAP_PER_ROW, runs[1].second, 0} : Broadcast{VC_MAP_PER_COLUMN, runs[1].second, 0};
+    if (n == 3 && runs[0].first) return Broadcast{VC_MAP_PER_GROUP, runs[2].second, runs[1].second};
+    return std::nullopt;
+}
+
+// The expression of an operand that broadcasts to `count` values.
+MapExpr broadcast_expr(const Storage& s, std::size_t offset, std::size_t count, const Broadcast& b) {
+    if (b.kind == VC_MAP_FULL) return operand_expr(s, offset, count);
+    const auto& h = as_hip(s);
+    auto n = std::make_shared<MapNode>();
+    n->kind = MapNode::Kind::Input;
+    (void)h.ptr();
+    n->input = std::const_pointer_cast<HipStorage>(h.shared_from_this());
+    n->offset = offset;
+    n->input_kind = b.kind;
+    n->cols = b.cols;
+    n->axis_length = b.axis_length;
+    return n;
 }
 
 // A deferred elementwise operation on `count` values: build(x...) makes the
@@ -672,11 +748,12 @@ std::shared_ptr<HipStorage> pending_storage(std::size_t elements, MapExpr expr, 
 // largest) and become inputs.
 template <typename Build>
 std::shared_ptr<Storage> deferred_map(std::size_t count, std::vector<std::pair<const Storage*, std::size_t>> operands,
-                                      Build build) {
+                                      Build build, const std::vector<Broadcast>& views = {}) {
     std::lock_guard<std::recursive_mutex> lock(state_mutex());
     for (std::size_t round = 0; round <= operands.size(); ++round) {
         std::vector<MapExpr> ex;
-        for (const auto& [s, off] : operands) ex.push_back(operand_expr(*s, off, count));
+        for (std::size_t i = 0; i < operands.size(); ++i)
+            ex.push_back(broadcast_expr(*operands[i].first, operands[i].second, count, views.empty() ? Broadcast{} : views[i]));
         MapExpr e = build(ex);
         if (fits({e.get()})) return pending_storage(count, std::move(e));
         // Compute the operand expression with the most operations first.
@@ -698,7 +775,11 @@ std::shared_ptr<Storage> deferred_map(std::size_t count, std::vector<std::pair<c
     throw std::logic_error("elementwise expression does not fit one program");
 }
 
-bool contiguous(const Shape& shape, const Strides& strides) { return strides == contiguous_strides(shape); }
+// Whether one matrix view serves both operands.
+bool views_agree(const Broadcast& a, const Broadcast& b) {
+    return (!a.cols || !b.cols || a.cols == b.cols) &&
+           (!a.axis_length || !b.axis_length || a.axis_length == b.axis_length);
+}
 
 }  // namespace
 
@@ -781,11 +862,21 @@ std::shared_ptr<Storage> HipBackend::binary(const Storage& a, std::size_t a_offs
     if (b_shape == out_shape && numel(a_shape) == 1) {
         if (auto s = hip_host_scalar(a)) return binary_scalar(b, b_offset, count, *s, true, operation);
     }
-    if (deferring() && count > 0 && a_shape == out_shape && b_shape == out_shape && contiguous(a_shape, a_strides) &&
-        contiguous(b_shape, b_strides)) {
+    if (deferring() && count > 0) {
         const int op = binary_code(operation);  // VC_MAP_ADD..VC_MAP_DIV share the binary codes
-        return deferred_map(count, {{&a, a_offset}, {&b, b_offset}},
-                            [op](std::vector<MapExpr>& x) { return op_expr(op, x[0], x[1]); });
+        const auto va = broadcast_of(a_shape, a_strides, out_shape), vb = broadcast_of(b_shape, b_strides, out_shape);
+        // Expanding a gradient (detail::broadcast_to): an operand and a host-known zero, both smaller.
+        const auto ka = numel(a_shape) == 1 ? hip_host_scalar(a) : std::nullopt;
+        const auto kb = numel(b_shape) == 1 ? hip_host_scalar(b) : std::nullopt;
+        if (va && kb)
+            return deferred_map(count, {{&a, a_offset}},
+                                [op, kb](std::vector<MapExpr>& x) { return op_expr(op, x[0], constant_expr(*kb)); }, {*va});
+        if (vb && ka)
+            return deferred_map(count, {{&b, b_offset}},
+                                [op, ka](std::vector<MapExpr>& x) { return op_expr(op, constant_expr(*ka), x[0]); }, {*vb});
+        if (va && vb && views_agree(*va, *vb))
+            return deferred_map(count, {{&a, a_offset}, {&b, b_offset}},
+                                [op](std::vector<MapExpr>& x) { return op_expr(op, x[0], x[1]); }, {*va, *vb});
     }
     auto out = fresh(count);
     if (count == 0) return out;
@@ -945,8 +1036,17 @@ std::shared_ptr<Storage> HipBackend::reduce_axis(const Storage& input, std::size
         // Column sums of a pending expression: one more output of its program.
         if (deferring() && length > 0 && inner >= 64 && length * inner == input.size()) {
             std::lock_guard<std::recursive_mutex> lock(state_mutex());
-            if (MapExpr e = as_hip(input).map_expr()) return pending_storage(inner, e, length);
+            if (MapExpr e = as_hip(input).map_expr())
+                if (fits({e.get()}, inner)) return pending_storage(inner, e, length);
         }
+    }
+    // Row sums of a pending expression: summed as it is computed. (It is computed again where something
+    // else reads it, from inputs that this program has just read.)
+    if (operation == cpu::ReduceOp::Sum && inner == 1 && offset == 0 && outer > 1 && length > 1 && deferring() &&
+        outer * length == input.size() && input.size() < (std::size_t(1) << 31)) {
+        std::lock_guard<std::recursive_mutex> lock(state_mutex());
+        if (MapExpr e = as_hip(input).map_expr())
+            if (e->kind == MapNode::Kind::Op && fits({e.get()}, length)) return pending_storage(outer, e, length, true);
     }
     auto out = fresh(outer * inner);
     if (outer * inner == 0) return out;
@@ -960,6 +1060,20 @@ std::shared_ptr<Storage> HipBackend::scatter_axis(const Storage& values, std::si
                                                   const Storage& indices, std::size_t indices_offset,
                                                   std::size_t outer, std::size_t length, std::size_t inner) {
     require(*this);
+    const std::size_t count = outer * length * inner;
+    if (deferring() && count > 0 && count < (std::size_t(1) << 31)) {
+        // Where the index is the position along the axis, the value: one
+        // operation of the pass's expressions.
+        const bool last = inner == 1;
+        const Broadcast view = last ? Broadcast{VC_MAP_PER_ROW, length, 0} : Broadcast{VC_MAP_PER_GROUP, inner, length};
+        return deferred_map(count, {{&indices, indices_offset}, {&values, values_offset}},
+                            [last, view](std::vector<MapExpr>& x) {
+                                MapExpr e = op_expr(last ? VC_MAP_AT_COLUMN : VC_MAP_AT_ROW, x[0], x[1]);
+                                e->cols = view.cols;
+                                e->axis_length = view.axis_length;
+                                return e;
+                            }, {view, view});
+    }
     auto out = fresh(outer * length * inner);
     if (outer * length * inner == 0) return out;
     check(vc_hip_scatter_axis(dptr(values, values_offset), dptr(indices, indices_offset), out->ptr(), outer, length,
@@ -1045,23 +1159,24 @@ void HipBackend::flush_elementwise() {
     // can share a pass with, then the remaining expressions, as many per
     // program as fit.
     std::vector<bool> done(live.size(), false);
-    auto elements_of = [](const HipStorage& h) { return h.sum_expr() ? h.sum_rows() * h.size() : h.size(); };
+    auto elements_of = [](const HipStorage& h) { return h.sum_expr() ? h.sum_rows() * h.sum_cols() : h.size(); };
     for (int sums_first = 1; sums_first >= 0; --sums_first) {
         for (std::size_t i = 0; i < live.size(); ++i) {
             if (done[i] || (sums_first != 0) != (live[i]->sum_expr() != nullptr)) continue;
             std::vector<HipStorage*> group{live[i].get()};
             std::vector<const MapNode*> roots{live[i]->sum_expr() ? live[i]->sum_expr().get() : live[i]->map_expr().get()};
             std::size_t n_out = live[i]->sum_expr() ? 0 : 1, n_sum = live[i]->sum_expr() ? 1 : 0;
+            const std::size_t cols = live[i]->sum_expr() ? live[i]->sum_cols() : 0;
             done[i] = true;
             for (std::size_t j = i + 1; j < live.size(); ++j) {
                 if (done[j] || elements_of(*live[j]) != elements_of(*live[i])) continue;
                 const bool sum = live[j]->sum_expr() != nullptr;
-                if (sum && (n_sum == VC_HIP_MAP_SUMS || (n_sum > 0 && live[j]->size() != group[0]->size()) ||
-                            (n_sum == 0)))
+                if (sum && (n_sum == VC_HIP_MAP_SUMS || n_sum == 0 || live[j]->sum_cols() != cols ||
+                            live[j]->row_sums() != group[0]->row_sums()))
                     continue;
                 if (!sum && n_out == VC_HIP_MAP_OUTPUTS) continue;
                 roots.push_back(sum ? live[j]->sum_expr().get() : live[j]->map_expr().get());
-                if (!fits(roots)) {
+                if (!fits(roots, cols)) {
                     roots.pop_back();
                     continue;
                 }
@@ -1235,19 +1350,20 @@ std::pair<std::shared_ptr<Storage>, std::shared_ptr<Storage>> HipBackend::divide
             return {std::make_shared<HipStorage>(&r, 1), nullptr};
         }
     }
-    if (deferring() && count > 0 && a_shape == out_shape && b_shape == out_shape && contiguous(a_shape, a_strides) &&
-        contiguous(b_shape, b_strides)) {
+    const auto va = deferring() && count > 0 ? broadcast_of(a_shape, a_strides, out_shape) : std::nullopt;
+    const auto vb = deferring() && count > 0 ? broadcast_of(b_shape, b_strides, out_shape) : std::nullopt;
+    if (va && vb && views_agree(*va, *vb)) {
         // grad / b and -(grad * a) / (b * b), as div_backward_kernel computes them.
         std::shared_ptr<Storage> da, db;
         if (need_a)
             da = deferred_map(count, {{&grad, grad_offset}, {&b, b_offset}},
-                              [](std::vector<MapExpr>& x) { return op_expr(VC_MAP_DIV, x[0], x[1]); });
+                              [](std::vector<MapExpr>& x) { return op_expr(VC_MAP_DIV, x[0], x[1]); }, {Broadcast{}, *vb});
         if (need_b)
             db = deferred_map(count, {{&grad, grad_offset}, {&a, a_offset}, {&b, b_offset}},
                               [](std::vector<MapExpr>& x) {
                                   return op_expr(VC_MAP_DIV, op_expr(VC_MAP_NEG, op_expr(VC_MAP_MUL, x[0], x[1]), nullptr),
                                                  op_expr(VC_MAP_MUL, x[2], x[2]));
-                              });
+                              }, {Broadcast{}, *va, *vb});
         return {da, db};
     }
     std::shared_ptr<HipStorage> ga = need_a ? fresh(count) : nullptr;

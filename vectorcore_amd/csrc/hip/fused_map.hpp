@@ -4,7 +4,10 @@
 // interpreters compile in parallel; fused_map.hip holds the C ABI.
 #pragma once
 
+#include "reduce_common.hpp"
 #include "vc_hip_internal.hpp"
+
+#include <algorithm>
 
 namespace vchip {
 namespace fmap {
@@ -25,12 +28,52 @@ static_assert(kSlots == 16, "a slot is one element of a 16-wide register vector"
 struct Program {
     const float* in[kInputs];
     float* out[kOutputs];
+    float* sum[kSums];  // row sums (map_rows_kernel)
     float konst[kConsts];
     uint32_t code[kCode];  // op | a << 8 | b << 16 | dst << 24
     int n_code, n_const, n_out, n_sum;
     uint8_t out_slot[kOutputs];
     uint8_t sum_slot[kSums];
+    // Matrix programs (vc_hip_map_broadcast): how each input is indexed
+    // (VC_MAP_FULL ...), and the matrix.
+    uint8_t kind[kInputs];
+    uint32_t cols, len;
 };
+
+// The matrix coordinates of a thread's W values: row (group of rows and row in
+// the group) and column of each, and whether they lie in one row.
+template <int W>
+struct Place {
+    uint32_t r[W], group[W], in_group[W], c[W];
+    bool one_row;
+    // Columns c0 .. c0 + W - 1 of row r0, running on into the next rows.
+    __device__ void set(const Program& P, uint32_t r0, uint32_t c0) {
+        one_row = c0 + W <= P.cols;
+        uint32_t g0 = r0, a0 = 0;
+        if (P.len != 1) g0 = r0 / P.len, a0 = r0 - g0 * P.len;
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+            r[j] = r0, group[j] = g0, in_group[j] = a0, c[j] = c0;
+            if (++c0 == P.cols) {
+                c0 = 0, ++r0;
+                if (++a0 == P.len) a0 = 0, ++g0;
+            }
+        }
+    }
+};
+template <int W>
+__device__ inline Place<W> place_of(const Program& P, uint32_t e) {  // elements e .. e + W - 1
+    Place<W> at;
+    const uint32_t r = e / P.cols;
+    at.set(P, r, e - r * P.cols);
+    return at;
+}
+template <int W>
+__device__ inline Place<W> place_at(const Program& P, uint32_t r, uint32_t c) {
+    Place<W> at;
+    at.set(P, r, c);
+    return at;
+}
 
 // W values per slot: one element (W = 1) or four consecutive ones (W = 4).
 template <int W>
@@ -70,6 +113,12 @@ __device__ inline Vals<W> load(const float* __restrict__ p) {
     return o;
 }
 template <int W>
+__device__ inline void store_any(float* __restrict__ p, const Vals<W>& v) {
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+    if constexpr (W == 4) *reinterpret_cast<f4u*>(p) = f4{v.v[0], v.v[1], v.v[2], v.v[3]};
+    else p[0] = v.v[0];
+}
+template <int W>
 __device__ inline void store(float* __restrict__ p, const Vals<W>& v) {
     if constexpr (W == 4) {
         __builtin_nontemporal_store(f4{v.v[0], v.v[1], v.v[2], v.v[3]}, reinterpret_cast<f4*>(p));
@@ -78,10 +127,26 @@ __device__ inline void store(float* __restrict__ p, const Vals<W>& v) {
     }
 }
 
+// W consecutive values on any 4-byte boundary, through the caches (vectors
+// that every row reads; a 16-byte load needs 4-byte alignment only).
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+template <int W>
+__device__ inline Vals<W> load_any(const float* __restrict__ p) {
+    Vals<W> o;
+    if constexpr (W == 4) {
+        const f4 x = *reinterpret_cast<const f4u*>(p);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o.v[j] = x[j];
+    } else {
+        o.v[0] = p[0];
+    }
+    return o;
+}
+
 // The first Code instructions (Code >= n_code), unrolled so that every word
-// is a kernel-argument scalar.
-template <int Code, int W>
-__device__ inline void run(Regs<W>& r, const Program& P) {
+// is a kernel-argument scalar. `at`: the values' coordinates (matrix programs).
+template <int Code, bool Matrix, int W>
+__device__ inline void run(Regs<W>& r, const Program& P, const Place<W>& at) {
 #pragma unroll
     for (int k = 0; k < Code; ++k) {
         if (k >= P.n_code) continue;  // uniform: the rest of the loop is skipped
@@ -90,6 +155,17 @@ __device__ inline void run(Regs<W>& r, const Program& P) {
                   id = int(word >> 24);
         const Vals<W> a = get(r, ia), b = get(r, ib);
         Vals<W> v;
+        if constexpr (Matrix) {
+            if (op >= VC_MAP_AT_ROW) {  // VC_MAP_AT_ROW or VC_MAP_AT_COLUMN
+#pragma unroll
+                for (int j = 0; j < W; ++j) {
+                    const uint32_t axis = op == VC_MAP_AT_ROW ? at.in_group[j] : at.c[j];
+                    v.v[j] = int(a.v[j]) == int(axis) ? b.v[j] : 0.0f;
+                }
+                put(r, id, v);
+                continue;
+            }
+        }
         switch (op) {
             case VC_MAP_ADD:
 #pragma unroll
@@ -143,6 +219,35 @@ __device__ inline void load_inputs(Regs<W>& r, const Program& P, int64_t e) {
     for (int j = 0; j < NIn; ++j) put(r, j, v[j]);
 }
 
+// As load_inputs for a matrix program: element group e lies at `at`.
+template <int NIn, int W>
+__device__ inline void load_matrix_inputs(Regs<W>& r, const Program& P, int64_t e, const Place<W>& at) {
+    Vals<W> v[NIn];
+#pragma unroll
+    for (int j = 0; j < NIn; ++j) {
+        const float* in = P.in[j];
+        if (P.kind[j] == VC_MAP_FULL) {
+            v[j] = load_any<W>(in + e);
+        } else if (P.kind[j] == VC_MAP_PER_COLUMN) {
+            if (at.one_row) v[j] = load_any<W>(in + at.c[0]);
+            else
+#pragma unroll
+                for (int w = 0; w < W; ++w) v[j].v[w] = in[at.c[w]];
+        } else if (P.kind[j] == VC_MAP_PER_ROW) {
+            v[j].v[0] = in[at.r[0]];
+#pragma unroll
+            for (int w = 1; w < W; ++w) v[j].v[w] = at.one_row ? v[j].v[0] : in[at.r[w]];
+        } else {  // VC_MAP_PER_GROUP
+            if (at.one_row) v[j] = load_any<W>(in + int64_t(at.group[0]) * P.cols + at.c[0]);
+            else
+#pragma unroll
+                for (int w = 0; w < W; ++w) v[j].v[w] = in[int64_t(at.group[w]) * P.cols + at.c[w]];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NIn; ++j) put(r, j, v[j]);
+}
+
 template <int W>
 __device__ inline void store_outputs(const Regs<W>& r, const Program& P, int64_t e) {
 #pragma unroll
@@ -158,8 +263,76 @@ __global__ __launch_bounds__(kMapBlock) void map_flat_kernel(Program P, int64_t 
     const int64_t stride = int64_t(gridDim.x) * blockDim.x;
     for (int64_t g = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; g < groups; g += stride) {
         load_inputs<NIn, W>(r, P, g * W);
-        run<Code>(r, P);
+        run<Code, false>(r, P, Place<W>{});
         store_outputs(r, P, g * W);
+    }
+}
+
+// map_flat_kernel of a matrix program: full inputs and outputs are read and
+// written as there, whatever the columns; the other inputs by coordinates. The
+// last group of count % W values is a launch of its own from element `first`.
+template <int NIn, int W, int Code>
+__global__ __launch_bounds__(kMapBlock) void map_matrix_kernel(Program P, int64_t groups, int64_t first) {
+    Regs<W> r;
+    set_constants(r, P, NIn);
+    const int64_t stride = int64_t(gridDim.x) * blockDim.x;
+    for (int64_t g = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; g < groups; g += stride) {
+        const int64_t e = first + g * W;
+        const Place<W> at = place_of<W>(P, uint32_t(e));
+        load_matrix_inputs<NIn, W>(r, P, e, at);
+        run<Code, true>(r, P, at);
+        store_outputs(r, P, e);
+    }
+}
+
+// A matrix program with the row sums of P.sum_slot[s] for s < P.n_sum: Lanes
+// threads (a wavefront or the workgroup) take a row, W columns at a time; the
+// last group of a row whose length is no multiple of W is moved back to end
+// with the row (its first values are computed and written twice, and added
+// once). Sums in double: each lane in column order, then red::wave_sum's order,
+// then wave order.
+template <int NIn, int W, int Lanes, int Code>
+__global__ __launch_bounds__(kMapBlock) void map_rows_kernel(Program P, int64_t rows) {
+    constexpr int kWaves = Lanes / 64;
+    __shared__ double wave_part[kSums][4];
+    const int t = int(threadIdx.x) % Lanes, lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6;
+    const uint32_t cols = P.cols;
+    Regs<W> r;
+    set_constants(r, P, NIn);
+    const int64_t step = int64_t(gridDim.x) * (kMapBlock / Lanes);
+    for (int64_t row = int64_t(blockIdx.x) * (kMapBlock / Lanes) + int(threadIdx.x) / Lanes; row < rows; row += step) {
+        double acc[kSums] = {0.0, 0.0};
+        for (uint32_t c = uint32_t(t) * W; c < cols; c += Lanes * W) {
+            const uint32_t c1 = c + W <= cols ? c : cols - W;
+            const int64_t e = row * cols + c1;
+            const Place<W> at = place_at<W>(P, uint32_t(row), c1);
+            load_matrix_inputs<NIn, W>(r, P, e, at);
+            run<Code, true>(r, P, at);
+#pragma unroll
+            for (int j = 0; j < kOutputs; ++j)
+                if (j < P.n_out) store_any<W>(P.out[j] + e, get(r, P.out_slot[j]));
+#pragma unroll
+            for (int s = 0; s < kSums; ++s)
+                if (s < P.n_sum) {
+                    const Vals<W> v = get(r, P.sum_slot[s]);
+#pragma unroll
+                    for (int j = 0; j < W; ++j) acc[s] += c1 + uint32_t(j) >= c ? double(v.v[j]) : 0.0;
+                }
+        }
+#pragma unroll
+        for (int s = 0; s < kSums; ++s) acc[s] = red::wave_sum(acc[s]);
+        if constexpr (kWaves > 1) {
+            if (lane == 0)
+                for (int s = 0; s < kSums; ++s) wave_part[s][wave] = acc[s];
+            __syncthreads();
+            for (int s = 0; s < kSums; ++s) {
+                acc[s] = wave_part[s][0];
+                for (int k = 1; k < kWaves; ++k) acc[s] += wave_part[s][k];
+            }
+            __syncthreads();
+        }
+        if (t == 0)
+            for (int s = 0; s < P.n_sum; ++s) P.sum[s][row] = float(acc[s]);
     }
 }
 
@@ -171,7 +344,7 @@ __global__ __launch_bounds__(kMapBlock) void map_flat_kernel(Program P, int64_t 
 // in row order; the four waves' sums are added in wave order and written as
 // partial row y: part[s][y][col]. column_partials_kernel then adds the gy
 // partial rows in a fixed order.
-template <int NIn, int W, int Code, int NSum>
+template <int NIn, int W, int Code, int NSum, bool Matrix>
 __global__ __launch_bounds__(kMapBlock) void map_columns_kernel(Program P, int64_t rows, int64_t cols,
                                                                 double* __restrict__ part) {
     __shared__ double wave_part[NSum][4][64 * W];
@@ -188,8 +361,14 @@ __global__ __launch_bounds__(kMapBlock) void map_columns_kernel(Program P, int64
     if (col < cols) {
         for (int64_t row = int64_t(blockIdx.y) * 4 + w; row < rows; row += step) {
             const int64_t e = row * cols + col;
-            load_inputs<NIn, W>(r, P, e);
-            run<Code>(r, P);
+            if constexpr (Matrix) {
+                const Place<W> at = place_at<W>(P, uint32_t(row), uint32_t(col));
+                load_matrix_inputs<NIn, W>(r, P, e, at);
+                run<Code, true>(r, P, at);
+            } else {
+                load_inputs<NIn, W>(r, P, e);
+                run<Code, false>(r, P, Place<W>{});
+            }
             store_outputs(r, P, e);
 #pragma unroll
             for (int s = 0; s < NSum; ++s) {
@@ -265,12 +444,50 @@ template <int NIn>
 void launch_columns(Device& d, const Program& P, int64_t rows, int64_t cols, bool vec, double* part) {
     const ColumnGrid g = column_grid(rows, cols, vec ? 4 : 1);
     const dim3 grid(unsigned(g.col_blocks), unsigned(g.gy));
-    if (vec && P.n_code <= kShortCode && P.n_sum == 1)  // the common case: a short program, one sum
-        launch(map_columns_kernel<NIn, 4, kShortCode, 1>, grid, dim3(kMapBlock), 0, d.stream, P, rows, cols, part);
-    else if (vec)
-        launch(map_columns_kernel<NIn, 4, kCode, kSums>, grid, dim3(kMapBlock), 0, d.stream, P, rows, cols, part);
-    else
-        launch(map_columns_kernel<NIn, 1, kCode, kSums>, grid, dim3(kMapBlock), 0, d.stream, P, rows, cols, part);
+    if (P.cols != 0) {  // a matrix program
+        if (vec && P.n_code <= kShortCode && P.n_sum == 1)
+            launch(map_columns_kernel<NIn, 4, kShortCode, 1, true>, grid, dim3(kMapBlock), 0, d.stream, P, rows, cols, part);
+        else if (vec)
+            launch(map_columns_kernel<NIn, 4, kCode, kSums, true>, grid, dim3(kMapBlock), 0, d.stream, P, rows, cols, part);
+        else
+            launch(map_columns_kernel<NIn, 1, kCode, kSums, true>, grid, dim3(kMapBlock), 0, d.stream, P, rows, cols, part);
+    } else if (vec && P.n_code <= kShortCode && P.n_sum == 1) {  // the common case: a short program, one sum
+        launch(map_columns_kernel<NIn, 4, kShortCode, 1, false>, grid, dim3(kMapBlock), 0, d.stream, P, rows, cols, part);
+    } else if (vec) {
+        launch(map_columns_kernel<NIn, 4, kCode, kSums, false>, grid, dim3(kMapBlock), 0, d.stream, P, rows, cols, part);
+    } else {
+        launch(map_columns_kernel<NIn, 1, kCode, kSums, false>, grid, dim3(kMapBlock), 0, d.stream, P, rows, cols, part);
+    }
+}
+
+// A matrix program without sums.
+template <int NIn>
+void launch_matrix(Device& d, const Program& P, int64_t count, bool vec) {
+    const int64_t groups = vec ? count / 4 : 0;
+    if (groups > 0 && P.n_code <= kShortCode)
+        launch(map_matrix_kernel<NIn, 4, kShortCode>, dim3(grid_1d(size_t(groups), kMapBlock, kFlatBlocks)), dim3(kMapBlock),
+               0, d.stream, P, groups, int64_t(0));
+    else if (groups > 0)
+        launch(map_matrix_kernel<NIn, 4, kCode>, dim3(grid_1d(size_t(groups), kMapBlock, kFlatBlocks)), dim3(kMapBlock), 0,
+               d.stream, P, groups, int64_t(0));
+    if (groups * 4 < count) {
+        const int64_t rest = count - groups * 4;
+        launch(map_matrix_kernel<NIn, 1, kCode>, dim3(grid_1d(size_t(rest), kMapBlock, kFlatBlocks)), dim3(kMapBlock), 0,
+               d.stream, P, rest, groups * 4);
+    }
+}
+
+// A matrix program with row sums: a wavefront per row, or a workgroup for few long rows.
+template <int NIn>
+void launch_rows(Device& d, const Program& P, int64_t rows) {
+    const bool wide = rows < 2048 && P.cols > 1024;
+    const unsigned grid = unsigned(std::min<int64_t>(wide ? rows : (rows + 3) / 4, kFlatBlocks));
+    const bool brief = P.n_code <= kShortCode;
+    if (P.cols < 4) launch(map_rows_kernel<NIn, 1, 64, kCode>, dim3(grid), dim3(kMapBlock), 0, d.stream, P, rows);
+    else if (wide && brief) launch(map_rows_kernel<NIn, 4, 256, kShortCode>, dim3(grid), dim3(kMapBlock), 0, d.stream, P, rows);
+    else if (wide) launch(map_rows_kernel<NIn, 4, 256, kCode>, dim3(grid), dim3(kMapBlock), 0, d.stream, P, rows);
+    else if (brief) launch(map_rows_kernel<NIn, 4, 64, kShortCode>, dim3(grid), dim3(kMapBlock), 0, d.stream, P, rows);
+    else launch(map_rows_kernel<NIn, 4, 64, kCode>, dim3(grid), dim3(kMapBlock), 0, d.stream, P, rows);
 }
 
 }  // namespace fmap

@@ -11,6 +11,8 @@ namespace fmap {
 
 template void launch_flat<VC_MAP_NIN>(Device&, const Program&, int64_t, bool);
 template void launch_columns<VC_MAP_NIN>(Device&, const Program&, int64_t, int64_t, bool, double*);
+template void launch_matrix<VC_MAP_NIN>(Device&, const Program&, int64_t, bool);
+template void launch_rows<VC_MAP_NIN>(Device&, const Program&, int64_t);
 
 }  // namespace fmap
 }  // namespace vchip
