@@ -24,7 +24,12 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 constexpr unsigned kBlock = 256;
 
 __device__ inline f4 ld4(const float* p) { return *reinterpret_cast<const f4*>(p); }
-__device__ inline void st4(float* p, f4 v) { __builtin_nontemporal_store(v, reinterpret_cast<f4*>(p)); }
+// Stream: non-temporal, past the caches (see stream_stores).
+template <bool Stream>
+__device__ inline void st4(float* p, f4 v) {
+    if constexpr (Stream) __builtin_nontemporal_store(v, reinterpret_cast<f4*>(p));
+    else *reinterpret_cast<f4*>(p) = v;
+}
 
 // ---- operation functors ------------------------------------------------------
 
@@ -71,38 +76,38 @@ template <class F>
 __device__ inline f4 apply4(F f, f4 a, f4 b) { return f4{f(a.x, b.x), f(a.y, b.y), f(a.z, b.z), f(a.w, b.w)}; }
 
 // y[i] = f(x[i]). n4 vectors, then `tail` scalars after them.
-template <class F>
+template <bool Stream, class F>
 __device__ inline void map1_body(const float* __restrict__ x, float* __restrict__ y, size_t n4, size_t tail, F f) {
     const size_t stride = size_t(gridDim.x) * blockDim.x;
     size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     for (; i + 3 * stride < n4; i += 4 * stride) {
         f4 v0 = ld4(x + 4 * i), v1 = ld4(x + 4 * (i + stride)), v2 = ld4(x + 4 * (i + 2 * stride)),
            v3 = ld4(x + 4 * (i + 3 * stride));
-        st4(y + 4 * i, apply4(f, v0));
-        st4(y + 4 * (i + stride), apply4(f, v1));
-        st4(y + 4 * (i + 2 * stride), apply4(f, v2));
-        st4(y + 4 * (i + 3 * stride), apply4(f, v3));
+        st4<Stream>(y + 4 * i, apply4(f, v0));
+        st4<Stream>(y + 4 * (i + stride), apply4(f, v1));
+        st4<Stream>(y + 4 * (i + 2 * stride), apply4(f, v2));
+        st4<Stream>(y + 4 * (i + 3 * stride), apply4(f, v3));
     }
-    for (; i < n4; i += stride) st4(y + 4 * i, apply4(f, ld4(x + 4 * i)));
+    for (; i < n4; i += stride) st4<Stream>(y + 4 * i, apply4(f, ld4(x + 4 * i)));
     const size_t t = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (t < tail) y[4 * n4 + t] = f(x[4 * n4 + t]);
 }
 
-template <class F>
+template <bool Stream, class F>
 __global__ __launch_bounds__(kBlock) void map1_kernel(const float* __restrict__ x, float* __restrict__ y, size_t n4,
                                                       size_t tail, F f) {
-    map1_body(x, y, n4, tail, f);
+    map1_body<Stream>(x, y, n4, tail, f);
 }
 
 // y[i] = x[i] op s[0] (or s[0] op x[i]) with s a one-element device operand.
-template <class Op, bool ScalarFirst>
+template <class Op, bool ScalarFirst, bool Stream>
 __global__ __launch_bounds__(kBlock) void scalar_operand_kernel(const float* __restrict__ x, const float* __restrict__ s,
                                                                 float* __restrict__ y, size_t n4, size_t tail) {
-    map1_body(x, y, n4, tail, ScalarOp<Op, ScalarFirst>{s[0]});
+    map1_body<Stream>(x, y, n4, tail, ScalarOp<Op, ScalarFirst>{s[0]});
 }
 
 // y[i] = f(a[i], b[i]).
-template <class F>
+template <bool Stream, class F>
 __global__ __launch_bounds__(kBlock) void map2_kernel(const float* __restrict__ a, const float* __restrict__ b,
                                                       float* __restrict__ y, size_t n4, size_t tail, F f) {
     const size_t stride = size_t(gridDim.x) * blockDim.x;
@@ -112,12 +117,12 @@ __global__ __launch_bounds__(kBlock) void map2_kernel(const float* __restrict__ 
            a3 = ld4(a + 4 * (i + 3 * stride));
         f4 b0 = ld4(b + 4 * i), b1 = ld4(b + 4 * (i + stride)), b2 = ld4(b + 4 * (i + 2 * stride)),
            b3 = ld4(b + 4 * (i + 3 * stride));
-        st4(y + 4 * i, apply4(f, a0, b0));
-        st4(y + 4 * (i + stride), apply4(f, a1, b1));
-        st4(y + 4 * (i + 2 * stride), apply4(f, a2, b2));
-        st4(y + 4 * (i + 3 * stride), apply4(f, a3, b3));
+        st4<Stream>(y + 4 * i, apply4(f, a0, b0));
+        st4<Stream>(y + 4 * (i + stride), apply4(f, a1, b1));
+        st4<Stream>(y + 4 * (i + 2 * stride), apply4(f, a2, b2));
+        st4<Stream>(y + 4 * (i + 3 * stride), apply4(f, a3, b3));
     }
-    for (; i < n4; i += stride) st4(y + 4 * i, apply4(f, ld4(a + 4 * i), ld4(b + 4 * i)));
+    for (; i < n4; i += stride) st4<Stream>(y + 4 * i, apply4(f, ld4(a + 4 * i), ld4(b + 4 * i)));
     const size_t t = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (t < tail) y[4 * n4 + t] = f(a[4 * n4 + t], b[4 * n4 + t]);
 }
@@ -184,7 +189,7 @@ __global__ __launch_bounds__(kBlock) void axpy_list_kernel(AxpyList L) {
         const float* t = L.t[k] + e;
         const float* src = L.s[k] + e;
         if (e + 4 <= L.count[k]) {
-            st4(o, apply4(f, ld4(t), ld4(src)));
+            st4<true>(o, apply4(f, ld4(t), ld4(src)));
         } else {
             for (int64_t i = 0; e + i < L.count[k]; ++i) o[i] = f(t[i], src[i]);
         }
@@ -213,7 +218,7 @@ __global__ __launch_bounds__(kBlock) void fill_kernel(float* __restrict__ y, siz
 
 // Rank-2 broadcast over [rows, cols]: a at (r*as0 + c*as1), b likewise, with
 // as1, bs1 in {0, 1}. One workgroup row-chunk per block, columns across lanes.
-template <class Op, bool Vec>
+template <class Op, bool Vec, bool Stream>
 __global__ __launch_bounds__(kBlock) void bcast2_kernel(const float* __restrict__ a, const float* __restrict__ b,
                                                         float* __restrict__ y, int64_t rows, int64_t cols, int64_t as0,
                                                         int64_t as1, int64_t bs0, int64_t bs1) {
@@ -226,7 +231,7 @@ __global__ __launch_bounds__(kBlock) void bcast2_kernel(const float* __restrict_
             for (int64_t c = int64_t(threadIdx.x) * 4; c < cols; c += int64_t(blockDim.x) * 4) {
                 const f4 av = as1 ? ld4(ar + c) : f4{ar[0], ar[0], ar[0], ar[0]};
                 const f4 bv = bs1 ? ld4(br + c) : f4{br[0], br[0], br[0], br[0]};
-                st4(yr + c, f4{op(av.x, bv.x), op(av.y, bv.y), op(av.z, bv.z), op(av.w, bv.w)});
+                st4<Stream>(yr + c, f4{op(av.x, bv.x), op(av.y, bv.y), op(av.z, bv.z), op(av.w, bv.w)});
             }
         } else {
             for (int64_t c = threadIdx.x; c < cols; c += blockDim.x) yr[c] = op(ar[c * as1], br[c * bs1]);
@@ -278,10 +283,19 @@ __global__ __launch_bounds__(kBlock) void div_backward_kernel(const float* __res
 
 // ---- host-side launch helpers ---------------------------------------------------
 
-unsigned stream_grid(size_t items) {
+unsigned stream_grid(size_t items, unsigned per_cu = 4) {
     Device& d = device();
-    return grid_1d(items, kBlock, static_cast<unsigned>(d.cu_count > 0 ? d.cu_count * 4 : 1024));
+    return grid_1d(items, kBlock, static_cast<unsigned>(d.cu_count > 0 ? d.cu_count : 256) * per_cu);
 }
+
+// Whether a pass over `bytes` stores past the caches. While the operands and
+// the result fit the 256 MB memory-side cache the next pass finds the result
+// there, and 16 workgroups per CU instead of 4 keep it busy: a chain of ReLUs
+// over 64 MiB tensors takes 21.9 us a pass, against 27.4 with streamed stores
+// and 4 workgroups (23.9 and 29.2 with one of the two changed). Over 512 MiB
+// tensors the streamed stores are faster, 245 against 259 us.
+bool stream_stores(double bytes) { return bytes > 256e6; }
+unsigned map_grid(size_t vectors, bool stream) { return stream_grid(vectors ? vectors : 1, stream ? 4 : 16); }
 
 template <class F>
 void launch_map1(const char* label, const float* x, float* y, size_t n, F f, double bytes_per_elem) {
@@ -291,7 +305,10 @@ void launch_map1(const char* label, const float* x, float* y, size_t n, F f, dou
     Profiled p(label, 0.0, bytes_per_elem * double(n));
     if (aligned16(x) && aligned16(y)) {
         const size_t n4 = n / 4, tail = n % 4;
-        launch(map1_kernel<F>, dim3(stream_grid(n4 ? n4 : 1)), dim3(kBlock), 0, d.stream, x, y, n4, tail, f);
+        const bool stream = stream_stores(bytes_per_elem * double(n));
+        const dim3 grid(map_grid(n4, stream));
+        if (stream) launch(map1_kernel<true, F>, grid, dim3(kBlock), 0, d.stream, x, y, n4, tail, f);
+        else launch(map1_kernel<false, F>, grid, dim3(kBlock), 0, d.stream, x, y, n4, tail, f);
     } else {
         launch(map1_scalar_kernel<F>, dim3(stream_grid(n)), dim3(kBlock), 0, d.stream, x, y, n, f);
     }
@@ -307,7 +324,10 @@ void launch_map2(const char* label, const float* a, const float* b, float* y, si
     Profiled p(label, 0.0, bytes_per_elem * double(n));
     if (aligned16(a) && aligned16(b) && aligned16(y)) {
         const size_t n4 = n / 4, tail = n % 4;
-        launch(map2_kernel<F>, dim3(stream_grid(n4 ? n4 : 1)), dim3(kBlock), 0, d.stream, a, b, y, n4, tail, f);
+        const bool stream = stream_stores(bytes_per_elem * double(n));
+        const dim3 grid(map_grid(n4, stream));
+        if (stream) launch(map2_kernel<true, F>, grid, dim3(kBlock), 0, d.stream, a, b, y, n4, tail, f);
+        else launch(map2_kernel<false, F>, grid, dim3(kBlock), 0, d.stream, a, b, y, n4, tail, f);
     } else {
         launch(map2_scalar_kernel<F>, dim3(stream_grid(n)), dim3(kBlock), 0, d.stream, a, b, y, n, f);
     }
@@ -331,12 +351,16 @@ void launch_binary(const float* a, const float* b, float* y, size_t n, const Bca
         if (aligned16(x) && aligned16(y)) {
             Profiled p(label, 0.0, 8.0 * double(n));
             const size_t n4 = n / 4, tail = n % 4;
-            if (scalar_first)
-                launch((scalar_operand_kernel<Op, true>), dim3(stream_grid(n4 ? n4 : 1)), dim3(kBlock), 0,
-                                   d.stream, x, s, y, n4, tail);
+            const bool stream = stream_stores(8.0 * double(n));
+            const dim3 grid(map_grid(n4, stream));
+            if (scalar_first && stream)
+                launch((scalar_operand_kernel<Op, true, true>), grid, dim3(kBlock), 0, d.stream, x, s, y, n4, tail);
+            else if (scalar_first)
+                launch((scalar_operand_kernel<Op, true, false>), grid, dim3(kBlock), 0, d.stream, x, s, y, n4, tail);
+            else if (stream)
+                launch((scalar_operand_kernel<Op, false, true>), grid, dim3(kBlock), 0, d.stream, x, s, y, n4, tail);
             else
-                launch((scalar_operand_kernel<Op, false>), dim3(stream_grid(n4 ? n4 : 1)), dim3(kBlock), 0,
-                                   d.stream, x, s, y, n4, tail);
+                launch((scalar_operand_kernel<Op, false, false>), grid, dim3(kBlock), 0, d.stream, x, s, y, n4, tail);
             after_launch(label);
             p.done();
             return;
@@ -348,12 +372,15 @@ void launch_binary(const float* a, const float* b, float* y, size_t n, const Bca
                          (m.b_stride[1] == 0 || (aligned16(b) && m.b_stride[0] % 4 == 0));
         const unsigned grid = static_cast<unsigned>(std::min<int64_t>(rows, int64_t(d.cu_count) * 16));
         Profiled p(label, 0.0, 8.0 * double(n));
-        if (vec)
-            launch((bcast2_kernel<Op, true>), dim3(grid), dim3(kBlock), 0, d.stream, a, b, y, rows, cols,
-                               m.a_stride[0], m.a_stride[1], m.b_stride[0], m.b_stride[1]);
+        if (vec && stream_stores(8.0 * double(n)))
+            launch((bcast2_kernel<Op, true, true>), dim3(grid), dim3(kBlock), 0, d.stream, a, b, y, rows, cols,
+                   m.a_stride[0], m.a_stride[1], m.b_stride[0], m.b_stride[1]);
+        else if (vec)
+            launch((bcast2_kernel<Op, true, false>), dim3(grid), dim3(kBlock), 0, d.stream, a, b, y, rows, cols,
+                   m.a_stride[0], m.a_stride[1], m.b_stride[0], m.b_stride[1]);
         else
-            launch((bcast2_kernel<Op, false>), dim3(grid), dim3(kBlock), 0, d.stream, a, b, y, rows, cols,
-                               m.a_stride[0], m.a_stride[1], m.b_stride[0], m.b_stride[1]);
+            launch((bcast2_kernel<Op, false, false>), dim3(grid), dim3(kBlock), 0, d.stream, a, b, y, rows, cols,
+                   m.a_stride[0], m.a_stride[1], m.b_stride[0], m.b_stride[1]);
         after_launch(label);
         p.done();
         return;
