@@ -370,6 +370,11 @@ int vc_hip_reduce_sum(const float* in, size_t count, float* out);
  * argmax return the first maximum (argmax as a float index), and a NaN first
  * element wins, as in src/cpu/cpu_backend.cpp:443-457. */
 int vc_hip_reduce_axis(const float* in, float* out, size_t outer, size_t length, size_t inner, int op);
+/* vc_hip_reduce_axis with VC_REDUCE_MAX and with VC_REDUCE_ARGMAX in one pass
+ * over the input: the same values. What a maximum that needs a gradient asks
+ * for (src/ops.cpp:318-342 reduces twice). */
+int vc_hip_reduce_axis_max_argmax(const float* in, float* max_out, float* argmax_out, size_t outer, size_t length,
+                                  size_t inner);
 /* vc_hip_reduce_axis without any device allocation: the same kernels, the
  * same results bit for bit, with the partial results (column sums, max and
  * argmax splits) in a static 2 MiB device array (one per GPU, held until the

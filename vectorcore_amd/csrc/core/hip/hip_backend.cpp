@@ -1056,6 +1056,20 @@ std::shared_ptr<Storage> HipBackend::reduce_axis(const Storage& input, std::size
     return out;
 }
 
+std::pair<std::shared_ptr<Storage>, std::shared_ptr<Storage>> HipBackend::max_argmax(const Storage& input,
+                                                                                     std::size_t offset,
+                                                                                     std::size_t outer,
+                                                                                     std::size_t length,
+                                                                                     std::size_t inner) {
+    require(*this);
+    if (length == 0) throw std::invalid_argument("max/argmax over an empty axis is undefined");
+    auto best = fresh(outer * inner), indices = fresh(outer * inner);
+    if (outer * inner != 0)
+        check(vc_hip_reduce_axis_max_argmax(dptr(input, offset), best->ptr(), indices->ptr(), outer, length, inner),
+              "HIP axis reduction failed");
+    return {best, indices};
+}
+
 std::shared_ptr<Storage> HipBackend::scatter_axis(const Storage& values, std::size_t values_offset,
                                                   const Storage& indices, std::size_t indices_offset,
                                                   std::size_t outer, std::size_t length, std::size_t inner) {

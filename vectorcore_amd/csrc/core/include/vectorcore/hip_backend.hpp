@@ -143,6 +143,12 @@ public:
     [[nodiscard]] bool fuse_elementwise() const;
 
     // --- fused kernels used by the hip arm of the backward rules ---
+    // Maximum and argmax along the middle axis from one pass.
+    [[nodiscard]] std::pair<std::shared_ptr<Storage>, std::shared_ptr<Storage>> max_argmax(const Storage& input,
+                                                                                           std::size_t offset,
+                                                                                           std::size_t outer,
+                                                                                           std::size_t length,
+                                                                                           std::size_t inner);
     // Softmax or log-softmax along the middle axis, with the rows' maxima and
     // sums for softmax_backward.
     [[nodiscard]] std::pair<std::shared_ptr<Storage>, std::shared_ptr<Storage>> softmax_forward(

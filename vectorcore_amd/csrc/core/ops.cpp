@@ -17,6 +17,7 @@
 #include <optional>
 #include <stdexcept>
 #include <string>
+#include <tuple>
 #include <utility>
 #include <vector>
 
@@ -467,10 +468,17 @@ Tensor mean(const Tensor& v) {
 Tensor max(const Tensor& v, std::int64_t axis, bool keepdim) {
     const AxisSplit s = split_axis(v.shape(), axis);
     const Shape out_shape = keepdim ? s.kept : s.removed;
-    auto out = detail::make_tensor(reduce_storage(v, s, cpu::ReduceOp::Max), out_shape, false);
-    if (!grad_enabled() || !v.requires_grad()) return out;
+    const bool gradient = grad_enabled() && v.requires_grad();
+    std::shared_ptr<Storage> best, where;
+    if (gradient && v.device() == Device::hip())
+        std::tie(best, where) = hip().max_argmax(st(v), off(v), s.outer, s.length, s.inner);
+    else
+        best = reduce_storage(v, s, cpu::ReduceOp::Max);
+    auto out = detail::make_tensor(std::move(best), out_shape, false);
+    if (!gradient) return out;
     // The gradient goes to the first maximal element along the axis.
-    const Tensor indices = detail::make_tensor(reduce_storage(v, s, cpu::ReduceOp::Argmax), out_shape, false);
+    if (!where) where = reduce_storage(v, s, cpu::ReduceOp::Argmax);
+    const Tensor indices = detail::make_tensor(std::move(where), out_shape, false);
     const Shape in_shape = v.shape();
     detail::attach_grad_fn(out, {v}, [indices, s, in_shape](const Tensor& g) {
         std::shared_ptr<Storage> r;

@@ -237,6 +237,8 @@ int vc_hip_map_broadcast(const vc_hip_map_program* program, const vc_hip_map_mat
         Program P = program_of(p);
         P.cols = uint32_t(p.cols);
         P.len = uint32_t(m.axis_length);
+        set_magic(P.cols, P.cols_magic, P.cols_shift);
+        set_magic(P.len, P.len_magic, P.len_shift);
         bool vec = true;
         double bytes = 4.0 * double(p.rows * p.cols) * double(p.n_outputs);
         for (size_t j = 0; j < p.n_inputs; ++j) {

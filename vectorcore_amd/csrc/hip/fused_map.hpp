@@ -38,7 +38,21 @@ struct Program {
     // (VC_MAP_FULL ...), and the matrix.
     uint8_t kind[kInputs];
     uint32_t cols, len;
+    uint32_t cols_magic, cols_shift, len_magic, len_shift;  // for divide()
 };
+
+// n / d for n < 2^31 as a multiplication: magic = floor(2^(31 + l) / d) + 1 and
+// shift = 31 + l with l = ceil(log2 d) (the error of magic / 2^shift is below
+// 2^-shift <= 2^-31 / d, less than what separates n / d from the next whole number).
+inline void set_magic(uint32_t d, uint32_t& magic, uint32_t& shift) {
+    uint32_t l = 0;
+    while ((uint64_t(1) << l) < d) ++l;
+    magic = uint32_t((uint64_t(1) << (31 + l)) / d + 1);
+    shift = 31 + l;
+}
+__device__ inline uint32_t divide(uint32_t n, uint32_t magic, uint32_t shift) {
+    return uint32_t((uint64_t(n) * magic) >> shift);
+}
 
 // The matrix coordinates of a thread's W values: row (group of rows and row in
 // the group) and column of each, and whether they lie in one row.
@@ -50,7 +64,7 @@ struct Place {
     __device__ void set(const Program& P, uint32_t r0, uint32_t c0) {
         one_row = c0 + W <= P.cols;
         uint32_t g0 = r0, a0 = 0;
-        if (P.len != 1) g0 = r0 / P.len, a0 = r0 - g0 * P.len;
+        if (P.len != 1) g0 = divide(r0, P.len_magic, P.len_shift), a0 = r0 - g0 * P.len;
 #pragma unroll
         for (int j = 0; j < W; ++j) {
             r[j] = r0, group[j] = g0, in_group[j] = a0, c[j] = c0;
@@ -64,7 +78,7 @@ struct Place {
 template <int W>
 __device__ inline Place<W> place_of(const Program& P, uint32_t e) {  // elements e .. e + W - 1
     Place<W> at;
-    const uint32_t r = e / P.cols;
+    const uint32_t r = divide(e, P.cols_magic, P.cols_shift);
     at.set(P, r, e - r * P.cols);
     return at;
 }

@@ -51,12 +51,12 @@ __device__ inline Best combine(Best a, Best b) {
 }
 
 // ---- rows: inner == 1, one wavefront per row -----------------------------------
-// Op: 0 sum, 1 max, 2 argmax. With NV > 0 (rows of at most 256 NV elements, a
+// Op: 0 sum, 1 max, 2 argmax, 3 max and (in out2) argmax. With NV > 0 (rows of at most 256 NV elements, a
 // multiple of 4) each lane loads its NV float4 at once before reducing;
 // otherwise it streams. Both visit a lane's elements in the same order.
 template <int Op, bool Vec, int NV>
-__global__ __launch_bounds__(kBlock) void rows_kernel(const float* __restrict__ x, float* __restrict__ out, int64_t rows,
-                                                      int64_t len) {
+__global__ __launch_bounds__(kBlock) void rows_kernel(const float* __restrict__ x, float* __restrict__ out,
+                                                      float* __restrict__ out2, int64_t rows, int64_t len) {
     const int lane = threadIdx.x % kWave;
     const int64_t waves_per_grid = int64_t(gridDim.x) * (blockDim.x / kWave);
     for (int64_t r = int64_t(blockIdx.x) * (blockDim.x / kWave) + threadIdx.x / kWave; r < rows; r += waves_per_grid) {
@@ -123,7 +123,8 @@ __global__ __launch_bounds__(kBlock) void rows_kernel(const float* __restrict__ 
                 const float first = NV > 0 ? v[0].x : row[0];
                 if (first != first) b = Best{first, 0};
                 if (b.i == kNone) b.i = 0;
-                out[r] = Op == 1 ? b.v : float(b.i);
+                out[r] = Op != 2 ? b.v : float(b.i);
+                if (Op == 3) out2[r] = float(b.i);
             }
         }
     }
@@ -133,8 +134,8 @@ __global__ __launch_bounds__(kBlock) void rows_kernel(const float* __restrict__ 
 // Walks the axis in order exactly like the reference loop; used when there
 // are enough outputs to fill the device.
 template <int Op>
-__global__ __launch_bounds__(kBlock) void cols_kernel(const float* __restrict__ x, float* __restrict__ out, int64_t outer,
-                                                      int64_t len, int64_t inner) {
+__global__ __launch_bounds__(kBlock) void cols_kernel(const float* __restrict__ x, float* __restrict__ out,
+                                                      float* __restrict__ out2, int64_t outer, int64_t len, int64_t inner) {
     const int64_t total = outer * inner;
     const int64_t stride = int64_t(gridDim.x) * blockDim.x;
     for (int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; t < total; t += stride) {
@@ -154,8 +155,68 @@ __global__ __launch_bounds__(kBlock) void cols_kernel(const float* __restrict__ 
                     idx = a;
                 }
             }
-            out[t] = Op == 1 ? best : float(idx);
+            out[t] = Op != 2 ? best : float(idx);
+            if (Op == 3) out2[t] = float(idx);
         }
+    }
+}
+
+// ---- columns, max and argmax: a workgroup takes 16 W adjacent columns of one outer index ------
+// Row lane r of RowLanes walks rows r, r + RowLanes, ... in order with eight
+// rows in flight (W = 4: 16-byte loads on any 4-byte boundary); the row lanes'
+// best are then combined in lane order, ties to the smaller index. One launch
+// and one read of x. Bound by HBM: 64 x 197 x 768 along the middle axis 20.1
+// us with one thread per column and range and a combining launch, now 10.
+template <int Op, int W, int RowLanes>
+__global__ __launch_bounds__(16 * RowLanes) void cols_best_kernel(const float* __restrict__ x, float* __restrict__ out,
+                                                                  float* __restrict__ out2, int64_t len, int64_t inner,
+                                                                  int64_t chunks) {
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int kFlight = 8;
+    __shared__ float best_v[RowLanes][16 * W];
+    __shared__ int best_i[RowLanes][16 * W];
+    const int c = threadIdx.x % 16, rl = threadIdx.x / 16;
+    const int64_t o = blockIdx.x / chunks, first_col = (blockIdx.x % chunks) * 16 * W, col = first_col + c * W;
+    const float* const base = x + o * len * inner + col;
+    Best b[W];
+#pragma unroll
+    for (int w = 0; w < W; ++w) b[w] = red::no_best();
+    for (int64_t a0 = rl; a0 < len; a0 += kFlight * RowLanes) {
+        float v[kFlight][W];
+#pragma unroll
+        for (int u = 0; u < kFlight; ++u) {
+            const float* const p = base + (a0 + u * RowLanes) * inner;
+            const bool row_ok = a0 + u * RowLanes < len;
+            if (W == 4 && row_ok && col + 3 < inner) {
+                const f4 q = *reinterpret_cast<const f4u*>(p);
+#pragma unroll
+                for (int w = 0; w < W; ++w) v[u][w] = q[w];
+            } else {
+#pragma unroll
+                for (int w = 0; w < W; ++w) v[u][w] = row_ok && col + w < inner ? p[w] : -__builtin_huge_valf();
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kFlight; ++u)
+#pragma unroll
+            for (int w = 0; w < W; ++w) red::consider_ordered(b[w], v[u][w], int(a0 + u * RowLanes));
+    }
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+        best_v[rl][c * W + w] = b[w].v;
+        best_i[rl][c * W + w] = b[w].i;
+    }
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < 16 * W && first_col + t < inner) {
+        Best r{best_v[0][t], best_i[0][t]};
+        for (int k = 1; k < RowLanes; ++k) r = combine(r, Best{best_v[k][t], best_i[k][t]});
+        const float first = x[o * len * inner + first_col + t];
+        if (first != first) r = Best{first, 0};
+        if (r.i == kNone) r.i = 0;
+        const int64_t at = o * inner + first_col + t;
+        out[at] = Op != 2 ? r.v : float(r.i);
+        if (Op == 3) out2[at] = float(r.i);
     }
 }
 
@@ -602,6 +663,7 @@ class PartialMemory {
 public:
     virtual ~PartialMemory() = default;
     virtual void* take(size_t bytes) = 0;
+    virtual void require(size_t) const {}  // fails where take would
 };
 
 class PoolPartials final : public PartialMemory {
@@ -615,8 +677,33 @@ private:
     std::vector<std::unique_ptr<Scratch>> held_;
 };
 
+// Whether a max/argmax over columns takes cols_best_kernel: an axis worth its
+// 16 row lanes, and enough workgroups for the chip or an axis that a few read
+// quickly (longer ones are split over workgroups).
+int64_t best_chunks(int64_t inner) { return (inner + (inner >= 64 ? 63 : 15)) / (inner >= 64 ? 64 : 16); }
+bool best_in_one(int64_t outer, int64_t len, int64_t inner) {
+    const int64_t blocks = outer * best_chunks(inner);
+    return len >= 16 && blocks <= std::numeric_limits<int>::max() && (blocks >= 128 || len <= 1024);
+}
+
+template <int Op>
+void launch_cols_best(Device& d, const float* in, float* out, float* out2, int64_t outer, int64_t len, int64_t inner) {
+    const int64_t chunks = best_chunks(inner);
+    const dim3 grid{unsigned(outer * chunks)};
+    const bool few = outer * chunks < 2 * int64_t(d.cu_count) && len > 64;  // more row lanes for fewer workgroups
+    if (inner >= 64 && few)
+        launch(cols_best_kernel<Op, 4, 32>, grid, dim3(512), 0, d.stream, in, out, out2, len, inner, chunks);
+    else if (inner >= 64)
+        launch(cols_best_kernel<Op, 4, 16>, grid, dim3(256), 0, d.stream, in, out, out2, len, inner, chunks);
+    else if (few)
+        launch(cols_best_kernel<Op, 1, 64>, grid, dim3(1024), 0, d.stream, in, out, out2, len, inner, chunks);
+    else
+        launch(cols_best_kernel<Op, 1, 16>, grid, dim3(256), 0, d.stream, in, out, out2, len, inner, chunks);
+}
+
+// out2: the argmax beside a max (op VC_REDUCE_MAX), or null.
 void reduce_axis(const float* in, float* out, int64_t outer, int64_t len, int64_t inner, int op,
-                 PartialMemory& memory) {
+                 PartialMemory& memory, float* out2 = nullptr) {
     Device& d = require_device();
     if (op < VC_REDUCE_SUM || op > VC_REDUCE_ARGMAX) fail(VC_HIP_ERR_INVALID_ARGUMENT, "unknown reduction");
     if (len == 0 && op != VC_REDUCE_SUM) fail(VC_HIP_ERR_INVALID_ARGUMENT, "max/argmax over an empty axis is undefined");
@@ -637,7 +724,7 @@ void reduce_axis(const float* in, float* out, int64_t outer, int64_t len, int64_
         const unsigned grid = unsigned(std::min<int64_t>((outer + 3) / 4, int64_t(d.cu_count) * 64));
         const int64_t nv = vec ? (len + kWave * 4 - 1) / (kWave * 4) : 0;
 #define VC_ROWS_NV(OP, VEC, NV) \
-    launch((rows_kernel<OP, VEC, NV>), dim3(grid), dim3(kBlock), 0, d.stream, in, out, outer, len)
+    launch((rows_kernel<OP, VEC, NV>), dim3(grid), dim3(kBlock), 0, d.stream, in, out, out2, outer, len)
 #define VC_ROWS(OP)                                 \
     if (!vec) VC_ROWS_NV(OP, false, 0);             \
     else if (nv <= 1) VC_ROWS_NV(OP, true, 1);      \
@@ -647,6 +734,7 @@ void reduce_axis(const float* in, float* out, int64_t outer, int64_t len, int64_
     else if (nv <= 16) VC_ROWS_NV(OP, true, 16);    \
     else VC_ROWS_NV(OP, true, 0)
         if (op == VC_REDUCE_SUM) { VC_ROWS(0); }
+        else if (op == VC_REDUCE_MAX && out2) { VC_ROWS(3); }
         else if (op == VC_REDUCE_MAX) { VC_ROWS(1); }
         else { VC_ROWS(2); }
 #undef VC_ROWS
@@ -655,11 +743,25 @@ void reduce_axis(const float* in, float* out, int64_t outer, int64_t len, int64_
         p.done();
         return;
     }
+    if (op != VC_REDUCE_SUM && best_in_one(outer, len, inner)) {
+        // No partial results; the allocation-free entry point's limit is one of shapes, and stays.
+        if (total < target_threads && len >= 64)
+            memory.require(size_t(best_plan(len, total, target_threads).segs * total) * (sizeof(float) + sizeof(int)));
+        if (op == VC_REDUCE_ARGMAX) launch_cols_best<2>(d, in, out, nullptr, outer, len, inner);
+        else if (out2) launch_cols_best<3>(d, in, out, out2, outer, len, inner);
+        else launch_cols_best<1>(d, in, out, nullptr, outer, len, inner);
+        after_launch(label);
+        p.done();
+        return;
+    }
     if (total >= target_threads || len < 64) {
         const unsigned grid = grid_1d(size_t(total), kBlock, unsigned(d.cu_count) * 64);
-        if (op == VC_REDUCE_SUM) launch(cols_kernel<0>, dim3(grid), dim3(kBlock), 0, d.stream, in, out, outer, len, inner);
-        else if (op == VC_REDUCE_MAX) launch(cols_kernel<1>, dim3(grid), dim3(kBlock), 0, d.stream, in, out, outer, len, inner);
-        else launch(cols_kernel<2>, dim3(grid), dim3(kBlock), 0, d.stream, in, out, outer, len, inner);
+#define VC_COLS(OP) launch(cols_kernel<OP>, dim3(grid), dim3(kBlock), 0, d.stream, in, out, out2, outer, len, inner)
+        if (op == VC_REDUCE_SUM) VC_COLS(0);
+        else if (op == VC_REDUCE_ARGMAX) VC_COLS(2);
+        else if (out2) VC_COLS(3);
+        else VC_COLS(1);
+#undef VC_COLS
         after_launch(label);
         p.done();
         return;
@@ -704,6 +806,11 @@ void reduce_axis(const float* in, float* out, int64_t outer, int64_t len, int64_
     int* pi = reinterpret_cast<int*>(mem + size_t(b.segs * total) * sizeof(float));
     launch(cols_best_partial_kernel, grid1, dim3(kBlock), 0, d.stream, in, pv, pi, outer, len, inner, b.seg_len);
     after_launch(label);
+    if (out2) {
+        launch(cols_best_combine_kernel<2>, dim3(grid2), dim3(kBlock), 0, d.stream, in, pv, pi, out2, outer, len, inner,
+               b.segs);
+        after_launch(label);
+    }
     if (op == VC_REDUCE_MAX)
         launch(cols_best_combine_kernel<1>, dim3(grid2), dim3(kBlock), 0, d.stream, in, pv, pi, out, outer, len, inner,
                b.segs);
@@ -752,14 +859,18 @@ class StaticPartials final : public PartialMemory {
 public:
     explicit StaticPartials(void* base) : base_(static_cast<char*>(base)) {}
     void* take(size_t bytes) override {
+        require(bytes);
+        const size_t begin = (used_ + 255) / 256 * 256;
+        used_ = begin + bytes;
+        return base_ + begin;
+    }
+    void require(size_t bytes) const override {
         const size_t begin = (used_ + 255) / 256 * 256;
         if (bytes > kNoAllocScratchBytes || begin > kNoAllocScratchBytes - bytes)
             fail(VC_HIP_ERR_INVALID_ARGUMENT,
                  "vc_hip_reduce_axis_noalloc: this reduction needs " + std::to_string(begin + bytes) +
                      " bytes of partial results; the allocation-free entry point holds " +
                      std::to_string(kNoAllocScratchBytes) + " (use vc_hip_reduce_axis)");
-        used_ = begin + bytes;
-        return base_ + begin;
     }
 
 private:
@@ -821,6 +932,16 @@ int vc_hip_reduce_axis(const float* in, float* out, size_t outer, size_t length,
     return guard([&] {
         PoolPartials memory;
         reduce_axis(in, out, int64_t(outer), int64_t(length), int64_t(inner), op, memory);
+    });
+}
+
+int vc_hip_reduce_axis_max_argmax(const float* in, float* max_out, float* argmax_out, size_t outer, size_t length,
+                                  size_t inner) {
+    return guard([&] {
+        if (outer * inner != 0 && (!max_out || !argmax_out))
+            fail(VC_HIP_ERR_INVALID_ARGUMENT, "vc_hip_reduce_axis_max_argmax: null output");
+        PoolPartials memory;
+        reduce_axis(in, max_out, int64_t(outer), int64_t(length), int64_t(inner), VC_REDUCE_MAX, memory, argmax_out);
     });
 }
 
