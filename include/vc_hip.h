@@ -163,6 +163,11 @@ int vc_hip_binary(const float* a, const size_t* a_shape, const size_t* a_strides
  * src/tensor.cpp:323-330), so no device scalar has to be read:
  * out = a op s (scalar_first == 0) or s op a (scalar_first != 0). */
 int vc_hip_binary_scalar(const float* a, size_t count, float s, int scalar_first, float* out, int op);
+/* vc_hip_binary_scalar on one value, followed by vc_hip_mirror_scalar(out), in
+ * one launch: the last step of a mean (src/tensor.cpp:220), whose value
+ * loss.item() reads. Like the mirrors, no counterpart in the reference. */
+int vc_hip_binary_scalar_published(const float* a, float s, int scalar_first, float* out, int op,
+                                   vc_hip_mirror** mirror);
 /* MetalBackend::unary (metal_backend.hpp:32-33). */
 int vc_hip_unary(const float* in, float* out, size_t count, int op);
 /* MetalBackend::axpy_inplace (metal_backend.hpp:53-54): target += alpha * source. */
@@ -365,6 +370,9 @@ int vc_hip_transpose_last2(const float* in, float* out, size_t batch, size_t row
 /* MetalBackend::reduce_sum (metal_backend.hpp:44-45): out[0] = sum(in),
  * accumulated in double over a shape-fixed partition (deterministic). */
 int vc_hip_reduce_sum(const float* in, size_t count, float* out);
+/* vc_hip_reduce_sum followed by vc_hip_mirror_scalar(out), in one launch. Like
+ * the mirrors, no counterpart in the reference. */
+int vc_hip_reduce_sum_published(const float* in, size_t count, float* out, vc_hip_mirror** mirror);
 /* MetalBackend::reduce_axis (metal_backend.hpp:46-48): [outer, length, inner]
  * -> [outer, inner]. Sum accumulates in double in a shape-fixed order; max and
  * argmax return the first maximum (argmax as a float index), and a NaN first

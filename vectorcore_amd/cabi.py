@@ -102,6 +102,7 @@ _SIGNATURES = {
     "vc_hip_fill": ([_vp, _sz, _f], _i),
     "vc_hip_binary": ([_vp, _szp, _szp, _sz, _vp, _szp, _szp, _sz, _vp, _szp, _sz, _i], _i),
     "vc_hip_binary_scalar": ([_vp, _sz, _f, _i, _vp, _i], _i),
+    "vc_hip_binary_scalar_published": ([_vp, _f, _i, _vp, _i, ctypes.POINTER(_vp)], _i),
     "vc_hip_unary": ([_vp, _vp, _sz, _i], _i),
     "vc_hip_axpy": ([_vp, _vp, _sz, _f], _i),
     "vc_hip_axpy_batch": ([ctypes.POINTER(_vp), ctypes.POINTER(_vp), ctypes.POINTER(_vp), _szp, _sz, _f], _i),
@@ -127,6 +128,7 @@ _SIGNATURES = {
     "vc_hip_matmul_reduce": ([_vp, _vp, _vp, _sz, _sz, _sz, _sz, _sz, _sz, _i, _i], _i),
     "vc_hip_transpose_last2": ([_vp, _vp, _sz, _sz, _sz], _i),
     "vc_hip_reduce_sum": ([_vp, _sz, _vp], _i),
+    "vc_hip_reduce_sum_published": ([_vp, _sz, _vp, ctypes.POINTER(_vp)], _i),
     "vc_hip_reduce_axis": ([_vp, _vp, _sz, _sz, _sz, _i], _i),
     "vc_hip_reduce_axis_max_argmax": ([_vp, _vp, _vp, _sz, _sz, _sz], _i),
     "vc_hip_reduce_axis_noalloc": ([_vp, _vp, _sz, _sz, _sz, _i], _i),

@@ -192,18 +192,8 @@ public:
         return true;
     }
 
-    // Publishes this one-element storage's value, as computed so far in stream
-    // order, for host_copy (vc_hip_mirror_scalar).
-    void publish() {
-        std::lock_guard<std::recursive_mutex> lock(state_mutex());
-        if (elements_ != 1) return;
-        vc_hip_mirror* m = nullptr;
-        check(vc_hip_mirror_scalar(ptr(), &m), "HIP launch failed");
-        adopt_mirror(m);
-    }
-
-    // Takes a mirror already published from this one-element storage (its
-    // producer wrote the host slot, vc_hip_xent_forward_published).
+    // Takes a mirror published from this one-element storage (its producer
+    // wrote the host slot, vc_hip_xent_forward_published).
     void adopt_mirror(vc_hip_mirror* m) {
         std::lock_guard<std::recursive_mutex> lock(state_mutex());
         if (mirror_) (void)vc_hip_mirror_release(mirror_);
@@ -898,6 +888,14 @@ std::shared_ptr<Storage> HipBackend::binary_scalar(const Storage& a, std::size_t
     }
     auto out = fresh(count);
     if (count == 0) return out;
+    if (count == 1) {  // published, as the sums and losses that it scales are: item() on a mean waits for it only
+        vc_hip_mirror* published = nullptr;
+        check(vc_hip_binary_scalar_published(dptr(a, a_offset), s, scalar_first ? 1 : 0, out->ptr(),
+                                             binary_code(operation), &published),
+              "HIP binary op failed");
+        out->adopt_mirror(published);
+        return out;
+    }
     check(vc_hip_binary_scalar(dptr(a, a_offset), count, s, scalar_first ? 1 : 0, out->ptr(), binary_code(operation)),
           "HIP binary op failed");
     return out;
@@ -1017,8 +1015,10 @@ std::shared_ptr<Storage> HipBackend::transpose_last2(const Storage& input, std::
 std::shared_ptr<Storage> HipBackend::reduce_sum(const Storage& input, std::size_t offset, std::size_t count) {
     require(*this);
     auto out = fresh(1);
-    check(vc_hip_reduce_sum(count ? dptr(input, offset) : nullptr, count, out->ptr()), "HIP sum failed");
-    out->publish();  // item() on the sum then waits for this point of the stream only
+    vc_hip_mirror* published = nullptr;  // item() on the sum then waits for this point of the stream only
+    check(vc_hip_reduce_sum_published(count ? dptr(input, offset) : nullptr, count, out->ptr(), &published),
+          "HIP sum failed");
+    out->adopt_mirror(published);
     return out;
 }
 

@@ -196,6 +196,17 @@ __global__ __launch_bounds__(kBlock) void axpy_list_kernel(AxpyList L) {
     }
 }
 
+// One value: y[0] = f(x[0]), also written to a mirror's host slot.
+template <class F>
+__global__ __launch_bounds__(64) void publish_kernel(const float* __restrict__ x, float* __restrict__ y,
+                                                     float* __restrict__ host, F f) {
+    if (threadIdx.x == 0) {
+        const float v = f(x[0]);
+        y[0] = v;
+        host[0] = v;
+    }
+}
+
 // Scalar fallbacks for buffers that are not 16-byte aligned.
 template <class F>
 __global__ __launch_bounds__(kBlock) void map1_scalar_kernel(const float* __restrict__ x, float* __restrict__ y, size_t n, F f) {
@@ -336,6 +347,20 @@ void launch_map2(const char* label, const float* a, const float* b, float* y, si
 }
 
 template <class Op>
+void launch_publish(const float* x, float s, bool scalar_first, float* y, vc_hip_mirror* m) {
+    Device& d = require_device();
+    Profiled p("scalar_publish", 0.0, 8.0);
+    if (scalar_first)
+        launch_publishing(m, publish_kernel<ScalarOp<Op, true>>, dim3(1), dim3(64), d.stream, x, y, m->host,
+                          ScalarOp<Op, true>{s});
+    else
+        launch_publishing(m, publish_kernel<ScalarOp<Op, false>>, dim3(1), dim3(64), d.stream, x, y, m->host,
+                          ScalarOp<Op, false>{s});
+    after_launch("scalar_publish");
+    p.done();
+}
+
+template <class Op>
 void launch_binary(const float* a, const float* b, float* y, size_t n, const Bcast& m, const char* label) {
     Device& d = require_device();
     // Same shape: a plain map.
@@ -451,6 +476,23 @@ int vc_hip_binary_scalar(const float* a, size_t count, float s, int scalar_first
                           : launch_map1("scalar_div", a, out, count, ScalarOp<DivOp, false>{s}, 8.0);
             default: fail(VC_HIP_ERR_INVALID_ARGUMENT, "unknown binary operation");
         }
+    });
+}
+
+int vc_hip_binary_scalar_published(const float* a, float s, int scalar_first, float* out, int op,
+                                   vc_hip_mirror** mirror) {
+    return guard([&] {
+        const bool sf = scalar_first != 0;
+        if (!a || !out) fail(VC_HIP_ERR_INVALID_ARGUMENT, "vc_hip_binary_scalar_published: null buffer");
+        with_mirror(mirror, "vc_hip_binary_scalar_published", [&](vc_hip_mirror* m) {
+            switch (op) {
+                case VC_BINARY_ADD: return launch_publish<AddOp>(a, s, sf, out, m);
+                case VC_BINARY_SUBTRACT: return launch_publish<SubOp>(a, s, sf, out, m);
+                case VC_BINARY_MULTIPLY: return launch_publish<MulOp>(a, s, sf, out, m);
+                case VC_BINARY_DIVIDE: return launch_publish<DivOp>(a, s, sf, out, m);
+                default: fail(VC_HIP_ERR_INVALID_ARGUMENT, "unknown binary operation");
+            }
+        });
     });
 }
 

@@ -821,6 +821,41 @@ void reduce_axis(const float* in, float* out, int64_t outer, int64_t len, int64_
     p.done();
 }
 
+// The last value on its way to the output, also written to a mirror's host slot.
+struct Publish {
+    float* host;
+    __device__ float operator()(float s) const {
+        host[0] = s;
+        return s;
+    }
+};
+
+void reduce_sum(const float* in, size_t count, float* out, vc_hip_mirror* publish) {
+    Device& d = require_device();
+    if (!out) fail(VC_HIP_ERR_INVALID_ARGUMENT, "vc_hip_reduce_sum: null output");
+    const int64_t n = int64_t(count);
+    const int64_t chunk = red::sum_chunk(n);
+    // One launch: at most 2048 chunks (sum_chunk), at least one block.
+    const int64_t blocks = std::max<int64_t>(1, (n + chunk - 1) / chunk);
+    Scratch part(size_t(blocks) * sizeof(double));
+    Profiled p("reduce_sum", double(n), 4.0 * double(n));
+    const dim3 grid{unsigned(blocks)}, block{kBlock};
+    if (publish && aligned16(in))
+        launch_publishing(publish, red::sum_finish_kernel<true, Publish>, grid, block, d.stream, in, part.as<double>(),
+                          out, n, chunk, Publish{publish->host});
+    else if (publish)
+        launch_publishing(publish, red::sum_finish_kernel<false, Publish>, grid, block, d.stream, in, part.as<double>(),
+                          out, n, chunk, Publish{publish->host});
+    else if (aligned16(in))
+        launch(red::sum_finish_kernel<true, red::Identity>, grid, block, 0, d.stream, in, part.as<double>(), out, n,
+               chunk, red::Identity());
+    else
+        launch(red::sum_finish_kernel<false, red::Identity>, grid, block, 0, d.stream, in, part.as<double>(), out, n,
+               chunk, red::Identity());
+    after_launch("reduce_sum");
+    p.done();
+}
+
 // ---- partial results without allocation (vc_hip_reduce_axis_noalloc) ------------
 // A file-scope device array holds the partial results of the
 // allocation-free entry point; each GPU that loads the library holds its own
@@ -908,23 +943,12 @@ using namespace vchip;
 extern "C" {
 
 int vc_hip_reduce_sum(const float* in, size_t count, float* out) {
+    return guard([&] { reduce_sum(in, count, out, nullptr); });
+}
+
+int vc_hip_reduce_sum_published(const float* in, size_t count, float* out, vc_hip_mirror** mirror) {
     return guard([&] {
-        Device& d = require_device();
-        if (!out) fail(VC_HIP_ERR_INVALID_ARGUMENT, "vc_hip_reduce_sum: null output");
-        const int64_t n = int64_t(count);
-        const int64_t chunk = red::sum_chunk(n);
-        // One launch: at most 2048 chunks (sum_chunk), at least one block.
-        const int64_t blocks = std::max<int64_t>(1, (n + chunk - 1) / chunk);
-        Scratch part(size_t(blocks) * sizeof(double));
-        Profiled p("reduce_sum", double(n), 4.0 * double(n));
-        if (aligned16(in))
-            launch(red::sum_finish_kernel<true, red::Identity>, dim3(unsigned(blocks)), dim3(kBlock), 0, d.stream, in,
-                   part.as<double>(), out, n, chunk, red::Identity());
-        else
-            launch(red::sum_finish_kernel<false, red::Identity>, dim3(unsigned(blocks)), dim3(kBlock), 0, d.stream,
-                   in, part.as<double>(), out, n, chunk, red::Identity());
-        after_launch("reduce_sum");
-        p.done();
+        with_mirror(mirror, "vc_hip_reduce_sum_published", [&](vc_hip_mirror* m) { reduce_sum(in, count, out, m); });
     });
 }
 

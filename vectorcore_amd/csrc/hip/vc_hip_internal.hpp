@@ -175,6 +175,35 @@ inline void launch(F kernel, dim3 grid, dim3 block, uint32_t shmem, hipStream_t 
     hipExtLaunchKernelGGL(kernel, grid, block, shmem, stream, start, stop, 0u, args...);
 }
 
+// launch() of a kernel that writes a mirror's host slot: its dispatch carries
+// the mirror's completion event (recorded after it while the profiler holds
+// the dispatch's events).
+template <typename F, typename... Args>
+inline void launch_publishing(vc_hip_mirror* m, F kernel, dim3 grid, dim3 block, hipStream_t stream, Args... args) {
+    Profiled* p = Profiled::current();
+    if (p && p->stop_event()) {
+        launch(kernel, grid, block, 0, stream, args...);
+        check_hip(hipEventRecord(m->done, stream), "hipEventRecord");
+    } else {
+        hipExtLaunchKernelGGL(kernel, grid, block, 0, stream, nullptr, m->done, 0u, args...);
+    }
+}
+
+// forward(m) with a mirror taken for it, handed to *mirror on success.
+template <typename F>
+void with_mirror(vc_hip_mirror** mirror, const char* name, F&& forward) {
+    if (!mirror) fail(VC_HIP_ERR_INVALID_ARGUMENT, std::string(name) + ": null mirror");
+    *mirror = nullptr;
+    vc_hip_mirror* m = take_mirror();
+    try {
+        forward(m);
+    } catch (...) {
+        give_mirror(m);
+        throw;
+    }
+    *mirror = m;
+}
+
 // --- launch-shape checks -----------------------------------------------------
 inline unsigned grid_1d(size_t items, unsigned block, unsigned max_blocks) {
     size_t blocks = (items + block - 1) / block;

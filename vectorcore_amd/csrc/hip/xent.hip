@@ -874,21 +874,6 @@ void xent_forward(const float* logits, const int32_t* targets, size_t rows, size
     p.done();
 }
 
-// Runs forward(m) with a mirror taken for it, handed to *mirror on success.
-template <class F>
-void with_mirror(vc_hip_mirror** mirror, const char* name, F&& forward) {
-    if (!mirror) fail(VC_HIP_ERR_INVALID_ARGUMENT, std::string(name) + ": null mirror");
-    require_device();
-    vc_hip_mirror* m = take_mirror();
-    try {
-        forward(m);
-    } catch (...) {
-        give_mirror(m);
-        throw;
-    }
-    *mirror = m;
-}
-
 // The backward with the column sums of dx (vc_hip_xent_backward_colsum):
 // for rows of at most 2048 classes the kernel keeps one partial row per
 // kColRows rows, finished next by column_partials_kernel or, with `pending`,
