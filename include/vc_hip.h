@@ -264,13 +264,18 @@ int vc_hip_map(const vc_hip_map_program* program);
  * input_kinds[j], one value per element, per column (cols values), per row
  * (rows values) or, the rows being groups of axis_length, per group and column
  * (rows / axis_length * cols values; axis_length divides rows). Two more
- * operations: AT_ROW gives slot b where int(slot a) is the row's number within
+ * positions: AT_ROW gives slot b where int(slot a) is the row's number within
  * its group and 0 elsewhere, AT_COLUMN the same for the column (the gradient
- * of a maximum along an axis). row_sums[s] ([rows]) receives the sums of slot
+ * of a maximum along an axis); and the functions of slot a that vc_hip_unary
+ * has, with its bits (src/ops.cpp:361-413). row_sums[s] ([rows]) receives the sums of slot
  * row_sum_slots[s] over the columns, added in double in a fixed order; a
  * program has row sums or column sums. Fewer than 2^31 elements, at least one. */
 #define VC_MAP_AT_ROW 6
 #define VC_MAP_AT_COLUMN 7
+#define VC_MAP_RELU 8
+#define VC_MAP_SIGMOID 9
+#define VC_MAP_EXP 10
+#define VC_MAP_LOG 11
 #define VC_MAP_FULL 0
 #define VC_MAP_PER_COLUMN 1
 #define VC_MAP_PER_ROW 2

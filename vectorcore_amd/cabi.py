@@ -40,7 +40,7 @@ class MapProgram(ctypes.Structure):
                 ("rows", _sz), ("cols", _sz)]
 
 
-MAP_AT_ROW, MAP_AT_COLUMN = 6, 7
+MAP_AT_ROW, MAP_AT_COLUMN, MAP_RELU, MAP_SIGMOID, MAP_EXP, MAP_LOG = range(6, 12)
 MAP_FULL, MAP_PER_COLUMN, MAP_PER_ROW, MAP_PER_GROUP = range(4)
 
 

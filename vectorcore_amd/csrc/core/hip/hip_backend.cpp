@@ -633,7 +633,10 @@ std::atomic<bool>& fuse_flag() {
     return flag;
 }
 
-bool deferring() { return t_elementwise_depth > 0 && fuse_flag().load(); }
+// One forward op whose result needs a gradient (HipBackend::ForwardScope).
+thread_local bool t_forward = false;
+
+bool deferring() { return (t_elementwise_depth > 0 || t_forward) && fuse_flag().load(); }
 
 // The expression of an operand: its own when it is a whole pending
 // expression of `count` values, otherwise an input node over its buffer
@@ -683,7 +686,7 @@ std::shared_ptr<HipStorage> pending_storage(std::size_t elements, MapExpr expr, 
     std::vector<std::shared_ptr<HipStorage>> inputs;
     expr_inputs(*expr, inputs);
     for (const auto& in : inputs) in->add_reader(out);
-    t_pending.push_back(out);
+    if (t_elementwise_depth > 0) t_pending.push_back(out);
     return out;
 }
 
@@ -880,7 +883,7 @@ std::shared_ptr<Storage> HipBackend::binary(const Storage& a, std::size_t a_offs
 std::shared_ptr<Storage> HipBackend::binary_scalar(const Storage& a, std::size_t a_offset, std::size_t count, float s,
                                                    bool scalar_first, cpu::BinaryOp operation) {
     require(*this);
-    if (deferring() && count > 0) {
+    if (deferring() && count > (t_forward ? 1U : 0U)) {  // (a forward's one value is published below)
         const int op = binary_code(operation);
         return deferred_map(count, {{&a, a_offset}}, [op, s, scalar_first](std::vector<MapExpr>& x) {
             return scalar_first ? op_expr(op, constant_expr(s), x[0]) : op_expr(op, x[0], constant_expr(s));
@@ -888,7 +891,7 @@ std::shared_ptr<Storage> HipBackend::binary_scalar(const Storage& a, std::size_t
     }
     auto out = fresh(count);
     if (count == 0) return out;
-    if (count == 1) {  // published, as the sums and losses that it scales are: item() on a mean waits for it only
+    if (count == 1 && t_elementwise_depth == 0) {  // published, as the sums and losses that it scales are: item() on a mean waits for it only
         vc_hip_mirror* published = nullptr;
         check(vc_hip_binary_scalar_published(dptr(a, a_offset), s, scalar_first ? 1 : 0, out->ptr(),
                                              binary_code(operation), &published),
@@ -904,10 +907,18 @@ std::shared_ptr<Storage> HipBackend::binary_scalar(const Storage& a, std::size_t
 std::shared_ptr<Storage> HipBackend::unary(const Storage& input, std::size_t offset, std::size_t count,
                                            cpu::UnaryOp operation) {
     require(*this);
-    if (deferring() && count > 0 &&
-        (operation == cpu::UnaryOp::Negate || operation == cpu::UnaryOp::ReluGradient)) {
-        const int op = operation == cpu::UnaryOp::Negate ? VC_MAP_NEG : VC_MAP_STEP;
-        return deferred_map(count, {{&input, offset}},
+    if (deferring() && count > (t_forward ? 1U : 0U)) {
+        int op = -1;
+        const bool matrix = count < (std::size_t(1) << 31);  // the functions' programs are matrix programs
+        switch (operation) {
+            case cpu::UnaryOp::Negate: op = VC_MAP_NEG; break;
+            case cpu::UnaryOp::ReluGradient: op = VC_MAP_STEP; break;
+            case cpu::UnaryOp::Relu: op = matrix ? VC_MAP_RELU : -1; break;
+            case cpu::UnaryOp::Sigmoid: op = matrix ? VC_MAP_SIGMOID : -1; break;
+            case cpu::UnaryOp::Exp: op = matrix ? VC_MAP_EXP : -1; break;
+            case cpu::UnaryOp::Log: op = matrix ? VC_MAP_LOG : -1; break;
+        }
+        if (op >= 0) return deferred_map(count, {{&input, offset}},
                             [op](std::vector<MapExpr>& x) { return op_expr(op, x[0], nullptr); });
     }
     auto out = fresh(count);
@@ -1042,11 +1053,15 @@ std::shared_ptr<Storage> HipBackend::reduce_axis(const Storage& input, std::size
     }
     // Row sums of a pending expression: summed as it is computed. (It is computed again where something
     // else reads it, from inputs that this program has just read.)
-    if (operation == cpu::ReduceOp::Sum && inner == 1 && offset == 0 && outer > 1 && length > 1 && deferring() &&
+    if (operation == cpu::ReduceOp::Sum && inner == 1 && offset == 0 && outer > 1 && length > 1 && fuse_flag().load() &&
         outer * length == input.size() && input.size() < (std::size_t(1) << 31)) {
         std::lock_guard<std::recursive_mutex> lock(state_mutex());
         if (MapExpr e = as_hip(input).map_expr())
-            if (e->kind == MapNode::Kind::Op && fits({e.get()}, length)) return pending_storage(outer, e, length, true);
+            if (e->kind == MapNode::Kind::Op && fits({e.get()}, length)) {
+                auto sums = pending_storage(outer, e, length, true);
+                if (t_elementwise_depth == 0) (void)sums->ptr();  // a forward's sum, computed here
+                return sums;
+            }
     }
     auto out = fresh(outer * inner);
     if (outer * inner == 0) return out;
@@ -1155,6 +1170,15 @@ bool HipBackend::defer_products() const { return defer_flag(); }
 
 void HipBackend::set_fuse_elementwise(bool enable) { fuse_flag() = enable; }
 bool HipBackend::fuse_elementwise() const { return fuse_flag(); }
+
+HipBackend::ForwardScope::ForwardScope(bool defer) : previous_(t_forward) { t_forward = defer; }
+HipBackend::ForwardScope::~ForwardScope() { t_forward = previous_; }
+
+void HipBackend::include(const std::shared_ptr<Storage>& storage) {
+    auto h = std::dynamic_pointer_cast<HipStorage>(storage);
+    std::lock_guard<std::recursive_mutex> lock(state_mutex());
+    if (h && h->map_pending()) t_pending.push_back(h);
+}
 
 HipBackend::ElementwiseScope::ElementwiseScope() {
     if (t_elementwise_depth++ == 0) t_pending.clear();

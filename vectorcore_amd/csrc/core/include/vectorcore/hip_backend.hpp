@@ -130,7 +130,21 @@ public:
     // are added in a different fixed order from reduce_axis's: deterministic
     // for either setting, they can differ in the last bit between the two. On
     // by default; VECTORCORE_HIP_FUSE=0 or set_fuse_elementwise(false) keeps
-    // every op eager.
+    // every op eager. The forward's elementwise ops whose result needs a
+    // gradient record expressions too (ForwardScope, one per op): the backward
+    // pass computes again what its rules read of them, in the programs that
+    // compute the gradients, and the pass's result with them (include); what
+    // else is read is computed then.
+    class ForwardScope {
+    public:
+        explicit ForwardScope(bool defer);
+        ~ForwardScope();
+        ForwardScope(const ForwardScope&) = delete;
+        ForwardScope& operator=(const ForwardScope&) = delete;
+
+    private:
+        bool previous_;
+    };
     class ElementwiseScope {
     public:
         ElementwiseScope();
@@ -139,6 +153,8 @@ public:
         ElementwiseScope& operator=(const ElementwiseScope&) = delete;
     };
     void flush_elementwise();
+    // Computes a still pending storage with the scope's, at its flush.
+    void include(const std::shared_ptr<Storage>& storage);
     void set_fuse_elementwise(bool enable);
     [[nodiscard]] bool fuse_elementwise() const;
 

@@ -46,6 +46,10 @@ HipBackend& hip() { return HipBackend::instance(); }
 const Storage& st(const Tensor& t) { return *t.impl()->storage; }
 std::size_t off(const Tensor& t) { return t.impl()->offset; }
 
+// hip: whether an elementwise result is recorded for the backward pass to
+// compute again, rather than computed now (HipBackend::ForwardScope).
+bool needs_gradient(const Tensor& v) { return grad_enabled() && v.requires_grad(); }
+
 void require_same_device(const Tensor& a, const Tensor& b) {
     if (a.device() != b.device())
         throw std::invalid_argument("tensor device mismatch: " + a.device().str() + " vs " + b.device().str());
@@ -61,9 +65,11 @@ Tensor binary_forward(const Tensor& a, const Tensor& b, cpu::BinaryOp op) {
             cpu::binary(a.data(), a.shape(), a.strides(), b.data(), b.shape(), b.strides(), s->mutable_data(), out_shape,
                         op);
             break;
-        case DeviceType::HIP:
+        case DeviceType::HIP: {
+            const HipBackend::ForwardScope forward(needs_gradient(a) || needs_gradient(b));
             s = hip().binary(st(a), off(a), a.shape(), a.strides(), st(b), off(b), b.shape(), b.strides(), out_shape, op);
             break;
+        }
         case DeviceType::METAL: metal_unavailable();
     }
     return detail::make_tensor(std::move(s), out_shape, false);
@@ -76,7 +82,11 @@ Tensor unary_forward(const Tensor& v, cpu::UnaryOp op) {
             s = make_cpu_storage(v.numel());
             cpu::unary(v.data(), s->mutable_data(), v.numel(), op);
             break;
-        case DeviceType::HIP: s = hip().unary(st(v), off(v), v.numel(), op); break;
+        case DeviceType::HIP: {
+            const HipBackend::ForwardScope forward(needs_gradient(v));
+            s = hip().unary(st(v), off(v), v.numel(), op);
+            break;
+        }
         case DeviceType::METAL: metal_unavailable();
     }
     return detail::make_tensor(std::move(s), v.shape(), false);

@@ -295,7 +295,10 @@ void Tensor::backward(const Tensor& gradient) const {
     std::optional<HipBackend::ElementwiseScope> fusion;
     if (gradient.device() == Device::hip()) fusion.emplace();
     run_backward(impl_, order, gradient);
-    if (fusion) HipBackend::instance().flush_elementwise();
+    if (fusion) {
+        HipBackend::instance().include(impl_->storage);  // the result itself, where nothing has read it yet
+        HipBackend::instance().flush_elementwise();
+    }
 }
 
 namespace {

@@ -9,6 +9,7 @@
 // reference's CPU kernels (src/cpu/cpu_backend.cpp:24-27, 291-316); the build
 // disables floating-point contraction, so no fused multiply-add changes a
 // rounding.
+#include "functions.hpp"
 #include "reduce_common.hpp"
 #include "vc_hip_internal.hpp"
 
@@ -39,19 +40,6 @@ struct MulOp { __device__ float operator()(float a, float b) const { return a * 
 struct DivOp { __device__ float operator()(float a, float b) const { return a / b; } };
 
 struct NegOp { __device__ float operator()(float x) const { return -x; } };
-struct ReluOp { __device__ float operator()(float x) const { return x > 0.0f ? x : 0.0f; } };
-struct ReluGradOp { __device__ float operator()(float x) const { return x > 0.0f ? 1.0f : 0.0f; } };
-struct SigmoidOp {
-    // The branch keeps exp() from overflowing (src/cpu/cpu_backend.cpp:302-307).
-    __device__ float operator()(float x) const {
-        if (x >= 0.0f) return 1.0f / (1.0f + expf(-x));
-        const float e = expf(x);
-        return e / (1.0f + e);
-    }
-};
-struct ExpOp { __device__ float operator()(float x) const { return expf(x); } };
-struct LogOp { __device__ float operator()(float x) const { return logf(x); } };
-
 // Binary op against a scalar held in a kernel argument.
 template <class Op, bool ScalarFirst>
 struct ScalarOp {

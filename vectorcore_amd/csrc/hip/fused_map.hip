@@ -125,7 +125,7 @@ void validate(const vc_hip_map_program& p, const vc_hip_map_matrix* m) {
     for (size_t k = 0; k < p.n_code; ++k) {
         const uint32_t w = p.code[k];
         const unsigned op = w & 255u, a = (w >> 8) & 255u, b = (w >> 16) & 255u, dst = w >> 24;
-        if (op > (m ? VC_MAP_AT_COLUMN : VC_MAP_STEP)) bad("unknown opcode at instruction " + std::to_string(k));
+        if (op > (m ? VC_MAP_LOG : VC_MAP_STEP)) bad("unknown opcode at instruction " + std::to_string(k));
         if (a >= unsigned(kSlots) || b >= unsigned(kSlots) || dst >= unsigned(kSlots))
             bad("slot out of range at instruction " + std::to_string(k));
         if (!(written >> a & 1u) || !(written >> b & 1u))

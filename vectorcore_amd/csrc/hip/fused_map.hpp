@@ -4,6 +4,7 @@
 // interpreters compile in parallel; fused_map.hip holds the C ABI.
 #pragma once
 
+#include "functions.hpp"
 #include "reduce_common.hpp"
 #include "vc_hip_internal.hpp"
 
@@ -157,56 +158,97 @@ __device__ inline Vals<W> load_any(const float* __restrict__ p) {
     return o;
 }
 
-// The first Code instructions (Code >= n_code), unrolled so that every word
-// is a kernel-argument scalar. `at`: the values' coordinates (matrix programs).
+// One instruction on the W values of every slot. `at`: their coordinates
+// (matrix programs).
+template <bool Matrix, int W>
+__device__ inline void step(Regs<W>& r, const Program& P, const Place<W>& at, uint32_t word) {
+            const int op = int(word & 255u), ia = int((word >> 8) & 255u), ib = int((word >> 16) & 255u),
+                      id = int(word >> 24);
+            const Vals<W> a = get(r, ia), b = get(r, ib);
+            Vals<W> v;
+            if constexpr (Matrix) {
+                if (op >= VC_MAP_AT_ROW) {
+                    switch (op) {
+                        case VC_MAP_RELU:
+    #pragma unroll
+                            for (int j = 0; j < W; ++j) v.v[j] = ReluOp()(a.v[j]);
+                            break;
+                        case VC_MAP_SIGMOID:
+    #pragma unroll
+                            for (int j = 0; j < W; ++j) v.v[j] = SigmoidOp()(a.v[j]);
+                            break;
+                        case VC_MAP_EXP:
+    #pragma unroll
+                            for (int j = 0; j < W; ++j) v.v[j] = ExpOp()(a.v[j]);
+                            break;
+                        case VC_MAP_LOG:
+    #pragma unroll
+                            for (int j = 0; j < W; ++j) v.v[j] = LogOp()(a.v[j]);
+                            break;
+                        default:  // VC_MAP_AT_ROW or VC_MAP_AT_COLUMN
+    #pragma unroll
+                            for (int j = 0; j < W; ++j) {
+                                const uint32_t axis = op == VC_MAP_AT_ROW ? at.in_group[j] : at.c[j];
+                                v.v[j] = int(a.v[j]) == int(axis) ? b.v[j] : 0.0f;
+                            }
+                            break;
+                    }
+                    put(r, id, v);
+                    return;
+                }
+            }
+            switch (op) {
+                case VC_MAP_ADD:
+    #pragma unroll
+                    for (int j = 0; j < W; ++j) v.v[j] = a.v[j] + b.v[j];
+                    break;
+                case VC_MAP_SUB:
+    #pragma unroll
+                    for (int j = 0; j < W; ++j) v.v[j] = a.v[j] - b.v[j];
+                    break;
+                case VC_MAP_MUL:
+    #pragma unroll
+                    for (int j = 0; j < W; ++j) v.v[j] = a.v[j] * b.v[j];
+                    break;
+                case VC_MAP_DIV:
+    #pragma unroll
+                    for (int j = 0; j < W; ++j) v.v[j] = a.v[j] / b.v[j];
+                    break;
+                case VC_MAP_NEG:
+    #pragma unroll
+                    for (int j = 0; j < W; ++j) v.v[j] = -a.v[j];
+                    break;
+                default:  // VC_MAP_STEP
+    #pragma unroll
+                    for (int j = 0; j < W; ++j) v.v[j] = a.v[j] > 0.0f ? 1.0f : 0.0f;
+                    break;
+            }
+            put(r, id, v);
+}
+
+// The program. Its words are kernel arguments: flat and plain column programs
+// unroll the first Code of them (Code >= n_code), so that every word is a
+// scalar. Matrix programs, whose functions make an instruction's code long, loop
+// over one copy of it, each word loaded while the one before runs: the unrolled
+// copies are no faster (bias, activations and their product on 4096 x 4096 with
+// gradients, 16 instructions: 116-127 us, 119 looped; rows of 8192 x 1024 to
+// mean 0 and variance 1: 229 us, 224 looped), and eight times the code.
 template <int Code, bool Matrix, int W>
 __device__ inline void run(Regs<W>& r, const Program& P, const Place<W>& at) {
-#pragma unroll
-    for (int k = 0; k < Code; ++k) {
-        if (k >= P.n_code) continue;  // uniform: the rest of the loop is skipped
-        const uint32_t word = P.code[k];
-        const int op = int(word & 255u), ia = int((word >> 8) & 255u), ib = int((word >> 16) & 255u),
-                  id = int(word >> 24);
-        const Vals<W> a = get(r, ia), b = get(r, ib);
-        Vals<W> v;
-        if constexpr (Matrix) {
-            if (op >= VC_MAP_AT_ROW) {  // VC_MAP_AT_ROW or VC_MAP_AT_COLUMN
-#pragma unroll
-                for (int j = 0; j < W; ++j) {
-                    const uint32_t axis = op == VC_MAP_AT_ROW ? at.in_group[j] : at.c[j];
-                    v.v[j] = int(a.v[j]) == int(axis) ? b.v[j] : 0.0f;
-                }
-                put(r, id, v);
-                continue;
-            }
+    if constexpr (Matrix) {
+        uint32_t next = P.code[0];
+#pragma nounroll
+        for (int k = 0; k < P.n_code; ++k) {
+            const uint32_t word = next;
+            next = P.code[k + 1 < kCode ? k + 1 : 0];
+            step<Matrix>(r, P, at, word);
         }
-        switch (op) {
-            case VC_MAP_ADD:
+    } else {
 #pragma unroll
-                for (int j = 0; j < W; ++j) v.v[j] = a.v[j] + b.v[j];
-                break;
-            case VC_MAP_SUB:
-#pragma unroll
-                for (int j = 0; j < W; ++j) v.v[j] = a.v[j] - b.v[j];
-                break;
-            case VC_MAP_MUL:
-#pragma unroll
-                for (int j = 0; j < W; ++j) v.v[j] = a.v[j] * b.v[j];
-                break;
-            case VC_MAP_DIV:
-#pragma unroll
-                for (int j = 0; j < W; ++j) v.v[j] = a.v[j] / b.v[j];
-                break;
-            case VC_MAP_NEG:
-#pragma unroll
-                for (int j = 0; j < W; ++j) v.v[j] = -a.v[j];
-                break;
-            default:  // VC_MAP_STEP
-#pragma unroll
-                for (int j = 0; j < W; ++j) v.v[j] = a.v[j] > 0.0f ? 1.0f : 0.0f;
-                break;
+        for (int k = 0; k < Code; ++k) {
+            if (k >= P.n_code) continue;  // uniform: the rest of the loop is skipped
+            step<Matrix>(r, P, at, P.code[k]);
         }
-        put(r, id, v);
     }
 }
 
@@ -285,7 +327,7 @@ __global__ __launch_bounds__(kMapBlock) void map_flat_kernel(Program P, int64_t 
 // map_flat_kernel of a matrix program: full inputs and outputs are read and
 // written as there, whatever the columns; the other inputs by coordinates. The
 // last group of count % W values is a launch of its own from element `first`.
-template <int NIn, int W, int Code>
+template <int NIn, int W>
 __global__ __launch_bounds__(kMapBlock) void map_matrix_kernel(Program P, int64_t groups, int64_t first) {
     Regs<W> r;
     set_constants(r, P, NIn);
@@ -294,7 +336,7 @@ __global__ __launch_bounds__(kMapBlock) void map_matrix_kernel(Program P, int64_
         const int64_t e = first + g * W;
         const Place<W> at = place_of<W>(P, uint32_t(e));
         load_matrix_inputs<NIn, W>(r, P, e, at);
-        run<Code, true>(r, P, at);
+        run<0, true>(r, P, at);
         store_outputs(r, P, e);
     }
 }
@@ -305,7 +347,7 @@ __global__ __launch_bounds__(kMapBlock) void map_matrix_kernel(Program P, int64_
 // with the row (its first values are computed and written twice, and added
 // once). Sums in double: each lane in column order, then red::wave_sum's order,
 // then wave order.
-template <int NIn, int W, int Lanes, int Code>
+template <int NIn, int W, int Lanes>
 __global__ __launch_bounds__(kMapBlock) void map_rows_kernel(Program P, int64_t rows) {
     constexpr int kWaves = Lanes / 64;
     __shared__ double wave_part[kSums][4];
@@ -321,7 +363,7 @@ __global__ __launch_bounds__(kMapBlock) void map_rows_kernel(Program P, int64_t 
             const int64_t e = row * cols + c1;
             const Place<W> at = place_at<W>(P, uint32_t(row), c1);
             load_matrix_inputs<NIn, W>(r, P, e, at);
-            run<Code, true>(r, P, at);
+            run<0, true>(r, P, at);
 #pragma unroll
             for (int j = 0; j < kOutputs; ++j)
                 if (j < P.n_out) store_any<W>(P.out[j] + e, get(r, P.out_slot[j]));
@@ -459,8 +501,8 @@ void launch_columns(Device& d, const Program& P, int64_t rows, int64_t cols, boo
     const ColumnGrid g = column_grid(rows, cols, vec ? 4 : 1);
     const dim3 grid(unsigned(g.col_blocks), unsigned(g.gy));
     if (P.cols != 0) {  // a matrix program
-        if (vec && P.n_code <= kShortCode && P.n_sum == 1)
-            launch(map_columns_kernel<NIn, 4, kShortCode, 1, true>, grid, dim3(kMapBlock), 0, d.stream, P, rows, cols, part);
+        if (vec && P.n_sum == 1)
+            launch(map_columns_kernel<NIn, 4, kCode, 1, true>, grid, dim3(kMapBlock), 0, d.stream, P, rows, cols, part);
         else if (vec)
             launch(map_columns_kernel<NIn, 4, kCode, kSums, true>, grid, dim3(kMapBlock), 0, d.stream, P, rows, cols, part);
         else
@@ -478,15 +520,12 @@ void launch_columns(Device& d, const Program& P, int64_t rows, int64_t cols, boo
 template <int NIn>
 void launch_matrix(Device& d, const Program& P, int64_t count, bool vec) {
     const int64_t groups = vec ? count / 4 : 0;
-    if (groups > 0 && P.n_code <= kShortCode)
-        launch(map_matrix_kernel<NIn, 4, kShortCode>, dim3(grid_1d(size_t(groups), kMapBlock, kFlatBlocks)), dim3(kMapBlock),
-               0, d.stream, P, groups, int64_t(0));
-    else if (groups > 0)
-        launch(map_matrix_kernel<NIn, 4, kCode>, dim3(grid_1d(size_t(groups), kMapBlock, kFlatBlocks)), dim3(kMapBlock), 0,
+    if (groups > 0)
+        launch(map_matrix_kernel<NIn, 4>, dim3(grid_1d(size_t(groups), kMapBlock, kFlatBlocks)), dim3(kMapBlock), 0,
                d.stream, P, groups, int64_t(0));
     if (groups * 4 < count) {
         const int64_t rest = count - groups * 4;
-        launch(map_matrix_kernel<NIn, 1, kCode>, dim3(grid_1d(size_t(rest), kMapBlock, kFlatBlocks)), dim3(kMapBlock), 0,
+        launch(map_matrix_kernel<NIn, 1>, dim3(grid_1d(size_t(rest), kMapBlock, kFlatBlocks)), dim3(kMapBlock), 0,
                d.stream, P, rest, groups * 4);
     }
 }
@@ -496,12 +535,9 @@ template <int NIn>
 void launch_rows(Device& d, const Program& P, int64_t rows) {
     const bool wide = rows < 2048 && P.cols > 1024;
     const unsigned grid = unsigned(std::min<int64_t>(wide ? rows : (rows + 3) / 4, kFlatBlocks));
-    const bool brief = P.n_code <= kShortCode;
-    if (P.cols < 4) launch(map_rows_kernel<NIn, 1, 64, kCode>, dim3(grid), dim3(kMapBlock), 0, d.stream, P, rows);
-    else if (wide && brief) launch(map_rows_kernel<NIn, 4, 256, kShortCode>, dim3(grid), dim3(kMapBlock), 0, d.stream, P, rows);
-    else if (wide) launch(map_rows_kernel<NIn, 4, 256, kCode>, dim3(grid), dim3(kMapBlock), 0, d.stream, P, rows);
-    else if (brief) launch(map_rows_kernel<NIn, 4, 64, kShortCode>, dim3(grid), dim3(kMapBlock), 0, d.stream, P, rows);
-    else launch(map_rows_kernel<NIn, 4, 64, kCode>, dim3(grid), dim3(kMapBlock), 0, d.stream, P, rows);
+    if (P.cols < 4) launch(map_rows_kernel<NIn, 1, 64>, dim3(grid), dim3(kMapBlock), 0, d.stream, P, rows);
+    else if (wide) launch(map_rows_kernel<NIn, 4, 256>, dim3(grid), dim3(kMapBlock), 0, d.stream, P, rows);
+    else launch(map_rows_kernel<NIn, 4, 64>, dim3(grid), dim3(kMapBlock), 0, d.stream, P, rows);
 }
 
 }  // namespace fmap
