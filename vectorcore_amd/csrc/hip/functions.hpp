@@ -9,11 +9,11 @@ namespace vchip {
 struct ReluOp { __device__ float operator()(float x) const { return x > 0.0f ? x : 0.0f; } };
 struct ReluGradOp { __device__ float operator()(float x) const { return x > 0.0f ? 1.0f : 0.0f; } };
 struct SigmoidOp {
-    // The branch keeps exp() from overflowing (src/cpu/cpu_backend.cpp:302-307).
+    // exp(-|x|) cannot overflow: 1 / (1 + e) from 0 up, e / (1 + e) below (src/cpu/cpu_backend.cpp:302-307),
+    // without a branch whose two sides a wavefront would run one after the other.
     __device__ float operator()(float x) const {
-        if (x >= 0.0f) return 1.0f / (1.0f + expf(-x));
-        const float e = expf(x);
-        return e / (1.0f + e);
+        const float e = expf(-fabsf(x));
+        return (x >= 0.0f ? 1.0f : e) / (1.0f + e);
     }
 };
 struct ExpOp { __device__ float operator()(float x) const { return expf(x); } };

@@ -241,9 +241,16 @@ int vc_hip_map_broadcast(const vc_hip_map_program* program, const vc_hip_map_mat
         set_magic(P.len, P.len_magic, P.len_shift);
         bool vec = true;
         double bytes = 4.0 * double(p.rows * p.cols) * double(p.n_outputs);
+        P.count = uint32_t(p.rows * p.cols);
         for (size_t j = 0; j < p.n_inputs; ++j) {
-            P.kind[j] = m.input_kinds[j];
-            if (m.input_kinds[j] == VC_MAP_FULL) bytes += 4.0 * double(p.rows * p.cols);
+            // One value per row of one column, per group of one row or per column of one row is one per
+            // element; the others have at most half as many values.
+            const int kind = m.input_kinds[j];
+            const size_t share = kind == VC_MAP_PER_COLUMN ? p.rows : kind == VC_MAP_PER_ROW ? p.cols
+                               : kind == VC_MAP_PER_GROUP  ? m.axis_length : 1;
+            P.kind[j] = share == 1 ? VC_MAP_FULL : m.input_kinds[j];
+            P.extent[j] = uint32_t(P.count / share);
+            if (P.kind[j] == VC_MAP_FULL) bytes += 4.0 * double(p.rows * p.cols);
         }
         for (size_t j = 0; j < p.n_outputs; ++j) vec = vec && aligned16(p.outputs[j]);
         const int n_in = int(p.n_inputs);

@@ -38,7 +38,8 @@ struct Program {
     // Matrix programs (vc_hip_map_broadcast): how each input is indexed
     // (VC_MAP_FULL ...), and the matrix.
     uint8_t kind[kInputs];
-    uint32_t cols, len;
+    uint32_t extent[kInputs];  // values of an input that is not full
+    uint32_t cols, len, count;
     uint32_t cols_magic, cols_shift, len_magic, len_shift;  // for divide()
 };
 
@@ -162,68 +163,70 @@ __device__ inline Vals<W> load_any(const float* __restrict__ p) {
 // (matrix programs).
 template <bool Matrix, int W>
 __device__ inline void step(Regs<W>& r, const Program& P, const Place<W>& at, uint32_t word) {
-            const int op = int(word & 255u), ia = int((word >> 8) & 255u), ib = int((word >> 16) & 255u),
-                      id = int(word >> 24);
-            const Vals<W> a = get(r, ia), b = get(r, ib);
-            Vals<W> v;
-            if constexpr (Matrix) {
-                if (op >= VC_MAP_AT_ROW) {
-                    switch (op) {
-                        case VC_MAP_RELU:
-    #pragma unroll
-                            for (int j = 0; j < W; ++j) v.v[j] = ReluOp()(a.v[j]);
-                            break;
-                        case VC_MAP_SIGMOID:
-    #pragma unroll
-                            for (int j = 0; j < W; ++j) v.v[j] = SigmoidOp()(a.v[j]);
-                            break;
-                        case VC_MAP_EXP:
-    #pragma unroll
-                            for (int j = 0; j < W; ++j) v.v[j] = ExpOp()(a.v[j]);
-                            break;
-                        case VC_MAP_LOG:
-    #pragma unroll
-                            for (int j = 0; j < W; ++j) v.v[j] = LogOp()(a.v[j]);
-                            break;
-                        default:  // VC_MAP_AT_ROW or VC_MAP_AT_COLUMN
-    #pragma unroll
-                            for (int j = 0; j < W; ++j) {
-                                const uint32_t axis = op == VC_MAP_AT_ROW ? at.in_group[j] : at.c[j];
-                                v.v[j] = int(a.v[j]) == int(axis) ? b.v[j] : 0.0f;
-                            }
-                            break;
+    const int op = int(word & 255u), ia = int((word >> 8) & 255u), ib = int((word >> 16) & 255u), id = int(word >> 24);
+    const Vals<W> a = get(r, ia);
+    Vals<W> v;
+    if constexpr (Matrix) {
+        if (op >= VC_MAP_AT_ROW) {
+            switch (op) {
+                case VC_MAP_RELU:
+#pragma unroll
+                    for (int j = 0; j < W; ++j) v.v[j] = ReluOp()(a.v[j]);
+                    break;
+                case VC_MAP_SIGMOID:
+#pragma unroll
+                    for (int j = 0; j < W; ++j) v.v[j] = SigmoidOp()(a.v[j]);
+                    break;
+                case VC_MAP_EXP:
+#pragma unroll
+                    for (int j = 0; j < W; ++j) v.v[j] = ExpOp()(a.v[j]);
+                    break;
+                case VC_MAP_LOG:
+#pragma unroll
+                    for (int j = 0; j < W; ++j) v.v[j] = LogOp()(a.v[j]);
+                    break;
+                default: {  // VC_MAP_AT_ROW or VC_MAP_AT_COLUMN
+                    const Vals<W> b = get(r, ib);
+#pragma unroll
+                    for (int j = 0; j < W; ++j) {
+                        const uint32_t axis = op == VC_MAP_AT_ROW ? at.in_group[j] : at.c[j];
+                        v.v[j] = int(a.v[j]) == int(axis) ? b.v[j] : 0.0f;
                     }
-                    put(r, id, v);
-                    return;
+                    break;
                 }
             }
-            switch (op) {
-                case VC_MAP_ADD:
-    #pragma unroll
-                    for (int j = 0; j < W; ++j) v.v[j] = a.v[j] + b.v[j];
-                    break;
-                case VC_MAP_SUB:
-    #pragma unroll
-                    for (int j = 0; j < W; ++j) v.v[j] = a.v[j] - b.v[j];
-                    break;
-                case VC_MAP_MUL:
-    #pragma unroll
-                    for (int j = 0; j < W; ++j) v.v[j] = a.v[j] * b.v[j];
-                    break;
-                case VC_MAP_DIV:
-    #pragma unroll
-                    for (int j = 0; j < W; ++j) v.v[j] = a.v[j] / b.v[j];
-                    break;
-                case VC_MAP_NEG:
-    #pragma unroll
-                    for (int j = 0; j < W; ++j) v.v[j] = -a.v[j];
-                    break;
-                default:  // VC_MAP_STEP
-    #pragma unroll
-                    for (int j = 0; j < W; ++j) v.v[j] = a.v[j] > 0.0f ? 1.0f : 0.0f;
-                    break;
-            }
             put(r, id, v);
+            return;
+        }
+    }
+    const Vals<W> b = get(r, ib);
+    switch (op) {
+        case VC_MAP_ADD:
+#pragma unroll
+            for (int j = 0; j < W; ++j) v.v[j] = a.v[j] + b.v[j];
+            break;
+        case VC_MAP_SUB:
+#pragma unroll
+            for (int j = 0; j < W; ++j) v.v[j] = a.v[j] - b.v[j];
+            break;
+        case VC_MAP_MUL:
+#pragma unroll
+            for (int j = 0; j < W; ++j) v.v[j] = a.v[j] * b.v[j];
+            break;
+        case VC_MAP_DIV:
+#pragma unroll
+            for (int j = 0; j < W; ++j) v.v[j] = a.v[j] / b.v[j];
+            break;
+        case VC_MAP_NEG:
+#pragma unroll
+            for (int j = 0; j < W; ++j) v.v[j] = -a.v[j];
+            break;
+        default:  // VC_MAP_STEP
+#pragma unroll
+            for (int j = 0; j < W; ++j) v.v[j] = a.v[j] > 0.0f ? 1.0f : 0.0f;
+            break;
+    }
+    put(r, id, v);
 }
 
 // The program. Its words are kernel arguments: flat and plain column programs
@@ -234,15 +237,11 @@ __device__ inline void step(Regs<W>& r, const Program& P, const Place<W>& at, ui
 // gradients, 16 instructions: 116-127 us, 119 looped; rows of 8192 x 1024 to
 // mean 0 and variance 1: 229 us, 224 looped), and eight times the code.
 template <int Code, bool Matrix, int W>
-__device__ inline void run(Regs<W>& r, const Program& P, const Place<W>& at) {
+__device__ inline void run(Regs<W>& r, const Program& P, const Place<W>& at, uint32_t words = 0) {
     if constexpr (Matrix) {
-        uint32_t next = P.code[0];
 #pragma nounroll
-        for (int k = 0; k < P.n_code; ++k) {
-            const uint32_t word = next;
-            next = P.code[k + 1 < kCode ? k + 1 : 0];
-            step<Matrix>(r, P, at, word);
-        }
+        for (int k = 0; k < P.n_code; ++k)
+            step<Matrix>(r, P, at, uint32_t(__builtin_amdgcn_readlane(int(words), k)));
     } else {
 #pragma unroll
         for (int k = 0; k < Code; ++k) {
@@ -304,6 +303,53 @@ __device__ inline void load_matrix_inputs(Regs<W>& r, const Program& P, int64_t 
     for (int j = 0; j < NIn; ++j) put(r, j, v[j]);
 }
 
+// As load_matrix_inputs where every lane's values lie in one row: each input is
+// one buffer load of W values whatever its kind, so that all of them are in
+// flight together (with a branch per kind each load was waited for before the
+// next: bias, activations and their product on 4096 x 4096 with gradients 123 us, 94 now). Element e_base (the same in all
+// lanes) + e_off is the lane's first; a one-value-per-row input's load starts
+// with its value and may run past the input, where the descriptor ends it.
+// Lane offsets fit 32 bits: e_off is below 2^28, and an input that is not
+// full has fewer than 2^30 values (see vc_hip_map_broadcast).
+template <int NIn, int W>
+__device__ inline void load_row_inputs(Regs<W>& r, const Program& P, uint32_t e_base, uint32_t e_off, const Place<W>& at) {
+    Vals<W> v[NIn];
+    const uint32_t in_group = at.group[0] * P.cols + at.c[0];
+#pragma unroll
+    for (int j = 0; j < NIn; ++j) {
+        const int kind = P.kind[j];
+        const bool full = kind == VC_MAP_FULL;
+        const uint32_t rest = P.count - e_base;
+        const uint32_t extent = full ? (rest < (1u << 29) ? rest : (1u << 29)) : P.extent[j];
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float*>(P.in[j] + (full ? e_base : 0u)), short(0), int(extent * 4u), 0x00020000);
+        const uint32_t at_j = full ? e_off : kind == VC_MAP_PER_COLUMN ? at.c[0] : kind == VC_MAP_PER_ROW ? at.r[0] : in_group;
+        if constexpr (W == 4) {
+            const f4 x = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rs, at_j * 4u, 0, 0));
+#pragma unroll
+            for (int w = 0; w < 4; ++w) v[j].v[w] = x[w];
+        } else {
+            v[j].v[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, at_j * 4u, 0, 0));
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NIn; ++j) {
+#pragma unroll
+        for (int w = 1; w < W; ++w) v[j].v[w] = P.kind[j] == VC_MAP_PER_ROW ? v[j].v[0] : v[j].v[w];
+        put(r, j, v[j]);
+    }
+}
+
+// Lane k holds instruction k of a matrix program: a readlane gives a word as a
+// scalar, without a wait on the scalar cache for each.
+__device__ inline uint32_t lane_words(const Program& P) {
+    static_assert(kCode <= 64, "a wavefront holds a program");
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t word = P.code[lane < uint32_t(kCode) ? lane : 0u];
+    asm volatile("" : "+v"(word));  // loaded here, in every lane, not in a branch that some lanes do not take
+    return word;
+}
+
 template <int W>
 __device__ inline void store_outputs(const Regs<W>& r, const Program& P, int64_t e) {
 #pragma unroll
@@ -327,16 +373,21 @@ __global__ __launch_bounds__(kMapBlock) void map_flat_kernel(Program P, int64_t 
 // map_flat_kernel of a matrix program: full inputs and outputs are read and
 // written as there, whatever the columns; the other inputs by coordinates. The
 // last group of count % W values is a launch of its own from element `first`.
-template <int NIn, int W>
+// OneRow: W values never cross the end of a row (W = 1, or cols % 4 == 0).
+template <int NIn, int W, bool OneRow>
 __global__ __launch_bounds__(kMapBlock) void map_matrix_kernel(Program P, int64_t groups, int64_t first) {
     Regs<W> r;
     set_constants(r, P, NIn);
+    const uint32_t words = lane_words(P);
     const int64_t stride = int64_t(gridDim.x) * blockDim.x;
-    for (int64_t g = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; g < groups; g += stride) {
+    for (int64_t g0 = int64_t(blockIdx.x) * blockDim.x; g0 < groups; g0 += stride) {
+        const int64_t g = g0 + threadIdx.x;
+        if (g >= groups) break;
         const int64_t e = first + g * W;
         const Place<W> at = place_of<W>(P, uint32_t(e));
-        load_matrix_inputs<NIn, W>(r, P, e, at);
-        run<0, true>(r, P, at);
+        if constexpr (OneRow) load_row_inputs<NIn, W>(r, P, uint32_t(first + g0 * W), threadIdx.x * W, at);
+        else load_matrix_inputs<NIn, W>(r, P, e, at);
+        run<0, true>(r, P, at, words);
         store_outputs(r, P, e);
     }
 }
@@ -351,19 +402,24 @@ template <int NIn, int W, int Lanes>
 __global__ __launch_bounds__(kMapBlock) void map_rows_kernel(Program P, int64_t rows) {
     constexpr int kWaves = Lanes / 64;
     __shared__ double wave_part[kSums][4];
-    const int t = int(threadIdx.x) % Lanes, lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6;
+    const int t = int(threadIdx.x) % Lanes, lane = int(threadIdx.x) & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
     const uint32_t cols = P.cols;
     Regs<W> r;
     set_constants(r, P, NIn);
+    const uint32_t words = lane_words(P);
     const int64_t step = int64_t(gridDim.x) * (kMapBlock / Lanes);
-    for (int64_t row = int64_t(blockIdx.x) * (kMapBlock / Lanes) + int(threadIdx.x) / Lanes; row < rows; row += step) {
+    for (int64_t row = int64_t(blockIdx.x) * (kMapBlock / Lanes) + wave / kWaves; row < rows; row += step) {
         double acc[kSums] = {0.0, 0.0};
-        for (uint32_t c = uint32_t(t) * W; c < cols; c += Lanes * W) {
+        for (uint32_t c0 = 0; c0 < cols; c0 += Lanes * W) {
+            const uint32_t c = c0 + uint32_t(t) * W;
+            if (c >= cols) break;
             const uint32_t c1 = c + W <= cols ? c : cols - W;
+            const uint32_t before = c0 < W ? c0 : W;  // c1 may lie in the group before c0
             const int64_t e = row * cols + c1;
             const Place<W> at = place_at<W>(P, uint32_t(row), c1);
-            load_matrix_inputs<NIn, W>(r, P, e, at);
-            run<0, true>(r, P, at);
+            load_row_inputs<NIn, W>(r, P, uint32_t(row) * cols + (c0 - before), c1 - (c0 - before), at);
+            run<0, true>(r, P, at, words);
 #pragma unroll
             for (int j = 0; j < kOutputs; ++j)
                 if (j < P.n_out) store_any<W>(P.out[j] + e, get(r, P.out_slot[j]));
@@ -404,8 +460,9 @@ template <int NIn, int W, int Code, int NSum, bool Matrix>
 __global__ __launch_bounds__(kMapBlock) void map_columns_kernel(Program P, int64_t rows, int64_t cols,
                                                                 double* __restrict__ part) {
     __shared__ double wave_part[NSum][4][64 * W];
-    const int lane = int(threadIdx.x) & 63, w = int(threadIdx.x) >> 6;
+    const int lane = int(threadIdx.x) & 63, w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
     const int64_t col = (int64_t(blockIdx.x) * 64 + lane) * W;
+    const uint32_t words = Matrix ? lane_words(P) : 0;
     const int64_t step = 4 * int64_t(gridDim.y);
     Regs<W> r;
     set_constants(r, P, NIn);
@@ -419,8 +476,8 @@ __global__ __launch_bounds__(kMapBlock) void map_columns_kernel(Program P, int64
             const int64_t e = row * cols + col;
             if constexpr (Matrix) {
                 const Place<W> at = place_at<W>(P, uint32_t(row), uint32_t(col));
-                load_matrix_inputs<NIn, W>(r, P, e, at);
-                run<Code, true>(r, P, at);
+                load_row_inputs<NIn, W>(r, P, uint32_t(row) * uint32_t(cols) + blockIdx.x * 64 * W, uint32_t(lane) * W, at);
+                run<Code, true>(r, P, at, words);
             } else {
                 load_inputs<NIn, W>(r, P, e);
                 run<Code, false>(r, P, Place<W>{});
@@ -520,12 +577,14 @@ void launch_columns(Device& d, const Program& P, int64_t rows, int64_t cols, boo
 template <int NIn>
 void launch_matrix(Device& d, const Program& P, int64_t count, bool vec) {
     const int64_t groups = vec ? count / 4 : 0;
-    if (groups > 0)
-        launch(map_matrix_kernel<NIn, 4>, dim3(grid_1d(size_t(groups), kMapBlock, kFlatBlocks)), dim3(kMapBlock), 0,
-               d.stream, P, groups, int64_t(0));
+    if (groups > 0) {
+        const dim3 grid(grid_1d(size_t(groups), kMapBlock, kFlatBlocks));
+        if (P.cols % 4 == 0) launch(map_matrix_kernel<NIn, 4, true>, grid, dim3(kMapBlock), 0, d.stream, P, groups, int64_t(0));
+        else launch(map_matrix_kernel<NIn, 4, false>, grid, dim3(kMapBlock), 0, d.stream, P, groups, int64_t(0));
+    }
     if (groups * 4 < count) {
         const int64_t rest = count - groups * 4;
-        launch(map_matrix_kernel<NIn, 1>, dim3(grid_1d(size_t(rest), kMapBlock, kFlatBlocks)), dim3(kMapBlock), 0,
+        launch(map_matrix_kernel<NIn, 1, true>, dim3(grid_1d(size_t(rest), kMapBlock, kFlatBlocks)), dim3(kMapBlock), 0,
                d.stream, P, rest, groups * 4);
     }
 }
