@@ -724,6 +724,9 @@ std::optional<Broadcast> broadcast_of(const Shape& shape, const Strides& strides
 MapExpr broadcast_expr(const Storage& s, std::size_t offset, std::size_t count, const Broadcast& b) {
     if (b.kind == VC_MAP_FULL) return operand_expr(s, offset, count);
     const auto& h = as_hip(s);
+    // A host-known value (the count of a mean's quotient) is a constant: as an input it would be uploaded, and
+    // ask for a view of one row.
+    if (const auto value = h.host_scalar()) return constant_expr(*value);
     auto n = std::make_shared<MapNode>();
     n->kind = MapNode::Kind::Input;
     (void)h.ptr();
