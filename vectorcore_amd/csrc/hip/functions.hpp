@@ -11,10 +11,8 @@ struct ReluGradOp { __device__ float operator()(float x) const { return x > 0.0f
 struct SigmoidOp {
     // exp(-|x|) cannot overflow: 1 / (1 + e) from 0 up, e / (1 + e) below (src/cpu/cpu_backend.cpp:302-307),
     // without a branch whose two sides a wavefront would run one after the other.
-    __device__ float operator()(float x) const {
-        const float e = expf(-fabsf(x));
-        return (x >= 0.0f ? 1.0f : e) / (1.0f + e);
-    }
+    __device__ static float of(float x, float e) { return (x >= 0.0f ? 1.0f : e) / (1.0f + e); }  // e = exp(-|x|)
+    __device__ float operator()(float x) const { return of(x, expf(-fabsf(x))); }
 };
 struct ExpOp { __device__ float operator()(float x) const { return expf(x); } };
 struct LogOp { __device__ float operator()(float x) const { return logf(x); } };
