@@ -76,3 +76,13 @@ def test_divided_by_a_host_scalar_along_an_axis():
         y.backward(vc.Tensor(np.cos(x), device=device))
         grads.append(t.grad.numpy())
     np.testing.assert_allclose(grads[0], grads[1], rtol=2e-5, atol=2e-6)
+
+
+@pytest.mark.parametrize("count", [1, 2, 3, 4, 5, 7, 1023, 1025, 4096 * 256 * 4 + 3])
+def test_flat_programs_end_with_the_count(count):
+    """The last vector of a count that is no multiple of 4 is moved back; nothing past the count is written."""
+    x = np.random.default_rng(count).standard_normal(count).astype(np.float32)
+    a, out = C.Buffer.of(x), C.Buffer.of(np.full(count + 4, 5.0, np.float32))
+    p = C.map_program([a.ptr], [3.0], [(C.MAP_MUL, 0, 1, 2), (C.MAP_ADD, 2, 0, 3)], [(out.ptr, 3)], [], 1, count)
+    C.check(C.lib().vc_hip_map(ctypes.byref(p)))
+    np.testing.assert_array_equal(out.numpy(), np.concatenate([x * np.float32(3.0) + x, np.full(4, 5.0, np.float32)]))

@@ -14,6 +14,8 @@ namespace vchip {
 namespace fmap {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
+// 16 bytes on any 4-byte boundary (a 16-byte load or store needs no more).
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 
 constexpr int kSlots = VC_HIP_MAP_SLOTS;
@@ -118,7 +120,7 @@ template <int W>
 __device__ inline Vals<W> load(const float* __restrict__ p) {
     Vals<W> o;
     if constexpr (W == 4) {
-        const f4 x = __builtin_nontemporal_load(reinterpret_cast<const f4*>(p));
+        const f4 x = __builtin_nontemporal_load(reinterpret_cast<const f4u*>(p));
         o.v[0] = x.x;
         o.v[1] = x.y;
         o.v[2] = x.z;
@@ -130,22 +132,20 @@ __device__ inline Vals<W> load(const float* __restrict__ p) {
 }
 template <int W>
 __device__ inline void store_any(float* __restrict__ p, const Vals<W>& v) {
-    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
     if constexpr (W == 4) *reinterpret_cast<f4u*>(p) = f4{v.v[0], v.v[1], v.v[2], v.v[3]};
     else p[0] = v.v[0];
 }
 template <int W>
 __device__ inline void store(float* __restrict__ p, const Vals<W>& v) {
     if constexpr (W == 4) {
-        __builtin_nontemporal_store(f4{v.v[0], v.v[1], v.v[2], v.v[3]}, reinterpret_cast<f4*>(p));
+        __builtin_nontemporal_store(f4u{v.v[0], v.v[1], v.v[2], v.v[3]}, reinterpret_cast<f4u*>(p));
     } else {
         __builtin_nontemporal_store(v.v[0], p);
     }
 }
 
 // W consecutive values on any 4-byte boundary, through the caches (vectors
-// that every row reads; a 16-byte load needs 4-byte alignment only).
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+// that every row reads).
 template <int W>
 __device__ inline Vals<W> load_any(const float* __restrict__ p) {
     Vals<W> o;
@@ -344,35 +344,44 @@ __device__ inline void store_outputs(const Regs<W>& r, const Program& P, int64_t
         if (j < P.n_out) store<W>(P.out[j] + e, get(r, P.out_slot[j]));
 }
 
-// Elements [0, count) in groups of W: thread t takes groups t, t + threads, ...
+// The first element of group g: the last group of a count that is no multiple
+// of W ends with the count, and computes and writes what it shares with the group
+// before it once more (the same values). A launch of its own for these elements
+// cost 2.5 us and the host's part.
+template <int W>
+__device__ inline int64_t group_start(int64_t g, int64_t count) {
+    return W == 1 || (g + 1) * W <= count ? g * W : count - W;
+}
+
+// Elements [0, count) (count >= W) in groups of W: thread t takes groups t, t + threads, ...
 template <int NIn, int W, int Code>
-__global__ __launch_bounds__(kMapBlock) void map_flat_kernel(Program P, int64_t groups) {
+__global__ __launch_bounds__(kMapBlock) void map_flat_kernel(Program P, int64_t count) {
     Regs<W> r;
     set_constants(r, P, NIn);
-    const int64_t stride = int64_t(gridDim.x) * blockDim.x;
+    const int64_t stride = int64_t(gridDim.x) * blockDim.x, groups = (count + W - 1) / W;
     for (int64_t g = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; g < groups; g += stride) {
-        load_inputs<NIn, W>(r, P, g * W);
+        const int64_t e = group_start<W>(g, count);
+        load_inputs<NIn, W>(r, P, e);
         run<Code, false>(r, P, Place<W>{});
-        store_outputs(r, P, g * W);
+        store_outputs(r, P, e);
     }
 }
 
 // map_flat_kernel of a matrix program: full inputs and outputs are read and
-// written as there, whatever the columns; the other inputs by coordinates. The
-// last group of count % W values is a launch of its own from element `first`.
+// written as there, whatever the columns; the other inputs by coordinates.
 // OneRow: W values never cross the end of a row (W = 1, or cols % 4 == 0).
 template <int NIn, int W, bool OneRow>
-__global__ __launch_bounds__(kMapBlock) void map_matrix_kernel(Program P, int64_t groups, int64_t first) {
+__global__ __launch_bounds__(kMapBlock) void map_matrix_kernel(Program P, int64_t count) {
     Regs<W> r;
     set_constants(r, P, NIn);
     const uint32_t words = lane_words(P);
-    const int64_t stride = int64_t(gridDim.x) * blockDim.x;
+    const int64_t stride = int64_t(gridDim.x) * blockDim.x, groups = (count + W - 1) / W;
     for (int64_t g0 = int64_t(blockIdx.x) * blockDim.x; g0 < groups; g0 += stride) {
         const int64_t g = g0 + threadIdx.x;
         if (g >= groups) break;
-        const int64_t e = first + g * W;
+        const int64_t e = group_start<W>(g, count);
         const Place<W> at = place_of<W>(P, uint32_t(e));
-        if constexpr (OneRow) load_row_inputs<NIn, W>(r, P, uint32_t(first + g0 * W), threadIdx.x * W, at);
+        if constexpr (OneRow) load_row_inputs<NIn, W>(r, P, uint32_t(g0 * W), threadIdx.x * W, at);
         else load_matrix_inputs<NIn, W>(r, P, e, at);
         run<0, true>(r, P, at, words);
         store_outputs(r, P, e);
@@ -502,26 +511,11 @@ constexpr unsigned kFlatBlocks = 4096;
 
 template <int NIn>
 void launch_flat(Device& d, const Program& P, int64_t count, bool vec) {
-    if (vec) {
-        const int64_t groups = count / 4;
-        if (groups > 0) {
-            const dim3 grid(grid_1d(size_t(groups), kMapBlock, kFlatBlocks));
-            if (P.n_code <= kShortCode)
-                launch(map_flat_kernel<NIn, 4, kShortCode>, grid, dim3(kMapBlock), 0, d.stream, P, groups);
-            else
-                launch(map_flat_kernel<NIn, 4, kCode>, grid, dim3(kMapBlock), 0, d.stream, P, groups);
-        }
-        const int64_t done = groups * 4;
-        if (done < count) {  // the last count % 4 elements
-            Program tail = P;
-            for (int j = 0; j < NIn; ++j) tail.in[j] += done;
-            for (int j = 0; j < P.n_out; ++j) tail.out[j] += done;
-            launch(map_flat_kernel<NIn, 1, kCode>, dim3(1), dim3(kMapBlock), 0, d.stream, tail, count - done);
-        }
-    } else {
-        launch(map_flat_kernel<NIn, 1, kCode>, dim3(grid_1d(size_t(count), kMapBlock, kFlatBlocks)), dim3(kMapBlock), 0,
-               d.stream, P, count);
-    }
+    vec = vec && count >= 4;
+    const dim3 grid(grid_1d(size_t(vec ? (count + 3) / 4 : count), kMapBlock, kFlatBlocks));
+    if (!vec) launch(map_flat_kernel<NIn, 1, kCode>, grid, dim3(kMapBlock), 0, d.stream, P, count);
+    else if (P.n_code <= kShortCode) launch(map_flat_kernel<NIn, 4, kShortCode>, grid, dim3(kMapBlock), 0, d.stream, P, count);
+    else launch(map_flat_kernel<NIn, 4, kCode>, grid, dim3(kMapBlock), 0, d.stream, P, count);
 }
 
 // The column traversal's grid: about 2048 workgroups, with gy (the number of
@@ -563,17 +557,11 @@ void launch_columns(Device& d, const Program& P, int64_t rows, int64_t cols, boo
 // A matrix program without sums.
 template <int NIn>
 void launch_matrix(Device& d, const Program& P, int64_t count, bool vec) {
-    const int64_t groups = vec ? count / 4 : 0;
-    if (groups > 0) {
-        const dim3 grid(grid_1d(size_t(groups), kMapBlock, kFlatBlocks));
-        if (P.cols % 4 == 0) launch(map_matrix_kernel<NIn, 4, true>, grid, dim3(kMapBlock), 0, d.stream, P, groups, int64_t(0));
-        else launch(map_matrix_kernel<NIn, 4, false>, grid, dim3(kMapBlock), 0, d.stream, P, groups, int64_t(0));
-    }
-    if (groups * 4 < count) {
-        const int64_t rest = count - groups * 4;
-        launch(map_matrix_kernel<NIn, 1, true>, dim3(grid_1d(size_t(rest), kMapBlock, kFlatBlocks)), dim3(kMapBlock), 0,
-               d.stream, P, rest, groups * 4);
-    }
+    vec = vec && count >= 4;
+    const dim3 grid(grid_1d(size_t(vec ? (count + 3) / 4 : count), kMapBlock, kFlatBlocks));
+    if (!vec) launch(map_matrix_kernel<NIn, 1, true>, grid, dim3(kMapBlock), 0, d.stream, P, count);
+    else if (P.cols % 4 == 0) launch(map_matrix_kernel<NIn, 4, true>, grid, dim3(kMapBlock), 0, d.stream, P, count);
+    else launch(map_matrix_kernel<NIn, 4, false>, grid, dim3(kMapBlock), 0, d.stream, P, count);
 }
 
 // A matrix program with row sums: a wavefront per row, or a workgroup for few long rows.
