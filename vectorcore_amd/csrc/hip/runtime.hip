@@ -7,6 +7,7 @@
 // vc_hip_synchronize (and, rarely, when the pinned staging ring or the pool
 // needs memory back), and in vc_hip_mirror_read, which waits for one point of
 // the stream only.
+#include "half_ring.hpp"
 #include "vc_hip_internal.hpp"
 
 #include <algorithm>
@@ -179,10 +180,9 @@ public:
     static constexpr size_t kCapacity = size_t(64) << 20;
     static constexpr size_t kChunk = size_t(16) << 20;
     // Uploads of up to kSmallUpload bytes go by upload_kernel through a ring
-    // of their own, in two halves: an event marks the end of a half's use
-    // when the ring moves on to the other, and is waited for before the half
-    // is used again.
+    // of their own, in two halves (HalfRing).
     static constexpr size_t kSmallUpload = size_t(256) << 10, kSmallHalf = size_t(1) << 20;
+    static_assert(kSmallUpload <= kSmallHalf, "a small upload fits a half");
 
     void upload(void* dst, const void* src, size_t bytes) {
         Device& d = require_device();
@@ -220,22 +220,19 @@ private:
     };
 
     void small_upload(Device& d, void* dst, const void* src, size_t bytes) {
-        if (!small_) {
+        for (hipEvent_t& e : small_done_)
+            if (!e) check_hip(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+        if (!small_)
             check_hip(hipHostMalloc(reinterpret_cast<void**>(&small_), 2 * kSmallHalf, hipHostMallocDefault),
                       "hipHostMalloc (small uploads)");
-            for (hipEvent_t& e : small_done_) check_hip(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
-        }
         const size_t n = (bytes + 15) / 16 * 16;
-        if (small_head_ % kSmallHalf + n > kSmallHalf || small_head_ == 2 * kSmallHalf) {
-            const size_t half = (small_head_ - 1) / kSmallHalf;
-            check_hip(hipEventRecord(small_done_[half], d.stream), "hipEventRecord");
-            small_used_[half] = true;
-            small_head_ = (1 - half) * kSmallHalf;
-            if (small_used_[1 - half]) check_hip(hipEventSynchronize(small_done_[1 - half]), "hipEventSynchronize (staging)");
-        }
-        unsigned char* const slot = small_ + small_head_;
+        unsigned char* const slot =
+            small_ + small_ring_.take(
+                         n, [&](int half) { check_hip(hipEventRecord(small_done_[half], d.stream), "hipEventRecord"); },
+                         [&](int half) {
+                             check_hip(hipEventSynchronize(small_done_[half]), "hipEventSynchronize (staging)");
+                         });
         std::memcpy(slot, src, bytes);
-        small_head_ += n;
         launch(upload_kernel, dim3(grid_1d(n / 16, 256, 64)), dim3(256), 0, d.stream, static_cast<const unsigned char*>(slot),
                static_cast<unsigned char*>(dst), bytes);
         after_launch("upload");
@@ -270,9 +267,8 @@ private:
 
     std::mutex mu_;
     unsigned char* small_ = nullptr;
-    size_t small_head_ = 0;
+    HalfRing small_ring_{kSmallHalf};
     hipEvent_t small_done_[2] = {};
-    bool small_used_[2] = {};
     char* base_ = nullptr;
     size_t head_ = 0;
     std::deque<Segment> inflight_;
