@@ -95,3 +95,27 @@ def test_softmax_refuses_its_modified_result_and_log_softmax_does_not():
         else:
             with pytest.raises(RuntimeError, match="modified in place"):
                 y.backward(g)
+
+
+@pytest.mark.parametrize("log", [False, True])
+@pytest.mark.parametrize("shape", [(533, 16, 9), (534, 16, 9),  # on the two sides of the choice
+                                   (70_000, 2, 2), (9000, 31, 3), (4000, 5, 70), (3, 4, 90_001), (20_000, 300, 2),
+                                   (300_001, 1, 2), (1 << 23, 2, 2)])  # 2^23 workgroups of 512 could not be launched
+def test_many_short_columns(shape, log):
+    test_both_directions_against_float64(shape, 1, log)
+
+
+@pytest.mark.parametrize("log", [False, True])
+def test_special_values_in_short_columns_match_the_cpu_device(log):
+    x = np.random.default_rng(4).standard_normal((1000, 5, 6)).astype(np.float32)
+    x[0, 2, 1], x[1, 3, 2], x[2, 0, 3], x[3, 4, 4] = np.inf, -np.inf, np.nan, np.nan
+    x[4, :, 5] = -np.inf
+    x[5, :, 0] = np.finfo(np.float32).min
+    got, want = [], []
+    for out, device in ((got, "hip"), (want, "cpu")):
+        t = vc.Tensor(x, requires_grad=True, device=device)
+        y = t.log_softmax(1) if log else t.softmax(1)
+        y.backward(vc.Tensor(np.ones(x.shape, np.float32), device=device))
+        out += [y.numpy(), t.grad.numpy()]
+    for a, b in zip(got, want):
+        np.testing.assert_allclose(a, b, rtol=1e-5, atol=2e-6)

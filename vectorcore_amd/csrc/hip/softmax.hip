@@ -13,7 +13,6 @@
 #include "vc_hip_internal.hpp"
 
 #include <algorithm>
-#include <limits>
 #include <string>
 
 namespace vchip {
@@ -306,9 +305,53 @@ __global__ __launch_bounds__(kCols * kRowLanes) void cols_backward_kernel(const 
     });
 }
 
+// inner > 1, many columns of few elements: a thread per column, which walks
+// the axis in order (the later walks find it in the caches).
+template <bool Log>
+__global__ __launch_bounds__(kRowBlock) void thin_forward_kernel(const float* __restrict__ x, float* __restrict__ y,
+                                                                 float* __restrict__ stats, int64_t outer, int64_t len,
+                                                                 int64_t inner) {
+    const int64_t total = outer * inner, stride = int64_t(gridDim.x) * kRowBlock;
+    for (int64_t t = int64_t(blockIdx.x) * kRowBlock + threadIdx.x; t < total; t += stride) {
+        const int64_t o = t / inner, base = o * len * inner + (t - o * inner);
+        float m = x[base];  // a NaN first element stays
+#pragma unroll 4
+        for (int64_t a = 1; a < len; ++a) m = x[base + a * inner] > m ? x[base + a * inner] : m;
+        double sum = 0.0;
+#pragma unroll 4
+        for (int64_t a = 0; a < len; ++a) sum += double(expf(x[base + a * inner] - m));
+        const float s = float(sum), l = logf(s);
+#pragma unroll 4
+        for (int64_t a = 0; a < len; ++a) y[base + a * inner] = result<Log>(x[base + a * inner], m, l);
+        if (stats) {
+            stats[2 * t] = m;
+            stats[2 * t + 1] = s;
+        }
+    }
+}
+
+template <bool Log>
+__global__ __launch_bounds__(kRowBlock) void thin_backward_kernel(const float* __restrict__ g, const float* __restrict__ x,
+                                                                  const float* __restrict__ stats, float* __restrict__ dx,
+                                                                  int64_t outer, int64_t len, int64_t inner) {
+    const int64_t total = outer * inner, stride = int64_t(gridDim.x) * kRowBlock;
+    for (int64_t t = int64_t(blockIdx.x) * kRowBlock + threadIdx.x; t < total; t += stride) {
+        const int64_t o = t / inner, base = o * len * inner + (t - o * inner);
+        const float m = stats[2 * t], s = stats[2 * t + 1], l = logf(s);
+        double sum = 0.0;
+#pragma unroll 4
+        for (int64_t a = 0; a < len; ++a) sum += double(through_exp<Log>(g[base + a * inner], x[base + a * inner], m, l));
+        const float ds = -float(sum) / s + 0.0f;
+#pragma unroll 4
+        for (int64_t a = 0; a < len; ++a)
+            dx[base + a * inner] = through_exp<Log>(g[base + a * inner], x[base + a * inner], m, l) +
+                                   ds * expf(x[base + a * inner] - m);
+    }
+}
+
 // The launch of a row or column kernel for [outer, len, inner].
-template <class Rows, class Long, class Cols>
-void dispatch(Device& d, int64_t outer, int64_t len, int64_t inner, Rows rows, Long longer, Cols cols) {
+template <class Rows, class Long, class Cols, class Thin>
+void dispatch(Device& d, int64_t outer, int64_t len, int64_t inner, Rows rows, Long longer, Cols cols, Thin thin) {
     if (inner == 1) {
         const unsigned grid = unsigned(std::min<int64_t>((outer + 3) / 4, int64_t(d.cu_count) * 64));
         const int64_t nv = (len + 255) / 256;
@@ -319,9 +362,15 @@ void dispatch(Device& d, int64_t outer, int64_t len, int64_t inner, Rows rows, L
         else longer(unsigned(std::min<int64_t>(outer, int64_t(d.cu_count) * 16)));
         return;
     }
-    const int64_t per_outer = (inner + kCols - 1) / kCols;
-    if (outer * per_outer > std::numeric_limits<int>::max()) fail(VC_HIP_ERR_OVERFLOW, "softmax too large");
-    cols(unsigned(outer * per_outer), per_outer);
+    const int64_t per_outer = (inner + kCols - 1) / kCols, groups = outer * per_outer, total = outer * inner;
+    // A workgroup per 16 columns costs about 3 ns per 256 rows once the chip is full, a thread per column 0.1 us per
+    // row for as many columns as the chip holds (512 x 128 x 16, both directions: 13 against 67 us; 4096 x 64 x 16: 70
+    // against 47; 100000 x 16 x 2: 856 against 80; composed 132). The first is thus chosen for fewer than 8600
+    // workgroups only.
+    if (0.003 * double(groups) * double((len + 255) / 256) <= 0.1 * double(len) * std::max(1.0, double(total) / 262144.0))
+        cols(unsigned(groups), per_outer);
+    else
+        thin(grid_1d(size_t(total), kRowBlock, unsigned(d.cu_count) * 64));
 }
 
 }  // namespace
@@ -354,6 +403,9 @@ int vc_hip_softmax_forward(const float* in, float* out, float* stats, size_t out
                 [&](unsigned grid, int64_t per_outer) {
                     launch(cols_forward_kernel<Log>, dim3(grid), dim3(kCols * kRowLanes), 0, d.stream, in, out, stats, len,
                            n, per_outer);
+                },
+                [&](unsigned grid) {
+                    launch(thin_forward_kernel<Log>, dim3(grid), dim3(kRowBlock), 0, d.stream, in, out, stats, o, len, n);
                 });
         };
         if (log_output) launch_all(std::true_type{});
@@ -386,6 +438,10 @@ int vc_hip_softmax_backward(const float* grad, const float* in, const float* sta
                 [&](unsigned grid, int64_t per_outer) {
                     launch(cols_backward_kernel<Log>, dim3(grid), dim3(kCols * kRowLanes), 0, d.stream, grad, in, stats,
                            out, len, n, per_outer);
+                },
+                [&](unsigned grid) {
+                    launch(thin_backward_kernel<Log>, dim3(grid), dim3(kRowBlock), 0, d.stream, grad, in, stats, out, o,
+                           len, n);
                 });
         };
         if (log_output) launch_all(std::true_type{});
