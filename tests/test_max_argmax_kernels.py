@@ -48,3 +48,10 @@ def test_an_empty_axis_and_null_outputs_are_refused():
         C.check(C.lib().vc_hip_reduce_axis_max_argmax(x.ptr, x.ptr, x.ptr, 2, 0, 2))
     with pytest.raises(ValueError):
         C.check(C.lib().vc_hip_reduce_axis_max_argmax(x.ptr, x.ptr, None, 1, 2, 2))
+
+
+@pytest.mark.parametrize("shape", [(5000, 16, 2), (30_000, 17, 3), (100_000, 16, 16), (16, 16, 8000), (4096, 24, 100),
+                                   (10_000, 64, 2), (20_000, 100, 2), (1024, 63, 63), (4096, 63, 63), (2000, 197, 8)])
+def test_short_and_narrow_columns_match_the_scan(shape):
+    """Shapes about where a workgroup of row lanes, a thread per column and a split axis take over from each other."""
+    test_both_reductions_match_the_scan(shape)

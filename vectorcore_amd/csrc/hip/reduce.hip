@@ -677,20 +677,36 @@ private:
     std::vector<std::unique_ptr<Scratch>> held_;
 };
 
-// Whether a max/argmax over columns takes cols_best_kernel: an axis worth its
-// 16 row lanes, and enough workgroups for the chip or an axis that a few read
-// quickly (longer ones are split over workgroups).
+// Whether a max/argmax over columns takes cols_best_kernel rather than a thread
+// per column or, with few columns and an axis of 64 or more, a split axis: by
+// what each costs in us, fitted to 494 shapes of 32 KiB to 1.6 GB. A workgroup
+// costs 1.1 ns (2.6 with 64 columns) for its first 128 rows and half that for
+// each further 128, a thread per column 0.09 us a row, a split 0.48 us a
+// segment, and each path reads at the rate that stands there. Shapes on the
+// two sides, there against here: 100000 x 16 x 16 22 against 105, 16 x 16 x
+// 8000 3.4 against 8.2, 2000 x 197 x 8 14 against 6.4, 512 x 197 x 768 106
+// against 52. A launch holds fewer than 2^32 threads.
 int64_t best_chunks(int64_t inner) { return (inner + (inner >= 64 ? 63 : 15)) / (inner >= 64 ? 64 : 16); }
-bool best_in_one(int64_t outer, int64_t len, int64_t inner) {
-    const int64_t blocks = outer * best_chunks(inner);
-    return len >= 16 && blocks <= std::numeric_limits<int>::max() && (blocks >= 128 || len <= 1024);
+bool best_few(int64_t blocks, int64_t len, int cu_count) { return blocks < 2 * int64_t(cu_count) && len > 64; }
+bool best_in_one(int64_t outer, int64_t len, int64_t inner, int cu_count, int64_t target_threads) {
+    const int64_t blocks = outer * best_chunks(inner), total = outer * inner;
+    if (len < 16 || blocks >= (int64_t(1) << 24) || (blocks < 128 && len > 1024)) return false;
+    const double bytes = 4.0 * double(outer) * double(len) * double(inner), rows = double(len);
+    const bool wide = inner >= 64;
+    const double least = best_few(blocks, len, cu_count) ? (wide ? 5.5 : 8.0) : 3.5;
+    const double issue = 3.0 + (wide ? 0.0026 : 0.0011) * double(blocks) * double((len + 127) / 128 + 1) / 2.0;
+    const double here = std::max({least, issue, 2.0 + bytes / (wide ? 5.5e6 : inner % 16 == 0 || inner < 16 ? 5e6 : 2.5e6)});
+    const bool split = len >= 64 && total < target_threads;
+    const double there = split ? 4.0 + 0.48 * double(best_plan(len, total, target_threads).segs) + bytes / 4e6
+                               : 0.7 + 0.09 * rows + bytes / (len < 64 ? 6e6 : inner < 16 ? 1.5e6 : 4e6);
+    return here < there;
 }
 
 template <int Op>
 void launch_cols_best(Device& d, const float* in, float* out, float* out2, int64_t outer, int64_t len, int64_t inner) {
     const int64_t chunks = best_chunks(inner);
     const dim3 grid{unsigned(outer * chunks)};
-    const bool few = outer * chunks < 2 * int64_t(d.cu_count) && len > 64;  // more row lanes for fewer workgroups
+    const bool few = best_few(outer * chunks, len, d.cu_count);  // more row lanes for fewer workgroups
     if (inner >= 64 && few)
         launch(cols_best_kernel<Op, 4, 32>, grid, dim3(512), 0, d.stream, in, out, out2, len, inner, chunks);
     else if (inner >= 64)
@@ -743,7 +759,7 @@ void reduce_axis(const float* in, float* out, int64_t outer, int64_t len, int64_
         p.done();
         return;
     }
-    if (op != VC_REDUCE_SUM && best_in_one(outer, len, inner)) {
+    if (op != VC_REDUCE_SUM && best_in_one(outer, len, inner, d.cu_count, target_threads)) {
         // No partial results; the allocation-free entry point's limit is one of shapes, and stays.
         if (total < target_threads && len >= 64)
             memory.require(size_t(best_plan(len, total, target_threads).segs * total) * (sizeof(float) + sizeof(int)));
