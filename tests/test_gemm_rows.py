@@ -119,3 +119,19 @@ def test_split_products_keep_their_epilogues(m, k, n):
         words[r // 32] |= (mask[r] > 0).astype(np.uint32) << np.uint32(r % 32)
     C.check(C.lib().vc_hip_matmul_relu_bits(pa, pb, c.ptr, m, k, n, 0, 0, C.Buffer.of(words, dtype=np.uint32).ptr))
     np.testing.assert_array_equal(c.numpy(), masked)
+
+
+@pytest.mark.parametrize("count,m,k,n", [(32, 768, 768, 768), (64, 512, 512, 512), (16, 1024, 512, 1024)])
+def test_reductions_of_many_outputs_take_the_large_tiles(count, m, k, n):
+    """A sum over many products is as much work as one product of count k: the 128 x 128 tiles, split over the
+    products, add in another order than the 32 x 32 tiles, so their bits tell which kernel ran."""
+    rng = np.random.default_rng(count)
+    a = C.Buffer.of(rng.standard_normal((count, k, m)).astype(np.float32))
+    b = C.Buffer.of(rng.standard_normal((count, k, n)).astype(np.float32))
+    c = C.Buffer((m, n))
+    results = []
+    for kernel in ("mfma", "mfma128"):
+        with C.gemm_kernel(kernel):
+            C.check(C.lib().vc_hip_matmul_reduce(a.ptr, b.ptr, c.ptr, m, k, n, count, k * m, k * n, 1, 0))
+        results.append(c.numpy())
+    np.testing.assert_array_equal(*results)

@@ -1582,6 +1582,13 @@ double big_cost(int64_t tiles, int64_t splits, double k, int cu_count, int width
     return rounds * (width == 256 ? 226.0 * k / double(splits) + 27.0 : 124.0 * k / double(splits) + 12.0);
 }
 
+// The products of a batch reduction that one split of `tiles` output tiles
+// adds, when the chip has `slots` workgroup slots.
+int64_t reduce_range(int64_t reduce, int64_t tiles, int64_t slots) {
+    const int64_t ranges = std::min((slots + tiles - 1) / tiles, reduce);
+    return (reduce + ranges - 1) / ranges;
+}
+
 // The tile width of gemm_big_kernel (256 or 128 columns of 256 rows) for a
 // product under the automatic setting, or 0 for the other kernels, from
 // measurements on MI355X against the 128 x 128 tiles:
@@ -1642,7 +1649,8 @@ Route choose_route(int mode, int64_t M, int64_t N, int64_t K, int64_t batch, int
     };
     const bool small_fits = reduce * ((K + kSmallDepth - 1) / kSmallDepth) <= std::numeric_limits<int>::max();
     const double k = double(K) / 1024.0;
-    const double small = small_cost((M + kSmallTile - 1) / kSmallTile * ((N + kSmallTile - 1) / kSmallTile) * batch, k);
+    const double small =
+        small_cost((M + kSmallTile - 1) / kSmallTile * ((N + kSmallTile - 1) / kSmallTile) * batch, k * double(reduce));
     // The larger tiles' estimates count the splits of a long K that gemm() gives them.
     const auto big = [&](int width) {
         const int64_t n = (M + BT - 1) / BT * ((N + width - 1) / width) * batch;
@@ -1650,6 +1658,10 @@ Route choose_route(int mode, int64_t M, int64_t N, int64_t K, int64_t batch, int
     };
     const auto tiles128 = [&] {
         const int64_t n = (M + BM - 1) / BM * ((N + BN - 1) / BN) * batch, slots = 2 * int64_t(cu_count);
+        if (reduce > 1) {  // ranges of the products
+            const int64_t each = reduce_range(reduce, n, slots), splits = (reduce + each - 1) / each;
+            return tiles128_cost(n, splits, k * double(each * splits), cu_count);
+        }
         const int64_t splits = n >= slots || K < 64 * BK ? 1 : std::min<int64_t>({4, (slots + n - 1) / n, K / (32 * BK)});
         return tiles128_cost(n, splits, k, cu_count);
     };
@@ -1782,7 +1794,7 @@ void gemm(const float* a, const float* b, float* c, int64_t M, int64_t N, int64_
     const int64_t want = (slots + tiles * batch - 1) / (tiles * batch);
     if (!simple && !small && tiles * batch < slots) {
         if (reduce > 1) {
-            r_per_split = (reduce + std::min(want, reduce) - 1) / std::min(want, reduce);
+            r_per_split = reduce_range(reduce, tiles * batch, slots);
             splits = int((reduce + r_per_split - 1) / r_per_split);
         } else if (tiles * batch <= kTinyTiles && kt_total >= 4) {
             // A handful of output tiles: one workgroup's K loop is a chain of
