@@ -135,3 +135,18 @@ def test_reductions_of_many_outputs_take_the_large_tiles(count, m, k, n):
             C.check(C.lib().vc_hip_matmul_reduce(a.ptr, b.ptr, c.ptr, m, k, n, count, k * m, k * n, 1, 0))
         results.append(c.numpy())
     np.testing.assert_array_equal(*results)
+
+
+@pytest.mark.parametrize("batch,m,k,n,tb", [(2, 1544, 36, 1160, 1), (8, 12960, 12, 48, 0), (1, 512, 48, 4736, 0)])
+def test_short_k_of_many_outputs_takes_the_large_tiles(batch, m, k, n, tb):
+    """About one round of 128 x 128 tiles and a K of one or two chunks: the small tiles' fixed cost decides."""
+    a, b, want, magnitude = operands(m, k, n, 0, tb, batch, k)
+    a, b, c = C.Buffer.of(a), C.Buffer.of(b), C.Buffer((batch, m, n))
+    za, zb = C.sizes([m * k * z for z in range(batch)]), C.sizes([k * n * z for z in range(batch)])
+    results = []
+    for kernel in ("mfma", "mfma128"):
+        with C.gemm_kernel(kernel):
+            C.check(C.lib().vc_hip_matmul(a.ptr, b.ptr, c.ptr, m, k, n, za, zb, batch, 0, tb))
+        results.append(c.numpy())
+    np.testing.assert_array_equal(*results)
+    check(results[0], want, magnitude, k, (batch, m, k, n))

@@ -1568,10 +1568,11 @@ const char* variant_label(bool ta, bool tb) {
 // - 128 x 128: 120 k + 10 for two per CU (6000 x 1000 x 1000: 125-130; 3000^3,
 //   two rounds: 670), 70 k + 7 for one per CU (2048 x 1024 x 2048: 69-75),
 //   10 to add the partial products of a split K;
-// - the 32 x 32 tiles are small enough to count by area: 0.34 k + 0.05 for each
+// - the 32 x 32 tiles are small enough to count by area: 0.34 k + 0.065 for each
 //   128 x 128 outputs (3000^3: 516; 2500 x 1500 x 1700: 140, against 185 on the
-//   128 x 128 tiles; 8191 x 257 x 1023: 70, against 47 on the 256 x 128).
-double small_cost(int64_t tiles32, double k) { return double(tiles32) / 16.0 * (0.34 * k + 0.05); }
+//   128 x 128 tiles; 8191 x 257 x 1023: 70, against 47 on the 256 x 128; 2 x
+//   1544 x 36 x 1160: 20, against 15 on the 128 x 128).
+double small_cost(int64_t tiles32, double k) { return double(tiles32) / 16.0 * (0.34 * k + 0.065); }
 double tiles128_cost(int64_t tiles, int64_t splits, double k, int cu_count) {
     const int64_t n = tiles * splits, rounds = (n + 2 * cu_count - 1) / (2 * cu_count);
     const double each = k / double(splits);
