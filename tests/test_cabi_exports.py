@@ -91,3 +91,18 @@ def test_a_c_program_compiles_and_links_against_the_header(tmp_path):
                         str(src), "-o", str(out), "-L", str(lib.parent), "-lvc_hip", f"-Wl,-rpath,{lib.parent}"],
                        capture_output=True, text=True)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("call", [
+    lambda lib, p, m: lib.vc_hip_reduce_sum_published(p, 4, p, m),
+    lambda lib, p, m: lib.vc_hip_binary_scalar_published(p, 1.0, 0, p, C.ADD, m),
+    lambda lib, p, m: lib.vc_hip_xent_forward_published(p, p, 1, 4, p, p, m),
+    lambda lib, p, m: lib.vc_hip_xent_forward_argmax(p, p, 1, 4, p, p, p, m),
+    lambda lib, p, m: lib.vc_hip_reduce_axis_max_argmax(p, p, p, 1, 4, 1),
+    lambda lib, p, m: lib.vc_hip_softmax_forward(p, p, p, 1, 4, 1, 0),
+    lambda lib, p, m: lib.vc_hip_softmax_backward(p, p, p, p, 1, 4, 1, 0)])
+def test_published_and_softmax_entry_points_report_an_unavailable_device(call):
+    if C.available():
+        pytest.skip("a GPU is present: the pointers below are the host's")
+    values, mirror = (ctypes.c_float * 8)(), ctypes.c_void_p()
+    assert call(C.lib(), ctypes.addressof(values), ctypes.byref(mirror)) == 5  # VC_HIP_ERR_UNAVAILABLE

@@ -194,6 +194,7 @@ template <typename F>
 void with_mirror(vc_hip_mirror** mirror, const char* name, F&& forward) {
     if (!mirror) fail(VC_HIP_ERR_INVALID_ARGUMENT, std::string(name) + ": null mirror");
     *mirror = nullptr;
+    require_device();  // before the mirrors' first host memory
     vc_hip_mirror* m = take_mirror();
     try {
         forward(m);
