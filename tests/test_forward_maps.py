@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import vectorcore_amd as vc
+from vectorcore_amd import cabi as C
 
 pytestmark = pytest.mark.gpu
 
@@ -103,3 +104,23 @@ def test_shapes_and_no_backward(shape, fused):
     np.testing.assert_array_equal((t * t).max(0).numpy(), (x * x).max(0))
     with np.errstate(all="ignore"):
         np.testing.assert_allclose(t.log().numpy(), np.log(x), rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("rows,cols,recorded", [(16_384, 3, True), (16_385, 3, False), (20_000, 127, False),
+                                                (20_000, 128, True)])
+def test_many_short_rows_are_summed_by_the_reduction(rows, cols, recorded):
+    x = RNG.standard_normal((rows, cols)).astype(np.float32)
+    w = RNG.standard_normal((rows, 1)).astype(np.float32)
+    t, tw = (vc.Tensor(v, requires_grad=True, device="hip") for v in (x, w))
+    C.profile(True)
+    C.profile_reset()
+    try:
+        s = (t * tw).sum(1)  # the row sum of a forward expression, and of a gradient (w's)
+        s.backward(vc.Tensor(np.ones(rows, np.float32), device="hip"))
+        got = s.numpy(), tw.grad.numpy(), t.grad.numpy()
+        assert ("fused_map_rows" in C.profile_read()) == recorded
+    finally:
+        C.profile(False)
+    np.testing.assert_allclose(got[0], (x * w).astype(np.float64).sum(1), rtol=2e-7, atol=1e-9)
+    np.testing.assert_allclose(got[1], x.astype(np.float64).sum(1, keepdims=True), rtol=2e-7, atol=1e-9)
+    np.testing.assert_array_equal(got[2], np.broadcast_to(w, x.shape))
