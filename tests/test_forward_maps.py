@@ -95,6 +95,24 @@ def test_a_chain_longer_than_a_program(fused):
     np.testing.assert_allclose(x.grad.numpy(), cx.grad.numpy(), rtol=1e-3, atol=1e-7)
 
 
+@pytest.mark.parametrize("length", [15, 16, 17, 33])
+def test_chains_about_the_longest_recorded_one(length):
+    """The next operation's operand is computed then; every result and gradient has the eager ops' bits."""
+    outcomes = []
+    for fuse in (True, False):
+        before = vc.hip_fuse_elementwise(fuse)
+        x = vc.Tensor(X, requires_grad=True, device="hip")
+        y, results = x, []
+        for k in range(length):
+            y = (y * 1.25, y.sigmoid(), y - 0.5, y.relu(), y * y)[k % 5] if k % 3 else y * y + y * 0.5
+            results.append(y)
+        y.backward(vc.Tensor(DY, device="hip"))
+        outcomes.append([r.numpy() for r in results[::4]] + [y.numpy(), x.grad.numpy()])
+        vc.hip_fuse_elementwise(before)
+    for a, b in zip(*outcomes):
+        np.testing.assert_array_equal(a, b)
+
+
 @pytest.mark.parametrize("shape", [(1,), (3,), (2, 1), (1, 5), (2, 3, 4), (1025,)])
 def test_shapes_and_no_backward(shape, fused):
     x = RNG.standard_normal(shape).astype(np.float32)
