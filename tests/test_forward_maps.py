@@ -132,6 +132,7 @@ def test_many_short_rows_are_summed_by_the_reduction(rows, cols, recorded):
     x = RNG.standard_normal((rows, cols)).astype(np.float32)
     w = RNG.standard_normal((rows, 1)).astype(np.float32)
     t, tw = (vc.Tensor(v, requires_grad=True, device="hip") for v in (x, w))
+    fuse = vc.hip_fuse_elementwise(True)
     C.profile(True)
     C.profile_reset()
     try:
@@ -141,6 +142,7 @@ def test_many_short_rows_are_summed_by_the_reduction(rows, cols, recorded):
         assert ("fused_map_rows" in C.profile_read()) == recorded
     finally:
         C.profile(False)
+        vc.hip_fuse_elementwise(fuse)
     np.testing.assert_allclose(got[0], (x * w).astype(np.float64).sum(1), rtol=2e-7, atol=1e-9)
     np.testing.assert_allclose(got[1], x.astype(np.float64).sum(1, keepdims=True), rtol=2e-7, atol=1e-9)
     np.testing.assert_array_equal(got[2], np.broadcast_to(w, x.shape))

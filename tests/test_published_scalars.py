@@ -3,6 +3,7 @@ computed: the value and the bits of the unpublished entry points, and item()
 on a mean returning before the work enqueued after it has drained."""
 
 import ctypes
+import os
 
 import numpy as np
 import pytest
@@ -44,6 +45,8 @@ def test_published_sums_and_quotients(n, profiled):
     assert C.lib().vc_hip_binary_scalar_published(data.ptr, 1.0, 0, out.ptr, 9, ctypes.byref(mirror)) == 1
 
 
+@pytest.mark.skipif(os.environ.get("VECTORCORE_HIP_SYNC_EACH") == "1",
+                    reason="every launch is waited for in this mode")
 def test_a_means_value_does_not_wait_for_later_work():
     x = np.random.default_rng(0).standard_normal((1 << 20,)).astype(np.float32)
     t, a = vc.Tensor(x, device="hip"), vc.Tensor(np.ones((2048, 2048), np.float32), device="hip")
