@@ -159,10 +159,49 @@ __device__ inline Vals<W> load_any(const float* __restrict__ p) {
     return o;
 }
 
-// One instruction on the W values of every slot. `at`: their coordinates
-// (matrix programs).
-template <bool Matrix, int W>
-__device__ inline void step(Regs<W>& r, const Program& P, const Place<W>& at, uint32_t word) {
+// One instruction on the W values of every slot, for programs whose words are
+// unrolled into scalars: what a word decides has to stay in scalar registers
+// from one element to the next, so nothing but its operation and slots is
+// derived from it. (matrix_step's order and signs spilled 193 scalar registers
+// to vector lanes here, 35 this way: two inputs and 20 instructions on 4096 x
+// 4096 88 us against 72.)
+template <int W>
+__device__ inline void plain_step(Regs<W>& r, uint32_t word) {
+    const int op = int(word & 255u), ia = int((word >> 8) & 255u), ib = int((word >> 16) & 255u), id = int(word >> 24);
+    const Vals<W> a = get(r, ia), b = get(r, ib);
+    Vals<W> v;
+    switch (op) {
+        case VC_MAP_ADD:
+#pragma unroll
+            for (int j = 0; j < W; ++j) v.v[j] = a.v[j] + b.v[j];
+            break;
+        case VC_MAP_SUB:
+#pragma unroll
+            for (int j = 0; j < W; ++j) v.v[j] = a.v[j] - b.v[j];
+            break;
+        case VC_MAP_MUL:
+#pragma unroll
+            for (int j = 0; j < W; ++j) v.v[j] = a.v[j] * b.v[j];
+            break;
+        case VC_MAP_DIV:
+#pragma unroll
+            for (int j = 0; j < W; ++j) v.v[j] = a.v[j] / b.v[j];
+            break;
+        case VC_MAP_NEG:
+#pragma unroll
+            for (int j = 0; j < W; ++j) v.v[j] = -a.v[j];
+            break;
+        default:  // VC_MAP_STEP
+#pragma unroll
+            for (int j = 0; j < W; ++j) v.v[j] = a.v[j] > 0.0f ? 1.0f : 0.0f;
+            break;
+    }
+    put(r, id, v);
+}
+
+// As plain_step for matrix programs. `at`: the coordinates of the W values.
+template <int W>
+__device__ inline void matrix_step(Regs<W>& r, const Program& P, const Place<W>& at, uint32_t word) {
     const int op = int(word & 255u), ia = int((word >> 8) & 255u), ib = int((word >> 16) & 255u), id = int(word >> 24);
     const Vals<W> a = get(r, ia);
     Vals<W> v;
@@ -189,29 +228,27 @@ __device__ inline void step(Regs<W>& r, const Program& P, const Place<W>& at, ui
 #pragma unroll
             for (int j = 0; j < W; ++j) v.v[j] = op == VC_MAP_NEG ? -a.v[j] : a.v[j] > 0.0f ? 1.0f : 0.0f;
         }
-    } else if constexpr (Matrix) {
-        if (op <= VC_MAP_AT_COLUMN) {
-            const Vals<W> b = get(r, ib);
+    } else if (op <= VC_MAP_AT_COLUMN) {
+        const Vals<W> b = get(r, ib);
 #pragma unroll
-            for (int j = 0; j < W; ++j) {
-                const uint32_t axis = op == VC_MAP_AT_ROW ? at.in_group[j] : at.c[j];
-                const uint32_t keep = int(a.v[j]) == int(axis) ? ~0u : 0u;
-                v.v[j] = __uint_as_float(__float_as_uint(b.v[j]) & keep);
-            }
-        } else if (op == VC_MAP_RELU) {
-#pragma unroll
-            for (int j = 0; j < W; ++j) v.v[j] = ReluOp()(a.v[j]);
-        } else if (op == VC_MAP_LOG) {
-#pragma unroll
-            for (int j = 0; j < W; ++j) v.v[j] = LogOp()(a.v[j]);
-        } else {  // VC_MAP_SIGMOID or VC_MAP_EXP, on one exponential
-            const bool sigmoid = op == VC_MAP_SIGMOID;
-#pragma unroll
-            for (int j = 0; j < W; ++j) v.v[j] = ExpOp()(sigmoid ? -fabsf(a.v[j]) : a.v[j]);
-            if (sigmoid)
-#pragma unroll
-                for (int j = 0; j < W; ++j) v.v[j] = SigmoidOp::of(a.v[j], v.v[j]);
+        for (int j = 0; j < W; ++j) {
+            const uint32_t axis = op == VC_MAP_AT_ROW ? at.in_group[j] : at.c[j];
+            const uint32_t keep = int(a.v[j]) == int(axis) ? ~0u : 0u;
+            v.v[j] = __uint_as_float(__float_as_uint(b.v[j]) & keep);
         }
+    } else if (op == VC_MAP_RELU) {
+#pragma unroll
+        for (int j = 0; j < W; ++j) v.v[j] = ReluOp()(a.v[j]);
+    } else if (op == VC_MAP_LOG) {
+#pragma unroll
+        for (int j = 0; j < W; ++j) v.v[j] = LogOp()(a.v[j]);
+    } else {  // VC_MAP_SIGMOID or VC_MAP_EXP, on one exponential
+        const bool sigmoid = op == VC_MAP_SIGMOID;
+#pragma unroll
+        for (int j = 0; j < W; ++j) v.v[j] = ExpOp()(sigmoid ? -fabsf(a.v[j]) : a.v[j]);
+        if (sigmoid)
+#pragma unroll
+            for (int j = 0; j < W; ++j) v.v[j] = SigmoidOp::of(a.v[j], v.v[j]);
     }
     put(r, id, v);
 }
@@ -228,12 +265,12 @@ __device__ inline void run(Regs<W>& r, const Program& P, const Place<W>& at, uin
     if constexpr (Matrix) {
 #pragma nounroll
         for (int k = 0; k < P.n_code; ++k)
-            step<Matrix>(r, P, at, uint32_t(__builtin_amdgcn_readlane(int(words), k)));
+            matrix_step(r, P, at, uint32_t(__builtin_amdgcn_readlane(int(words), k)));
     } else {
 #pragma unroll
         for (int k = 0; k < Code; ++k) {
             if (k >= P.n_code) continue;  // uniform: the rest of the loop is skipped
-            step<Matrix>(r, P, at, P.code[k]);
+            plain_step(r, P.code[k]);
         }
     }
 }
@@ -350,7 +387,7 @@ __device__ inline void store_outputs(const Regs<W>& r, const Program& P, int64_t
 // cost 2.5 us and the host's part.
 template <int W>
 __device__ inline int64_t group_start(int64_t g, int64_t count) {
-    return W == 1 || (g + 1) * W <= count ? g * W : count - W;
+    return W == 1 || g * W < count - W ? g * W : count - W;
 }
 
 // Elements [0, count) (count >= W) in groups of W: thread t takes groups t, t + threads, ...
@@ -456,7 +493,8 @@ template <int NIn, int W, int Code, int NSum, bool Matrix>
 __global__ __launch_bounds__(kMapBlock) void map_columns_kernel(Program P, int64_t rows, int64_t cols,
                                                                 double* __restrict__ part) {
     __shared__ double wave_part[NSum][4][64 * W];
-    const int lane = int(threadIdx.x) & 63, w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+    const int lane = int(threadIdx.x) & 63;
+    const int w = Matrix ? __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6) : int(threadIdx.x) >> 6;
     const int64_t col = (int64_t(blockIdx.x) * 64 + lane) * W;
     const uint32_t words = Matrix ? lane_words(P) : 0;
     const int64_t step = 4 * int64_t(gridDim.y);
