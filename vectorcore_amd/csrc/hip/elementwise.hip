@@ -385,7 +385,12 @@ void launch_binary(const float* a, const float* b, float* y, size_t n, const Bca
                          (m.b_stride[1] == 0 || (aligned16(b) && m.b_stride[0] % 4 == 0));
         const unsigned grid = static_cast<unsigned>(std::min<int64_t>(rows, int64_t(d.cu_count) * 16));
         Profiled p(label, 0.0, 8.0 * double(n));
-        if (vec && stream_stores(8.0 * double(n)))
+        // Through the caches only where the next pass gains by it (see stream_stores: from 2^22 elements on) and
+        // this one loses nothing: 300 x 20000 plus a row 8.7 us streamed, 9.8 through the caches, 5000 x 1024 4.8
+        // and 6.3, 32 x 100000 21.9 and 24.4, 100000 x 32 14.6 and 15.4; 4096 x 4096 19.9 either way.
+        const double moved = 8.0 * double(n);
+        const bool stream = stream_stores(moved) || moved < 64e6 || rows < d.cu_count || cols < 1024;
+        if (vec && stream)
             launch((bcast2_kernel<Op, true, true>), dim3(grid), dim3(kBlock), 0, d.stream, a, b, y, rows, cols,
                    m.a_stride[0], m.a_stride[1], m.b_stride[0], m.b_stride[1]);
         else if (vec)
