@@ -292,7 +292,11 @@ int vc_hip_map_broadcast(const vc_hip_map_program* program, const vc_hip_map_mat
 /* ---- matrix multiply ------------------------------------------------------- */
 /* MetalBackend::matmul (metal_backend.hpp:34-40): for z < batch,
  * c[z*m*n ...] = op(a + a_offsets[z]) @ op(b + b_offsets[z]); op transposes
- * when trans_* is set (a stored k x m, b stored n x k), read in place. */
+ * when trans_* is set (a stored k x m, b stored n x k), read in place. Products
+ * of few tiles split K and find the workgroup that finishes last with counters
+ * that the library holds: like the one-launch reductions, two of them must not
+ * run at the same time on one GPU (a recorded graph replayed alongside the
+ * library's stream). */
 int vc_hip_matmul(const float* a, const float* b, float* c, size_t m, size_t k, size_t n,
                   const size_t* a_offsets, const size_t* b_offsets, size_t batch, int trans_a, int trans_b);
 /* vc_hip_matmul followed by the ReLU backward rule in the same kernel:

@@ -27,10 +27,12 @@
 // operation a kernel, 157 now. What bounds such programs is the interpretation
 // (16 instructions on 4096 x 4096: 87 us, 46 for their bytes), not memory.
 //
-// Every element is read and written once, so loads and stores are
-// non-temporal (streamed past the caches). Measured on MI355X at 4096 x 4096
-// with four inputs, one output and one column sum: 60 us for 268 MB read and
-// 67 MB written (5.6 TB/s).
+// Flat and plain column programs read and write every element once, so their
+// loads and stores are non-temporal (streamed past the caches): four inputs,
+// one output and one column sum on 4096 x 4096, 340 MB, take 60 to 64 us with 4
+// to 10 instructions (5.3-5.6 TB/s, combine included). Matrix programs load
+// through the caches, which hold their small inputs, and stream their outputs;
+// programs with row sums store through the caches.
 #include "fused_map.hpp"
 #include "reduce_common.hpp"
 

@@ -1286,6 +1286,8 @@ constexpr int kSmallThreads = 64 * kSmallWaves;
 constexpr int kSmallStage = 2 * kSmallTile * kSmallDepth;  // floats of one wave's stage, A then B
 constexpr int kSmallLoads = 4;                             // loads per operand and chunk
 constexpr int kMaxSplitTiles = 1 << 14;
+// Ranges finished of each split tile, zero between launches: launches of this
+// kernel must not overlap (the library's one stream never lets them).
 __device__ unsigned int g_small_done[kMaxSplitTiles];
 
 // One operand's chunk loader: the operand's matrices are stored with row stride
